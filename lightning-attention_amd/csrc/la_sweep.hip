@@ -24,23 +24,22 @@ int prepare_plans() { return num_cus() > 0 ? 0 : (int)hipErrorInvalidDevice; }
 // rebuild their incoming state themselves.  A warm-up block costs about half a full block, so
 // chunk lengths shrink geometrically (len_c ~ (1 - rho)^c, rho = 0.5) to make all workgroups
 // finish together.  The caller's launch options can override the count.
-static int64_t warm_up_chunks(int64_t wgs, int64_t nblk) {
+static int64_t warm_up_chunks(int64_t wgs, int64_t nblk, int64_t min_blocks = 4) {
     const int64_t cus = num_cus();
     int64_t c = 1;
-    if (wgs * 2 <= cus && nblk >= 8) {
+    if (wgs * 2 <= cus && nblk >= 2 * min_blocks) {
         c = cus / wgs;
-        if (c > nblk / 4) c = nblk / 4;
+        if (c > nblk / min_blocks) c = nblk / min_blocks;
     }
     return c > 8 ? 8 : c < 1 ? 1 : c;
 }
 
-void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start /* [9] */) {
-    int64_t c = forced > 0 ? forced : warm_up_chunks(wgs, nblk);
+void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start /* [9] */, double rho, int64_t min_blocks) {
+    int64_t c = forced > 0 ? forced : warm_up_chunks(wgs, nblk, min_blocks);
     if (c > 8) c = 8;
     if (c > nblk) c = nblk;
     if (c < 1) c = 1;
     // geometric lengths, at least one block each, summing to nblk
-    const double rho = 0.5;
     double wsum = 0.0, wgt = 1.0;
     for (int i = 0; i < c; ++i) { wsum += wgt; wgt *= 1.0 - rho; }
     int64_t start = 0;

@@ -147,8 +147,9 @@ inline unsigned part_grid(const SweepPair& p) {
 
 // Count (up to 8) and first blocks, chunk_start[0 .. 8], of the warm-up chunks for a launch that would have
 // `wgs` workgroups with one chunk each, on a walk of nblk blocks; `forced` > 0 overrides the count.
+// `rho`: what a warm-up block costs of a full one; `min_blocks`: fewest blocks per chunk (on average).
 // Defined in la_sweep.hip.
-void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start);
+void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start, double rho = 0.5, int64_t min_blocks = 4);
 
 // Raises a kernel's dynamic LDS limit above the 64 KB default, once per kernel and device (the call is
 // not free and the limit stays).  `done` is the instantiation's own flag array, one entry per device.

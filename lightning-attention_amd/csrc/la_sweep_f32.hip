@@ -12,6 +12,13 @@
 //   state tiles   come in groups of four (kt = 4K + q); row rho of tile kt is feature
 //                 64K + 4 pi(rho) + q with pi(rho) = 4 (rho % 4) + rho / 4, so that one 16-byte read of a
 //                 y row (state update) or an x row (inter-block term) feeds the four tiles of a group.
+//
+// What bounds it: the fp32 matrix instruction (32 cycles each, 256 FLOP per cycle and CU).  A block costs the busiest
+// wave 48 of them for its score tiles, 64 + 40 for the output and 64 for the state (feature dim 64): 2.9 us at 2.4 GHz,
+// measured 4.2 (4.8 before fragments were requested a step ahead of their use and the global accesses went through
+// bounds-checked buffers without branches; 5.4 with four score tiles on the last wave).  Few sequences: the walk is cut
+// into chunks, whose warm-up blocks cost 1.5 us (0.9 for the matrix instructions) with their tiles double-buffered.
+// b1 h8 n1024 d64: forward 49.5 -> 30.8 us, backward 53 -> 36; b4 h32 n2048 d128: 325 -> 259 and 984 -> 764.
 #include "la_sweep_common.h"
 #include "lightning_attn_hip.h"
 
@@ -77,14 +84,32 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
     float rate = 0.f;
     if (DECAY) rate = a.s[unit % a.h];
 
-    float dfac[4][4], ofac[4], zfac[4][4], lamB = 1.f;
+    // the 16 x 16 score tiles of this wave (at most three: 48 instead of 64 matrix instructions for the busiest wave)
+    TileDeal deal = kDeal[w];
+    if (REVERSE) {
+        deal.itA = 3 - deal.itA; deal.jt0 = 3 - deal.jt0;
+        if (deal.itB >= 0) { deal.itB = 3 - deal.itB; deal.jt1 = 3 - deal.jt1; deal.jt2 = 3 - deal.jt2; }
+    }
+    const int itA = __builtin_amdgcn_readfirstlane(deal.itA), jt0 = __builtin_amdgcn_readfirstlane(deal.jt0);
+    const int itB = __builtin_amdgcn_readfirstlane(deal.itB), jt1 = __builtin_amdgcn_readfirstlane(deal.jt1);
+    const int jt2 = __builtin_amdgcn_readfirstlane(deal.jt2);
+    float dfac[3][4], ofac[4], zfac[4][4], lamB = 1.f;
+    {
+        const int its[3] = {itA, itB, itB}, jts[3] = {jt0, jt1, jt2};
+#pragma unroll
+        for (int sl = 0; sl < 3; ++sl)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = 16 * its[sl] + r, j = 16 * jts[sl] + 4 * g + v;
+                const int diff = REVERSE ? (j - i) : (i - j);
+                dfac[sl][v] = diff >= 0 ? (DECAY ? expf(-rate * (float)diff) : 1.f) : 0.f;
+            }
+    }
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int i = 16 * w + r, j = 16 * jt + 4 * g + v;
-            const int diff = REVERSE ? (j - i) : (i - j);
-            dfac[jt][v] = diff >= 0 ? (DECAY ? expf(-rate * (float)diff) : 1.f) : 0.f;
+            const int j = 16 * jt + 4 * g + v;
             zfac[jt][v] = DECAY ? expf(-rate * (float)(REVERSE ? j : 64 - j)) : 1.f;
         }
 #pragma unroll
@@ -100,160 +125,236 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
 
     const int64_t nblk = (n + 63) / 64;
     const int64_t it_first = a.chunk_start[chunk], it_end = a.chunk_start[chunk + 1];
-    uint4 xr[XC], yr[XC], zr[4];
+    u32x4 xr[XC], yr[XC], zr[4];
 
-    // block number `it` of the walk; x is not needed for a warm-up block
+    // Block number `it` of the walk; x is not needed for a warm-up block.  One bounds-checked buffer per tensor and
+    // block (tokens beyond n and features beyond dk / dv read as zero): no branches, and 32-bit offsets however long
+    // the sequence.
+    const int lrow = tid / (DKP / 4), lcol = (tid % (DKP / 4)) * 4;
+    const int zrow = tid / 16, zcol = col0 + (tid % 16) * 4;
+    const unsigned xoff = lcol < dk ? (unsigned)(lrow * dk + lcol) * 4u : kOob;
+    const unsigned zoff = zcol < dv ? (unsigned)(zrow * dv + zcol) * 4u : kOob;
     auto load_block = [&](int64_t it) {
         const int64_t tok0 = (REVERSE ? nblk - 1 - it : it) * 64;
-        const bool need_x = it >= it_first;
+        const unsigned rows = (unsigned)min((int64_t)64, n - tok0);
+        const __amdgpu_buffer_rsrc_t xb = make_rsrc(xg + tok0 * dk, it >= it_first ? rows * dk * 4u : 0u);
+        const __amdgpu_buffer_rsrc_t yb = make_rsrc(yg + tok0 * dk, rows * dk * 4u);
+        const __amdgpu_buffer_rsrc_t zb = make_rsrc(zg + tok0 * dv, rows * dv * 4u);
+#pragma unroll
+        for (int u = 0; u < XC; ++u) {
+            const unsigned off = xoff + (unsigned)(u * (1024 / DKP) * dk) * 4u;
+            xr[u] = buf_load16(xb, off);
+            yr[u] = buf_load16(yb, off);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) zr[u] = buf_load16(zb, zoff + (unsigned)(u * 16 * dv) * 4u);
+    };
+    auto stage_x = [&]() {
 #pragma unroll
         for (int u = 0; u < XC; ++u) {
             const int c = tid + 256 * u;
             const int row = c / (DKP / 4), col = (c % (DKP / 4)) * 4;
-            const bool ok = (tok0 + row < n) && (col < dk);
-            xr[u] = ok && need_x ? *reinterpret_cast<const uint4*>(xg + (tok0 + row) * dk + col) : make_uint4(0, 0, 0, 0);
-            yr[u] = ok ? *reinterpret_cast<const uint4*>(yg + (tok0 + row) * dk + col) : make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<u32x4*>(Xs + row * XS + col) = xr[u];
+        }
+    };
+    auto stage_yz = [&](float* Y, float* Z) {
+#pragma unroll
+        for (int u = 0; u < XC; ++u) {
+            const int c = tid + 256 * u;
+            const int row = c / (DKP / 4), col = (c % (DKP / 4)) * 4;
+            *reinterpret_cast<u32x4*>(Y + row * XS + col) = yr[u];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int c = tid + 256 * u;
             const int row = c / 16, col = (c % 16) * 4;
-            const bool ok = (tok0 + row < n) && (col0 + col < dv);
-            zr[u] = ok ? *reinterpret_cast<const uint4*>(zg + (tok0 + row) * dv + col0 + col) : make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<u32x4*>(Z + row * ZS + col) = zr[u];
         }
     };
-    auto stage_block = [&]() {
+    // z[j][16w + r] for the 16 tokens j = 16jt + 4g + v this lane contracts over
+    float zf[4][4];
+    auto read_z = [&](const float* Z) {
 #pragma unroll
-        for (int u = 0; u < XC; ++u) {
-            const int c = tid + 256 * u;
-            const int row = c / (DKP / 4), col = (c % (DKP / 4)) * 4;
-            *reinterpret_cast<uint4*>(Xs + row * XS + col) = xr[u];
-            *reinterpret_cast<uint4*>(Ys + row * XS + col) = yr[u];
-        }
+        for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int c = tid + 256 * u;
-            const int row = c / 16, col = (c % 16) * 4;
-            *reinterpret_cast<uint4*>(Zs + row * ZS + col) = zr[u];
-        }
+            for (int v = 0; v < 4; ++v) zf[jt][v] = Z[(16 * jt + 4 * g + v) * ZS + 16 * w + r];
     };
-
-    for (int c = tid; c < 64 * ZS / 4; c += 256) reinterpret_cast<uint4*>(Ps)[c] = make_uint4(0, 0, 0, 0);
-    load_block(0);
-    stage_block();
-    __syncthreads();
-
-    const int jlo = REVERSE ? w : 0, jhi = REVERSE ? 3 : w;
-
-    for (int64_t it = 0; it < it_end; ++it) {
-        const int64_t t = REVERSE ? nblk - 1 - it : it;
-        const bool have_next = it + 1 < it_end;
-        const bool warm = it < it_first;  // warm-up block: state update only
-        if (have_next) load_block(it + 1);
-
-        // 1. S^T tiles (rows j, columns i in [16w, 16w+16)) -> masked, decayed P[i][j]
-        if (!warm) {
-            f32x4 sacc[4];
+    // state = lam^64 state + y^T (z * Lupd); row r of tile 4K + q is feature 64K + 16 (r % 4) + 4 (r / 4) + q
+    auto update = [&](const float* Y) {
+        // fragments requested eight at a time, one batch ahead of their use
+        f32x4 ay[2][8];
+        auto fetch = [&](int bt) {
 #pragma unroll
-            for (int jt = 0; jt < 4; ++jt) sacc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < KT; ++kt) {
-                const f32x4 bx = *reinterpret_cast<const f32x4*>(Xs + (16 * w + r) * XS + 16 * kt + 4 * g);
-#pragma unroll
-                for (int jt = 0; jt < 4; ++jt) {
-                    if (jt >= jlo && jt <= jhi) {
-                        const f32x4 ay = *reinterpret_cast<const f32x4*>(Ys + (16 * jt + r) * XS + 16 * kt + 4 * g);
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) sacc[jt] = mma4(ay[v], bx[v], sacc[jt]);
-                    }
-                }
+            for (int i = 0; i < 8; ++i) {
+                const int K = bt / 2, jt = 2 * (bt % 2) + i / 4, v = i % 4;
+                ay[bt % 2][i] = *reinterpret_cast<const f32x4*>(Y + (16 * jt + 4 * g + v) * XS + 64 * K + 16 * (r & 3) + 4 * (r >> 2));
             }
-#pragma unroll
-            for (int jt = 0; jt < 4; ++jt) {
-                if (jt >= jlo && jt <= jhi) {
-                    f32x4 p;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) p[v] = sacc[jt][v] * dfac[jt][v];
-                    *reinterpret_cast<f32x4*>(Ps + (16 * w + r) * ZS + 16 * jt + 4 * g) = p;
-                }
-            }
-        }
-        __syncthreads();
-
-        if (wave_active) {
-            // z[j][16w + r] for the 16 tokens j = 16jt + 4g + v this lane contracts over
-            float zf[4][4];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        fetch(0);
+        if (DECAY) {
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) zf[jt][v] = Zs[(16 * jt + 4 * g + v) * ZS + 16 * w + r];
+                for (int v = 0; v < 4; ++v) zf[jt][v] *= zfac[jt][v];
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) st[kt][v] *= lamB;
+        }
+#pragma unroll
+        for (int bt = 0; bt < 2 * KG; ++bt) {
+            if (bt + 1 < 2 * KG) fetch(bt + 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    st[4 * (bt / 2) + q] = mma4(ay[bt % 2][i][q], zf[2 * (bt % 2) + i / 4][i % 4], st[4 * (bt / 2) + q]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
 
-            f32x4 oacc[4];
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                if (warm) continue;  // (block-uniform) no output from a warm-up block
-                oacc[i4] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                // 2a. inter-block: st[4K + q][v] holds row 4g + v of its tile, feature 64K + 16v + 4g + q
-#pragma unroll
-                for (int K = 0; K < KG; ++K) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const f32x4 bx = *reinterpret_cast<const f32x4*>(Xs + (16 * i4 + r) * XS + 64 * K + 16 * v + 4 * g);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) oacc[i4] = mma4(st[4 * K + q][v], bx[q], oacc[i4]);
-                    }
-                }
-                if (DECAY) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) oacc[i4][v] *= ofac[i4];
-                }
-                // 2b. intra-block: slot g of step (jt, v) is token 16jt + 4g + v
-#pragma unroll
-                for (int jt = 0; jt < 4; ++jt) {
-                    const bool need = REVERSE ? (jt >= i4) : (jt <= i4);
-                    if (need) {
-                        const f32x4 bp = *reinterpret_cast<const f32x4*>(Ps + (16 * i4 + r) * ZS + 16 * jt + 4 * g);
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) oacc[i4] = mma4(zf[jt][v], bp[v], oacc[i4]);
-                    }
-                }
+    // Warm-up: the blocks before the chunk, state update alone.  They need neither the x nor the P tile, whose LDS
+    // serves as the second y / z buffer: one barrier per block, the next block staged and the one after it requested
+    // from memory while this one is worked on.
+    load_block(0);
+    if (it_first > 0) {
+        stage_yz(Ys, Zs);
+        load_block(1);
+        for (int64_t it = 0; it < it_first; ++it) {
+            const bool odd = (it & 1) != 0;
+            __syncthreads();
+            if (wave_active) {
+                read_z(odd ? Ps : Zs);
+                update(odd ? Xs : Ys);
             }
-            const int col = col0 + 16 * w + 4 * g;
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const int64_t tok = t * 64 + 16 * i4 + r;
-                if (!warm && tok < n && col < dv) *reinterpret_cast<f32x4*>(og + tok * dv + col) = oacc[i4];
-            }
-            // 3. state = lam^64 state + y^T (z * Lupd)
-            if (have_next) {
-                if (DECAY) {
-#pragma unroll
-                    for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) zf[jt][v] *= zfac[jt][v];
-#pragma unroll
-                    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) st[kt][v] *= lamB;
-                }
-                // row r of tile 4K + q is feature 64K + 16 (r % 4) + 4 (r / 4) + q
-#pragma unroll
-                for (int K = 0; K < KG; ++K) {
-#pragma unroll
-                    for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const f32x4 ay = *reinterpret_cast<const f32x4*>(Ys + (16 * jt + 4 * g + v) * XS + 64 * K +
-                                                                             16 * (r & 3) + 4 * (r >> 2));
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) st[4 * K + q] = mma4(ay[q], zf[jt][v], st[4 * K + q]);
-                        }
-                }
+            if (it + 1 < it_first) {
+                stage_yz(odd ? Ys : Xs, odd ? Zs : Ps);
+                load_block(it + 2);
             }
         }
         __syncthreads();
+    }
+    // (tiles of P on the masked side of the diagonal are never written)
+    for (int c = tid; c < 64 * ZS / 4; c += 256) reinterpret_cast<uint4*>(Ps)[c] = make_uint4(0, 0, 0, 0);
+    stage_x();
+    stage_yz(Ys, Zs);
+    __syncthreads();
+
+    for (int64_t it = it_first; it < it_end; ++it) {
+        const bool have_next = it + 1 < it_end;
+        if (have_next) load_block(it + 1);
+
+        // 1. S^T tiles -> masked, decayed P[i][j]
+        auto frag = [&](const float* tile, int row16, int kt) { return *reinterpret_cast<const f32x4*>(tile + (16 * row16 + r) * XS + 16 * kt + 4 * g); };
+        auto put_p = [&](int sl, int i16, int j16, const f32x4& acc) {
+            f32x4 p;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) p[v] = acc[v] * dfac[sl][v];
+            *reinterpret_cast<f32x4*>(Ps + (16 * i16 + r) * ZS + 16 * j16 + 4 * g) = p;
+        };
+        f32x4 s0 = (f32x4){0.f, 0.f, 0.f, 0.f}, s1 = s0, s2 = s0;
+        if (itB >= 0) {
+            f32x4 xa[2], xb[2], y0[2], y1[2], y2[2];
+            auto fetch = [&](int kt) {
+                xa[kt % 2] = frag(Xs, itA, kt);
+                y0[kt % 2] = frag(Ys, jt0, kt);
+                xb[kt % 2] = frag(Xs, itB, kt);
+                y1[kt % 2] = frag(Ys, jt1, kt);
+                y2[kt % 2] = frag(Ys, jt2, kt);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            fetch(0);
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                if (kt + 1 < KT) fetch(kt + 1);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    s0 = mma4(y0[kt % 2][v], xa[kt % 2][v], s0);
+                    s1 = mma4(y1[kt % 2][v], xb[kt % 2][v], s1);
+                    s2 = mma4(y2[kt % 2][v], xb[kt % 2][v], s2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            put_p(1, itB, jt1, s1);
+            put_p(2, itB, jt2, s2);
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                const f32x4 xa = frag(Xs, itA, kt), y0 = frag(Ys, jt0, kt);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) s0 = mma4(y0[v], xa[v], s0);
+            }
+        }
+        put_p(0, itA, jt0, s0);
+        __syncthreads();
+
+        if (wave_active) {
+            f32x4 oacc[4];
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) oacc[i4] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            // 2a. inter-block: st[4K + q][v] holds row 4g + v of its tile, feature 64K + 16v + 4g + q.  Here and in 2b the
+            // fragments are requested one step ahead of their use (left to itself the scheduler sinks every read to
+            // its first use, and the wave pays an LDS round trip per step).
+            f32x4 bx[2][4], bp[2][4];
+            auto fetch_x = [&](int step) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) bx[step % 2][i4] = *reinterpret_cast<const f32x4*>(Xs + (16 * i4 + r) * XS + 16 * step + 4 * g);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto fetch_p = [&](int jt) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const bool need = REVERSE ? (jt >= i4) : (jt <= i4);
+                    if (need) bp[jt % 2][i4] = *reinterpret_cast<const f32x4*>(Ps + (16 * i4 + r) * ZS + 16 * jt + 4 * g);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            fetch_x(0);
+#pragma unroll
+            for (int step = 0; step < 4 * KG; ++step) {
+                if (step + 1 < 4 * KG) fetch_x(step + 1);
+                else {
+                    read_z(Zs);
+                    fetch_p(0);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) oacc[i4] = mma4(st[4 * (step / 4) + q][step % 4], bx[step % 2][i4][q], oacc[i4]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (DECAY) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) oacc[i4][v] *= ofac[i4];
+            }
+            // 2b. intra-block: slot g of step (jt, v) is token 16jt + 4g + v
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) {
+                if (jt + 1 < 4) fetch_p(jt + 1);
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        const bool need = REVERSE ? (jt >= i4) : (jt <= i4);
+                        if (need) oacc[i4] = mma4(zf[jt][v], bp[jt % 2][i4][v], oacc[i4]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int64_t tok0 = (REVERSE ? nblk - 1 - it : it) * 64;
+            const __amdgpu_buffer_rsrc_t ob = make_rsrc(og + tok0 * dv, (unsigned)min((int64_t)64, n - tok0) * dv * 4u);
+            const int col = col0 + 16 * w + 4 * g;
+            const unsigned ooff = col < dv ? (unsigned)(r * dv + col) * 4u : kOob;
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) buf_store16(ob, ooff + (unsigned)(16 * i4 * dv) * 4u, 0u, __builtin_bit_cast(u32x4, oacc[i4]));
+            if (have_next) update(Ys);
+        }
+        __syncthreads();
         if (have_next) {
-            stage_block();
+            stage_x();
+            stage_yz(Ys, Zs);
             __syncthreads();
         }
     }
@@ -342,11 +443,17 @@ static SweepArgsF32 make_args_f32(const void* x, const void* y, const void* z, v
     return a;
 }
 
+// What a warm-up block costs of a full one (1.5 of 4.2 us), and the fewest blocks a chunk is worth cutting off for.
+// b1 h8 d64 forward, us, by number of chunks 1 / 2 / 4 / 8: n = 1024 69.9 / 44.7 / 33.7 / 30.9, n = 4096 268 / 169 / 123 /
+// 108: as many as there are CUs for, down to two blocks each.
+static const double kWarmCost = 0.36;
+static const int64_t kMinBlocks = 2;
+
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
               int64_t n, int64_t dk, int64_t dv, bool reverse, int chunks, hipStream_t st) {
     if (dk > 128) return LA_E_UNSUPPORTED;
     SweepArgsF32 a = make_args_f32(x, y, z, out, s, bh, h, n, dk, dv);
-    plan_warm_up_chunks((bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start);
+    plan_warm_up_chunks((bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
     return reverse ? launch_dir_f32<true>(a, st) : launch_dir_f32<false>(a, st);
 }
 
@@ -359,7 +466,7 @@ int sweep_f32_bwd_once(const void* q, const void* k, const void* v, const void* 
     t.a[0] = make_args_f32(dout, v, k, dq, s, bh, h, n, d, d);
     t.a[1] = make_args_f32(v, dout, q, dk, s, bh, h, n, d, d);
     t.a[2] = make_args_f32(k, q, dout, dv, s, bh, h, n, d, d);
-    plan_warm_up_chunks((bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, chunks, &t.a[0].nchunk, t.a[0].chunk_start);
+    plan_warm_up_chunks((bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, chunks, &t.a[0].nchunk, t.a[0].chunk_start, kWarmCost, kMinBlocks);
     for (int i = 1; i < 3; ++i) {
         t.a[i].nchunk = t.a[0].nchunk;
         for (int j = 0; j < 9; ++j) t.a[i].chunk_start[j] = t.a[0].chunk_start[j];
