@@ -214,6 +214,26 @@ int la_bwd_saved(const void *q, const void *k, const void *v, const float *s, co
                  const float *saved, size_t saved_bytes, void *stream);
 
 /*
+ * The same pair with the library free to choose what is kept: the plain matrices above where they help, or - where
+ * the forward pass runs in chunks from scanned states (few long sequences) and the dQ sweep has the same chunks - the
+ * state slots the forward pass works with anyway.  The contents of `carry` are opaque: la_bwd_carry must be given what
+ * la_fwd_carry left for the same tensors, shapes and options on the same device; it only reads it.
+ * la_carry_bytes: bytes to provide (16-byte aligned), 0 where nothing would be kept.  With carry == NULL or too few
+ * bytes the calls are la_fwd_opts and la_bwd_opts; where bytes are provided la_fwd_carry needs no workspace.
+ */
+size_t la_carry_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, const la_launch_opts *opts);
+int la_fwd_carry(const void *q, const void *k, const void *v, const float *s, void *o,
+                 const int64_t *strides,
+                 int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype,
+                 void *workspace, size_t ws_bytes, const la_launch_opts *opts,
+                 void *carry, size_t carry_bytes, void *stream);
+int la_bwd_carry(const void *q, const void *k, const void *v, const float *s, const void *dout,
+                 void *dq, void *dk, void *dv, const int64_t *strides,
+                 int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype,
+                 void *workspace, size_t ws_bytes, const la_launch_opts *opts,
+                 const void *carry, size_t carry_bytes, void *stream);
+
+/*
  * la_fwd for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc) and so cannot supply the workspace that makes few
  * long sequences fast: same arguments without the workspace pair, same results bit for bit as la_fwd

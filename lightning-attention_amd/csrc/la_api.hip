@@ -10,7 +10,7 @@ int sweep(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, i
 int sweep_silu(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
 int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
-                   int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
+                   int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st);
 int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk,
                        int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
 int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv,
@@ -21,6 +21,12 @@ int sweep_saving(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64
                  float* save, int save_len, int width, hipStream_t st);
 int sweep_resumed(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                   const float* saved, int nchunk, int chunk_len, int width, hipStream_t st);
+SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts);
+int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
+                   float* carry, const SavedPlan& pl, hipStream_t st);
+int sweep_carried(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
+                  const float* carry, const SavedPlan& pl, hipStream_t st);
+double carried_us(int64_t e, const SavedPlan& pl);
 int prepare_srmsnorm();   // srmsnorm.hip
 int prepare_norm_gate();  // norm_gate.hip
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
@@ -95,10 +101,13 @@ static int check_tensor(const Tensor& t, int64_t b, int64_t h, int64_t n, int64_
 }
 
 // States for the backward pass (may be absent): memory the forward pass writes / the backward pass reads.
+// `carry`: in whichever of the two formats the shape has a use for, not only as plain matrices (la_carry_bytes).
 struct Saved {
     float* p;
     size_t bytes;
+    bool carry;
 };
+static const SavedPlan kNoPlan = {1, 0, 0, 0, 0};
 static bool saved_usable(const Saved& sv, const SavedPlan& pl) {
     return pl.nchunk > 1 && sv.p && sv.bytes >= pl.bytes && al16(sv.p);
 }
@@ -120,6 +129,8 @@ static int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
     if (sv.p) {
         const SavedPlan pl = plan_saved(b * h, n, d, e, dtype, opts);
         if (saved_usable(sv, pl)) return sweep_saving(io(q, k, v, o), s, b * h, h, n, d, e, dtype, sv.p, pl.chunk_len, pl.fwd_width, st);
+        const SavedPlan cp = sv.carry ? plan_carry(b * h, n, d, e, dtype, opts) : kNoPlan;
+        if (saved_usable(sv, cp)) return sweep_carrying(io(q, k, v, o), s, b * h, h, n, d, e, dtype, sv.p, cp, st);
     }
     return run(q, k, v, o, s, b * h, h, n, d, e, dtype, false, ws, opts, st);
 }
@@ -146,10 +157,13 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
         return sweep_f32_bwd_once(q.p, k.p, v.p, dout.p, const_cast<void*>(dq.p), const_cast<void*>(dk.p),
                                   const_cast<void*>(dv.p), s, b * h, h, n, d, opts.chunks, st);
     }
+    const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : kNoPlan;
+    const SavedPlan cp = sv.p && sv.carry && pl.nchunk <= 1 ? plan_carry(b * h, n, d, e, dtype, opts) : kNoPlan;
+    const bool carried = saved_usable(sv, cp);
     if (d == e && dtype != LA_FP32) {
         // few sequences: all three gradients in one launch, side by side (LA_E_UNSUPPORTED: not this time)
         rc = sweep_bwd_once(io(dout, v, k, dq), io(v, dout, q, dk), io(k, q, dout, dv), s, b * h, h, n, d, dtype, ws.p,
-                            ws.bytes, opts, st);
+                            ws.bytes, opts, carried ? carried_us(e, cp) : 0.0, st);
         if (rc != LA_E_UNSUPPORTED) return rc;
     }
     if (d != e && dtype != LA_FP32) {
@@ -158,7 +172,6 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
         if (rc == LA_OK) return run(k, q, dout, dv, s, b * h, h, n, d, e, dtype, true, ws, opts, st);
         if (rc != LA_E_UNSUPPORTED) return rc;
     }
-    const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : SavedPlan{1, 0, 0, 0, 0};
     if (saved_usable(sv, pl) && d == e) {
         // dK + dV first: their reverse walk starts at the end of the sequences, where the forward pass has just
         // been (what the last-level cache still holds of k, v, q is read there: -0.8 % per step at b4 h32 n8192
@@ -169,6 +182,8 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
     }
     if (saved_usable(sv, pl))  // the chunks of dQ start from the states the forward pass left
         rc = sweep_resumed(io(dout, v, k, dq), s, b * h, h, n, e, d, dtype, sv.p, pl.nchunk, pl.chunk_len, pl.dq_width, st);
+    else if (carried)
+        rc = sweep_carried(io(dout, v, k, dq), s, b * h, h, n, e, d, dtype, sv.p, cp, st);
     else
         rc = run(dout, v, k, dq, s, b * h, h, n, e, d, dtype, false, ws, opts, st);
     if (rc != LA_OK) return rc;
@@ -226,11 +241,11 @@ extern "C" size_t la_workspace_bytes(int which, int64_t b, int64_t h, int64_t n,
     return la_workspace_bytes_opts(which, b, h, n, d, e, dtype, nullptr);
 }
 
-extern "C" int la_fwd_save(const void* q, const void* k, const void* v, const float* s, void* o, const int64_t* strides,
-                           int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace,
-                           size_t ws_bytes, const la_launch_opts* opts, float* saved, size_t saved_bytes, void* stream) {
+namespace la {
+static int fwd_saved(const void* q, const void* k, const void* v, const float* s, void* o, const int64_t* strides, int64_t b,
+                     int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace, size_t ws_bytes,
+                     const la_launch_opts* opts, const Saved& sv, void* stream) {
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
-    const la::Saved sv = {saved, saved ? saved_bytes : 0};
     const la::Opts& op = opts ? *opts : la::kAuto;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
@@ -239,6 +254,21 @@ extern "C" int la_fwd_save(const void* q, const void* k, const void* v, const fl
         return la::fwd(dense(q, h, n, d), dense(k, h, n, d), dense(v, h, n, e), s, dense(o, h, n, e), b, h, n, d, e, dtype, ws, op, sv, st);
     return la::fwd(strided(q, strides), strided(k, strides + 3), strided(v, strides + 6), s, strided(o, strides + 9), b, h, n,
                    d, e, dtype, ws, op, sv, st);
+}
+}  // namespace la
+
+extern "C" int la_fwd_save(const void* q, const void* k, const void* v, const float* s, void* o, const int64_t* strides,
+                           int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace,
+                           size_t ws_bytes, const la_launch_opts* opts, float* saved, size_t saved_bytes, void* stream) {
+    return la::fwd_saved(q, k, v, s, o, strides, b, h, n, d, e, dtype, workspace, ws_bytes, opts,
+                         la::Saved{saved, saved ? saved_bytes : 0, false}, stream);
+}
+
+extern "C" int la_fwd_carry(const void* q, const void* k, const void* v, const float* s, void* o, const int64_t* strides,
+                            int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace,
+                            size_t ws_bytes, const la_launch_opts* opts, void* carry, size_t carry_bytes, void* stream) {
+    return la::fwd_saved(q, k, v, s, o, strides, b, h, n, d, e, dtype, workspace, ws_bytes, opts,
+                         la::Saved{static_cast<float*>(carry), carry ? carry_bytes : 0, true}, stream);
 }
 
 extern "C" int la_fwd_silu_supported(int64_t d, int64_t e, int dtype) {
@@ -250,7 +280,7 @@ extern "C" int la_fwd_silu(const void* q, const void* k, const void* v, const fl
                            size_t ws_bytes, const la_launch_opts* opts, void* stream) {
     if (la_supported(d, e, dtype) && !la_fwd_silu_supported(d, e, dtype)) return LA_E_UNSUPPORTED;
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
-    const la::Saved none = {nullptr, 0};
+    const la::Saved none = {nullptr, 0, false};
     const la::Opts& op = opts ? *opts : la::kAuto;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
@@ -282,12 +312,18 @@ extern "C" int64_t la_saved_state_interval(int64_t b, int64_t h, int64_t n, int6
     return pl.nchunk > 1 ? (int64_t)pl.chunk_len * 64 : 0;
 }
 
-extern "C" int la_bwd_saved(const void* q, const void* k, const void* v, const float* s, const void* dout, void* dq,
-                            void* dk, void* dv, const int64_t* strides, int64_t b, int64_t h, int64_t n, int64_t d,
-                            int64_t e, int dtype, void* workspace, size_t ws_bytes, const la_launch_opts* opts,
-                            const float* saved, size_t saved_bytes, void* stream) {
+extern "C" size_t la_carry_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, const la_launch_opts* opts) {
+    const la::Opts& o = opts ? *opts : la::kAuto;
+    if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
+    const la::SavedPlan pl = la::plan_saved(b * h, n, d, e, dtype, o);
+    return pl.nchunk > 1 ? pl.bytes : la::plan_carry(b * h, n, d, e, dtype, o).bytes;
+}
+
+namespace la {
+static int bwd_from(const void* q, const void* k, const void* v, const float* s, const void* dout, void* dq, void* dk, void* dv,
+                    const int64_t* strides, int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace,
+                    size_t ws_bytes, const la_launch_opts* opts, const Saved& sv, void* stream) {
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
-    const la::Saved sv = {const_cast<float*>(saved), saved ? saved_bytes : 0};
     const la::Opts& op = opts ? *opts : la::kAuto;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
@@ -298,6 +334,23 @@ extern "C" int la_bwd_saved(const void* q, const void* k, const void* v, const f
     return la::bwd(strided(q, strides), strided(k, strides + 3), strided(v, strides + 6), s, strided(dout, strides + 9),
                    strided(dq, strides + 12), strided(dk, strides + 15), strided(dv, strides + 18), b, h, n, d, e, dtype, ws,
                    op, sv, st);
+}
+}  // namespace la
+
+extern "C" int la_bwd_saved(const void* q, const void* k, const void* v, const float* s, const void* dout, void* dq,
+                            void* dk, void* dv, const int64_t* strides, int64_t b, int64_t h, int64_t n, int64_t d,
+                            int64_t e, int dtype, void* workspace, size_t ws_bytes, const la_launch_opts* opts,
+                            const float* saved, size_t saved_bytes, void* stream) {
+    return la::bwd_from(q, k, v, s, dout, dq, dk, dv, strides, b, h, n, d, e, dtype, workspace, ws_bytes, opts,
+                        la::Saved{const_cast<float*>(saved), saved ? saved_bytes : 0, false}, stream);
+}
+
+extern "C" int la_bwd_carry(const void* q, const void* k, const void* v, const float* s, const void* dout, void* dq,
+                            void* dk, void* dv, const int64_t* strides, int64_t b, int64_t h, int64_t n, int64_t d,
+                            int64_t e, int dtype, void* workspace, size_t ws_bytes, const la_launch_opts* opts,
+                            const void* carry, size_t carry_bytes, void* stream) {
+    return la::bwd_from(q, k, v, s, dout, dq, dk, dv, strides, b, h, n, d, e, dtype, workspace, ws_bytes, opts,
+                        la::Saved{static_cast<float*>(const_cast<void*>(carry)), carry ? carry_bytes : 0, true}, stream);
 }
 
 extern "C" int la_bwd_opts(const void* q, const void* k, const void* v, const float* s, const void* dout, void* dq,

@@ -209,10 +209,61 @@ static void set_width(SweepArgs& a, int width, int64_t dv) {
     }
 }
 
+// The shapes whose whole state fits the accumulators of one workgroup as a square tile, so that a sweep can start from
+// the transpose of another one's state: width code of those workgroups, -1 for other shapes.
+static int square_width(int64_t dk, int64_t dv) {
+    if (dk <= 64 && dv <= 64) return 0;
+    return dk > 64 && dk <= 128 && dv > 64 && dv <= 128 ? 1 : -1;
+}
+static bool own_choices(const Opts& o) {
+    return o.chunks == 0 && o.scan == LA_OPT_AUTO && o.wide == LA_OPT_AUTO && o.paired == LA_OPT_AUTO;
+}
+
+// dK + dV with d == e from scanned states that are collected once for both: dV carries Q^T dO, dK its transpose dO^T Q.
+// `nchunk` chunks of `chunk_len` blocks per sweep, collected as `ncollect` chunks of chunk_len / mul blocks (one
+// sweep collects, so there are CUs for mul times as many chunks).  nchunk == 1: not for this shape.
+struct SharedPlan {
+    int nchunk, chunk_len, ncollect, mul;
+    size_t bytes;
+    double us;
+};
+// In place of a collect of both sweeps it always pays (b1 h16 n32768 d128 without decay: collect + scan 105 + 7 -> 63 + 8
+// us).  Against two single walks that fill the chip in 64-column workgroups - which are then bound by the memory system and
+// take 1.95 us per block, not the 1.4 of block_us - the two extra launches have to be earned back: fwd + bwd at 64
+// sequences of d128, without / with: n = 1600 104 / 110 us, 2048 134 / 139, 4096 302 / 291, 16384 887 / 855.
+static SharedPlan plan_shared(int64_t bh, int64_t n, int64_t d, size_t scratch, const Opts& opts) {
+    const int own_width = column_width(bh, n, d, d, 2, scratch, opts), width = square_width(d, d);
+    const int64_t nblk = (n + 63) / 64, cus = num_cus(), units8 = (bh + 7) / 8 * 8;
+    SharedPlan none = {1, 0, 0, 1, 0, width_us(bh, n, d, d, 2, own_width, scratch, opts)};
+    if (own_width == 0 && d > 64 && d <= 128 && units8 * slices(d, d, 0) * 4 > cus) none.us *= 1.95 / 1.4;
+    if (width < 0 || !own_choices(opts)) return none;
+    const ScanPlan own = plan_scan(bh, n, d, d, 2, own_width, opts);
+    const bool scanned = own.nchunk > 1 && own.bytes <= scratch;
+    int64_t c = cus / (2 * units8);
+    if (c > nblk / 4) c = nblk / 4;
+    if (c > 32) c = 32;
+    if (c < 2 || bh > 65535) return none;
+    int64_t mul = cus / (units8 * c);
+    if (mul > 2) mul = 2;
+    SharedPlan pl;
+    const int64_t len = (nblk + c * mul - 1) / (c * mul);
+    pl.mul = (int)mul;
+    pl.chunk_len = (int)(len * mul);
+    pl.nchunk = (int)((nblk + pl.chunk_len - 1) / pl.chunk_len);
+    pl.ncollect = (int)((nblk + len - 1) / len);
+    if (pl.nchunk < 2) return none;
+    pl.bytes = (size_t)bh * (size_t)(pl.ncollect - 1) * pipe_state_floats((int)d, width) * sizeof(float);
+    pl.us = (0.5 * (double)len + (double)pl.chunk_len) * block_us(d, width) + 16.0 + 10.0 + (scanned ? 0.0 : 10.0);
+    return pl.us < none.us && pl.bytes <= scratch ? pl : none;
+}
+
 // Workspace the kernels can use for one launch of nprod sweeps (0: none).
 size_t sweep_workspace_bytes(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int dtype, const Opts& opts) {
     if (dtype != LA_BF16 && dtype != LA_FP16) return 0;
-    return plan_scan(bh, n, dk, dv, nprod, column_width(bh, n, dk, dv, nprod, (size_t)-1, opts), opts).bytes;
+    const size_t own = plan_scan(bh, n, dk, dv, nprod, column_width(bh, n, dk, dv, nprod, (size_t)-1, opts), opts).bytes;
+    if (nprod != 2) return own;
+    const size_t shared = plan_shared(bh, n, dk, (size_t)-1, opts).bytes;
+    return shared > own ? shared : own;
 }
 
 static int launch_planned(SweepPair& p, int64_t bh, int64_t n, int64_t dk, int64_t dv, int dtype, bool reverse, void* ws,
@@ -351,6 +402,52 @@ int sweep_resumed(const SweepIO& io, const float* s, int64_t bh, int64_t h, int6
     return sweep_pipe(p, dtype, false, st);
 }
 
+// A launch of one sweep in nchunk chunks of chunk_len blocks from state slots at `state`.
+static SweepPair chunked(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int width,
+                         int nchunk, int chunk_len, float* state) {
+    SweepPair p;
+    p.nprod = 1;
+    p.a[0] = make_args(io, s, bh, h, n, dk, dv);
+    set_width(p.a[0], width, dv);
+    p.a[0].nchunk = nchunk;
+    for (int j = 0; j < 9; ++j) p.a[0].chunk_start[j] = 0;
+    p.a[1] = p.a[0];
+    p.wide = width;
+    p.mode = kCollect;
+    p.chunk_len = chunk_len;
+    p.state = state;
+    return p;
+}
+
+// Where the forward pass runs in chunks from scanned states and the state tile is square, the slots it leaves behind
+// serve the dQ sweep of the backward pass (same chunks, transposed states): no collect and scan launches there.
+// b1 h16 n32768 d128 without decay: dQ 60 + 8 + 97 us -> 97; fwd + bwd 491 -> 424 us.
+// nchunk == 1: not for this shape.
+SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts) {
+    const SavedPlan none = {1, 0, 0, 0, 0};
+    const int width = square_width(d, e);
+    if ((dtype != LA_BF16 && dtype != LA_FP16) || width < 0 || !own_choices(opts)) return none;
+    if (column_width(bh, n, d, e, 1, (size_t)-1, opts) != width) return none;
+    const ScanPlan pl = plan_scan(bh, n, d, e, 1, width, opts);
+    return pl.nchunk > 1 ? SavedPlan{pl.nchunk, pl.chunk_len, pl.bytes, width, width} : none;
+}
+// The forward sweep by that plan, its slots in `carry`.
+int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
+                   float* carry, const SavedPlan& pl, hipStream_t st) {
+    return sweep_pipe(chunked(io, s, bh, h, n, dk, dv, pl.fwd_width, pl.nchunk, pl.chunk_len, carry), dtype, false, st);
+}
+// The dQ sweep from what sweep_carrying over (., z, y) left.
+int sweep_carried(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
+                  const float* carry, const SavedPlan& pl, hipStream_t st) {
+    SweepPair p = chunked(io, s, bh, h, n, dk, dv, pl.dq_width, pl.nchunk, pl.chunk_len, const_cast<float*>(carry));
+    p.shared = 1;
+    p.nslot = pl.nchunk - 1;
+    p.transposed = 1;
+    return sweep_pipe_apply(p, dtype, false, st);
+}
+// Estimated duration (us) of that launch.
+double carried_us(int64_t e, const SavedPlan& pl) { return (double)pl.chunk_len * block_us(e, pl.dq_width); }
+
 // Two sweeps of the same shape and direction in one launch.
 int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv,
            int dtype, bool reverse, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st) {
@@ -358,7 +455,24 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
         const int rc = sweep(io0, s, bh, h, n, dk, dv, dtype, reverse, ws, ws_bytes, opts, st);
         return rc != LA_OK ? rc : sweep(io1, s, bh, h, n, dk, dv, dtype, reverse, ws, ws_bytes, opts, st);
     }
+    const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
+    const SharedPlan sh = dk == dv && ws_ok ? plan_shared(bh, n, dk, ws_bytes, opts) : SharedPlan{1, 0, 0, 1, 0, 0.0};
     SweepPair p;
+    if (sh.nchunk > 1) {
+        // io0 (dK) and io1 (dV) have y and z swapped: io1's states, and for io0 their transposes
+        const int width = square_width(dk, dv);
+        p = chunked(io1, s, bh, h, n, dk, dv, width, sh.ncollect, sh.chunk_len / sh.mul, static_cast<float*>(ws));
+        const int rc = sweep_pipe_collect(p, dtype, reverse, st);
+        if (rc != LA_OK) return rc;
+        p = chunked(io0, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws));
+        p.a[1] = chunked(io1, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws)).a[0];
+        p.nprod = 2;
+        p.shared = 1;
+        p.nslot = sh.ncollect - 1;
+        p.slot_mul = sh.mul;
+        p.transposed = 1;
+        return sweep_pipe_apply(p, dtype, reverse, st);
+    }
     p.nprod = 2;
     p.a[0] = make_args(io0, s, bh, h, n, dk, dv);
     p.a[1] = make_args(io1, s, bh, h, n, dk, dv);
@@ -370,9 +484,9 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
 // the warm-up chunks the CUs left over allow.  Results are bit-identical to separate launches.
 // Returns LA_E_UNSUPPORTED when separate launches are to be used (they are estimated faster - scanned
 // chunk states on a long walk -, or the sweeps fill the chip anyway).  opts.once = LA_OPT_OFF / LA_OPT_ON:
-// never / whenever possible.
+// never / whenever possible.  dq_us > 0: what the dQ sweep alone would take from states the forward pass left.
 int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
-                   int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st) {
+                   int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
     if (dtype != LA_BF16 && dtype != LA_FP16) return LA_E_UNSUPPORTED;
     const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
     if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
@@ -385,11 +499,9 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
         if (wgs > 2 * cus) return LA_E_UNSUPPORTED;
         // what the separate launches would take, by the estimates behind their own plans
         const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-        double separate = 0.0;
-        for (int nprod = 1; nprod <= 2; ++nprod) {
-            const size_t scratch = ws_ok ? ws_bytes : 0;
-            separate += width_us(bh, n, d, d, nprod, column_width(bh, n, d, d, nprod, scratch, opts), scratch, opts);
-        }
+        const size_t scratch = ws_ok ? ws_bytes : 0;
+        const double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) +
+                                plan_shared(bh, n, d, scratch, opts).us;
         // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
         const double rounds = wgs > cus ? 2.0 : 1.0;
         if (rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) >= separate) return LA_E_UNSUPPORTED;

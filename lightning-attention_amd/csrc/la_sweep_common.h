@@ -119,6 +119,11 @@ struct SweepPair {
     int mode;
     int chunk_len;
     float* state;
+    // kApply from states that another launch over the same tensors collected: `shared` says that there is one set of
+    // slots per unit and slice for all sweeps of the launch, nslot slots to a set, chunk c starting from slot
+    // c * slot_mul - 1; bit i of `transposed`: sweep i has y and z in swapped roles, its state is the transpose of
+    // the collected one (square tiles of state only: feature dim as padded == columns of a workgroup).
+    int shared = 0, nslot = 0, slot_mul = 1, transposed = 0;
     // Forward walk in one piece (pipelined kernel, 64-column workgroups): after every save_len blocks but the
     // last the state is also written to `save`, per unit (number of such boundaries) row-major dk x dv float
     // matrices.  The sweep (x', y' = z, z' = y) then has exactly the transposed state at those boundaries
@@ -179,6 +184,9 @@ struct SavedPlan {
 // n, dk, dv, h, bh, nslice and the chunking must agree between the two sweeps of a pair.
 enum { kWarmUp = 0, kCollect = 1, kApply = 2, kResume = 3 };
 int sweep_pipe(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
+// The middle and the last of the three launches behind kCollect, for a launch whose states are shared.
+int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
+int sweep_pipe_apply(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 // One-time work per device, done ahead of the first launches: the dynamic LDS limits of every instantiation
 // of the pipelined kernels (la_sweep_pipe.hip) and of the float32 kernels (la_sweep_f32.hip), and the
 // device's compute-unit count (la_sweep.hip).

@@ -133,12 +133,21 @@ int sweep_pipe(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
     if (!p.state || p.chunk_len < 1) return LA_E_WORKSPACE;
     if (p.mode == kResume) return launch_any(p, dtype, reverse, st);  // the states are there already
     // three launches: local end states, their scan, the walk proper
+    const int rc = sweep_pipe_collect(p, dtype, reverse, st);
+    return rc != LA_OK ? rc : sweep_pipe_apply(p, dtype, reverse, st);
+}
+
+int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
+    if (!p.state || p.chunk_len < 1 || p.a[0].nchunk < 2 || p.shared) return LA_E_WORKSPACE;
     SweepPair q = p;
     q.mode = kCollect;
-    int rc = launch_any(q, dtype, reverse, st);
-    if (rc != LA_OK) return rc;
-    rc = launch_state_scan(p, st);
-    if (rc != LA_OK) return rc;
+    const int rc = launch_any(q, dtype, reverse, st);
+    return rc != LA_OK ? rc : launch_state_scan(p, st);
+}
+
+int sweep_pipe_apply(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
+    if (!p.state || p.chunk_len < 1 || p.a[0].nchunk < 2) return LA_E_WORKSPACE;
+    SweepPair q = p;
     q.mode = kApply;
     return launch_any(q, dtype, reverse, st);
 }

@@ -254,7 +254,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const int64_t it_end = cend;
     // the state slot of this workgroup's chunk: [unit][sweep][slice][chunk 0 .. nchunk-2][state waves' accumulators]
     constexpr size_t SF = (size_t)4 * NH * KT * 64 * 4;
-    float* const slot0 = pair.state + ((((size_t)unit * nprod + sub % nprod) * nslice + slice) * (size_t)(nchunk - 1)) * SF;
+    const bool shared = NF == 1 && pair.shared;  // (forms with square tiles of state only)
+    const size_t slot_set = shared ? (size_t)unit * nslice + slice : ((size_t)unit * nprod + sub % nprod) * nslice + slice;
+    float* const slot0 = pair.state + slot_set * (size_t)(shared ? pair.nslot : nchunk - 1) * SF;
 
     u32x4 xrA[XC], yrA[XC], zrA[ZC], xrB[XC], yrB[XC], zrB[ZC];
 
@@ -530,6 +532,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // the forms a forward pass that saves runs in, and the forms a pass that resumes runs in
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
+
+    // the forms whose tile of state is square, so that a sweep can start from another one's transposed state
+    constexpr bool TRANSPOSES = NF == 1 && 4 * NH == KT;
 
     f32x4 oacc[NH][4];  // state waves: the output tile of the block in progress, summed over the feature chunks
 
@@ -844,7 +849,22 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
         // this lane's part of a state slot: [wave][slab][tile][lane] accumulator quartets
         const size_t lane_slot = ((size_t)w * NH * KT * 64 + lane) * 4;
         const bool resume = mode == kApply && chunk > 0;
-        const float* const src = slot0 + (size_t)(chunk - 1) * SF + lane_slot;
+        const float* const slot = slot0 + (size_t)(shared ? chunk * pair.slot_mul - 1 : chunk - 1) * SF;
+        const float* const src = slot + lane_slot;
+        if constexpr (TRANSPOSES) {
+            if (resume && ((pair.transposed >> (sub % nprod)) & 1)) {
+                // state[k][c] = slot[c][k]: tile (kt; NH w + h) is the transpose of the slot's tile (NH w + h; kt)
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+#pragma unroll
+                    for (int kt = 0; kt < KT; ++kt) {
+                        const float* const m = slot + (size_t)(kt * KT + NH * w + h) * 256 + ((r >> 2) * 16 + 4 * g) * 4 + (r & 3);
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) st[h][kt][v] = m[4 * v];
+                    }
+                return;
+            }
+        }
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
@@ -931,6 +951,10 @@ static int launch_one(const SweepPair& pair, hipStream_t st) {
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
     if (pair.mode == kResume && (!RESUMES || pair.nprod != 1)) return LA_E_UNSUPPORTED;
+    if (pair.shared && NF != 1) return LA_E_UNSUPPORTED;
+    if (pair.transposed && (NF != 1 || 4 * NH != DKP / 16 || a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
+    // every chunk's slot must exist
+    if (pair.shared && (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot)) return LA_E_WORKSPACE;
     if (pair.save && (!SAVES || pair.nprod != 1 || pair.mode != kWarmUp || a.nchunk != 1)) return LA_E_UNSUPPORTED;
     const unsigned grid = (unsigned)(units8 * a.nslice * a.nchunk * pair.nprod);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, pair);

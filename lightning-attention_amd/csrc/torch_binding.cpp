@@ -102,11 +102,12 @@ struct Attn : public torch::autograd::Function<Attn> {
         const la_launch_opts* lo = op.given ? &op.o : nullptr;
         Tensor o = at::empty_like(v);  // same sizes as v; dense, in v's memory order
         const c10::DeviceGuard guard(q.device());
-        const size_t ws_bytes = la_workspace_bytes_opts(0, b, h, n, d, e, code, lo);
         Tensor ws, saved;
+        // (save_states arrives false when no backward pass can follow; a forward pass that leaves states works in
+        // their memory)
+        const size_t sv_bytes = op.save_states ? la_carry_bytes(b, h, n, d, e, code, lo) : 0;
+        const size_t ws_bytes = sv_bytes ? 0 : la_workspace_bytes_opts(0, b, h, n, d, e, code, lo);
         if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte));
-        // (save_states arrives false when no backward pass can follow)
-        const size_t sv_bytes = op.save_states ? la_saved_state_bytes(b, h, n, d, e, code, lo) : 0;
         if (sv_bytes) saved = at::empty({(int64_t)(sv_bytes / 4)}, q.options().dtype(at::kFloat));
         int64_t st[4][4], strides[12];
         const bool dense = q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && o.is_contiguous();
@@ -117,7 +118,7 @@ struct Attn : public torch::autograd::Function<Attn> {
                 for (int j = 0; j < 3; ++j) strides[3 * i + j] = st[i][j];
             }
         }
-        check(la_fwd_save(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.defined() ? s.data_ptr<float>() : nullptr, o.data_ptr(),
+        check(la_fwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.defined() ? s.data_ptr<float>() : nullptr, o.data_ptr(),
                           dense ? nullptr : strides, b, h, n, d, e, code, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, lo,
                           sv_bytes ? saved.data_ptr<float>() : nullptr, sv_bytes, stream_of(q)),
               "la_fwd");
@@ -155,7 +156,7 @@ struct Attn : public torch::autograd::Function<Attn> {
                 for (int j = 0; j < 3; ++j) strides[3 * i + j] = st[j];
             }
         const size_t sv_bytes = saved.defined() ? (size_t)saved.numel() * 4 : 0;
-        check(la_bwd_saved(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.defined() ? s.data_ptr<float>() : nullptr, dout.data_ptr(),
+        check(la_bwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.defined() ? s.data_ptr<float>() : nullptr, dout.data_ptr(),
                            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dense ? nullptr : strides, b, h, n, d, e, code,
                            ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, lo, sv_bytes ? saved.data_ptr<float>() : nullptr, sv_bytes,
                            stream_of(q)),

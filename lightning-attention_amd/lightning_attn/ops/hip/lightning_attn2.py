@@ -5,7 +5,7 @@ and lightning_attn2_no_decay.py:367-471: ``lightning_attn2(q, k, v, s)`` and
 ``lightning_attn2_no_decay(q, k, v)`` with q,k (b,h,n,d), v (b,h,n,e), s holding
 h float32 rates; outputs come from torch.empty, kernels go on the current stream,
 and the inputs are saved for backward - plus, for shapes where the library asks for
-them (la_saved_state_bytes in the header), a few float32 states of the forward walk that let
+them (la_carry_bytes in the header), a few float32 states of the forward walk that let
 the dQ sweep of the backward pass start mid-sequence (8 MiB at b4 h32 n8192 d=e=128).
 
 Where the reference copies (``.contiguous()`` on q, k, v, do, lightning_attn2.py:402-405,
@@ -83,7 +83,9 @@ def _fwd(q, k, v, s, for_backward=False, silu=False):
     o = torch.empty_like(v)  # same sizes as v; dense, in v's memory order
     opts = _lib.current_opts()
     with _lib.on_device(q.device):
-        ws_bytes = _lib.workspace_bytes(0, b, h, n, d, e, code, opts)
+        sv_bytes = _lib.carry_bytes(b, h, n, d, e, code, opts) if for_backward and not silu else 0
+        # (a forward pass that leaves states works in their memory)
+        ws_bytes = 0 if sv_bytes else _lib.workspace_bytes(0, b, h, n, d, e, code, opts)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
         sp = s.data_ptr() if s is not None else None
         wp = ws.data_ptr() if ws is not None else None
@@ -94,9 +96,8 @@ def _fwd(q, k, v, s, for_backward=False, silu=False):
             rc = L.la_fwd_silu(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, o.data_ptr(), strides, b, h, n, d, e, code,
                                wp, ws_bytes, op, _lib.stream_ptr(q.device))
         else:
-            sv_bytes = _lib.saved_state_bytes(b, h, n, d, e, code, opts) if for_backward else 0
             saved = torch.empty(sv_bytes // 4, dtype=torch.float32, device=q.device) if sv_bytes else None
-            rc = L.la_fwd_save(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, o.data_ptr(), strides, b, h, n, d, e, code,
+            rc = L.la_fwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, o.data_ptr(), strides, b, h, n, d, e, code,
                                wp, ws_bytes, op, saved.data_ptr() if saved is not None else None, sv_bytes,
                                _lib.stream_ptr(q.device))
     _lib.check(rc, "la_fwd")
@@ -121,7 +122,7 @@ def _bwd(q, k, v, s, do, opts=None, saved=None):
         wp = ws.data_ptr() if ws is not None else None
         dense = all(t.is_contiguous() for t in (q, k, v, do, dq, dk, dv))
         strides = None if dense else _strides(q, k, v, do, dq, dk, dv)
-        rc = L.la_bwd_saved(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, do.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+        rc = L.la_bwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, do.data_ptr(), dq.data_ptr(), dk.data_ptr(),
                             dv.data_ptr(), strides, b, h, n, d, e, code, wp, ws_bytes,
                             ctypes.byref(opts) if opts is not None else None,
                             saved.data_ptr() if saved is not None else None, saved.numel() * 4 if saved is not None else 0,

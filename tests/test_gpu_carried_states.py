@@ -1,0 +1,112 @@
+"""la_fwd_carry / la_bwd_carry where the forward pass runs in chunks from scanned states: the dQ sweep starts from the
+transposes of those states, and dK + dV from states collected once (dK from their transposes).
+
+* o is la_fwd's with the same workspace, bit for bit; the gradients agree with la_bwd's without a workspace (warm-up
+  chunks: states summed in the same order, operands rounded to the tensors' dtype in the other role: a few 1e-3 in the
+  2-norm, as for la_bwd_saved) and with the formula on a few sequences;
+* carry and workspace start as NaN: every slot that is read was written;
+* too few bytes of carry: exactly la_bwd_opts."""
+import ctypes
+
+import pytest
+import torch
+
+import oracle
+from util import assert_close_scaled, rel_norm
+
+pytestmark = pytest.mark.gpu
+
+from lightning_attn.ops import lightning_attn_func  # noqa: E402
+from lightning_attn.ops.hip import _lib  # noqa: E402
+from lightning_attn.utils import _build_slope_tensor  # noqa: E402
+
+CODE = {torch.bfloat16: 0, torch.float16: 1}
+
+CASES = [
+    # b, h, n, d, e, dtype, decay, token_major
+    (1, 16, 8192, 128, 128, torch.bfloat16, True, False),
+    (1, 13, 9057, 128, 128, torch.bfloat16, True, False),   # ragged, a short last chunk, units short of a multiple of 8
+    (2, 12, 6400, 96, 120, torch.float16, True, False),    # d != e: dQ alone
+    (4, 16, 4096, 128, 128, torch.bfloat16, True, True),   # projection layout; dK + dV: two chunks, four collected
+    (3, 15, 6113, 72, 72, torch.bfloat16, False, True),    # no decay, d off the tiles
+    (1, 16, 16384, 64, 64, torch.bfloat16, True, False),   # 64-column workgroups
+    (1, 9, 9001, 48, 40, torch.float16, False, False),
+]
+
+
+def _strides(*ts):
+    vals = []
+    for t in ts:
+        vals += list(t.stride())[:3]
+    return (ctypes.c_int64 * len(vals))(*vals)
+
+
+@pytest.mark.parametrize("b, h, n, d, e, dtype, decay, token_major", CASES)
+def test_gradients_from_carried_states(b, h, n, d, e, dtype, decay, token_major):
+    L = _lib.lib()
+    code = CODE[dtype]
+    g = torch.Generator().manual_seed(n)
+
+    def mk(c):
+        if token_major:
+            return torch.randn(b, n, h, c, generator=g).to(dtype).cuda().transpose(1, 2)
+        return torch.randn(b, h, n, c, generator=g).to(dtype).cuda()
+
+    q, k, v, do = mk(d), mk(d), mk(e), mk(e)
+    s = _build_slope_tensor(h).float().cuda().contiguous() if decay else None
+    sp = s.data_ptr() if decay else None
+    st = torch.cuda.current_stream().cuda_stream
+    nbytes = L.la_carry_bytes(b, h, n, d, e, code, None)
+    print("carry case", (b, h, n, d, e, dtype, decay, token_major), nbytes, flush=True)
+    assert nbytes > 0 and L.la_saved_state_bytes(b, h, n, d, e, code, None) == 0
+    assert nbytes == L.la_workspace_bytes(0, b, h, n, d, e, code)
+    nan = lambda size: torch.full((max(size, 16) // 4,), float("nan"), device="cuda")  # noqa: E731
+    carry, ws0 = nan(nbytes), nan(nbytes)
+    wb = L.la_workspace_bytes(1, b, h, n, d, e, code)
+    ws1 = nan(wb)
+
+    def fwd(ws, cr, cb):
+        o = torch.full_like(v, float("nan"))
+        rc = L.la_fwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, o.data_ptr(), _strides(q, k, v, o), b, h, n, d, e, code,
+                            ws.data_ptr() if ws is not None else None, nbytes if ws is not None else 0, None,
+                            cr.data_ptr() if cr is not None else None, cb, st)
+        assert rc == 0, L.la_error_string(rc)
+        return o
+
+    def bwd(ws, cr, cb):
+        gr = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        rc = L.la_bwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), sp, do.data_ptr(), *(t.data_ptr() for t in gr),
+                            _strides(q, k, v, do, *gr), b, h, n, d, e, code, ws.data_ptr() if ws is not None else None,
+                            wb if ws is not None else 0, None, cr.data_ptr() if cr is not None else None, cb, st)
+        assert rc == 0, L.la_error_string(rc)
+        return gr
+
+    o, o0 = fwd(None, carry, nbytes), fwd(ws0, None, 0)
+    got, plain, short = bwd(ws1, carry, nbytes), bwd(None, None, 0), bwd(None, carry, nbytes - 4)
+    torch.cuda.synchronize()
+    assert torch.equal(o, o0)
+    for a, p, sh in zip(got, plain, short):
+        assert torch.equal(p, sh)
+        assert rel_norm(a, p.float()) < 3e-3, rel_norm(a, p.float())
+    sel = [0, h - 1]
+    qs, ks, vs, ds = (t[-1:, sel].cpu().contiguous() for t in (q, k, v, do))
+    want = oracle.linear_attn_fwd_bwd(qs, ks, vs, s.cpu()[sel] if decay else None, ds, torch.float32)
+    for name, a, r in zip(("o", "dq", "dk", "dv"), [o] + got, want):
+        assert_close_scaled(a[-1:, sel], r, 2e-2, 2e-2, "carried %s" % name)
+        assert rel_norm(a[-1:, sel], r) < 1e-2, (name, rel_norm(a[-1:, sel], r))
+
+
+def test_carried_states_through_autograd_twice():
+    """The operators keep the states with the graph: a second backward pass over it gives the same gradients, and
+    save_states=False keeps the inputs only."""
+    q, k, v, do = (torch.randn(1, 16, 4096, 128, device="cuda", dtype=torch.bfloat16) for _ in range(4))
+    s = _build_slope_tensor(16).float().cuda()
+    ts = [t.requires_grad_() for t in (q, k, v)]
+    assert _lib.lib().la_carry_bytes(1, 16, 4096, 128, 128, 0, None) > 0
+    o = lightning_attn_func(*ts, s)
+    g1 = torch.autograd.grad(o, ts, do, retain_graph=True)
+    g2 = torch.autograd.grad(o, ts, do)
+    assert all(torch.equal(a, c) for a, c in zip(g1, g2))
+    with _lib.launch_opts(save_states=False):
+        g3 = torch.autograd.grad(lightning_attn_func(*ts, s), ts, do)
+    assert all(rel_norm(a, c.float()) < 3e-3 for a, c in zip(g1, g3))
