@@ -6,14 +6,18 @@
 //
 // Same data movement as the SimpleRMSNorm kernels: a row of o, g (and dy) is read once with 16-byte
 // non-temporal loads into registers, reduced, and the results written once.  TPR threads share a row:
-// one or two wavefronts (four or two rows to a workgroup of 256 threads) or a whole workgroup of 256,
-// 512 or 1024 threads.  The forward kernel takes one group of rows per workgroup and fetches weight and
+// 64, 128, 256, 512 or 1024, with as many rows side by side as the workgroup has room for.  The forward kernel takes one group of rows per workgroup and fetches weight and
 // bias from the caches.  The backward kernel walks the rows with a grid stride and gives every thread one
 // 16-byte chunk of the row: a thread always holds the same columns, so weight and bias stay in registers
 // as floats and the column sums (d weight, d bias) are accumulated in registers over all rows a thread
-// sees (118 registers: four waves per SIMD; with more chunks per thread it ran at two).  Those partial
+// sees (117 registers: four waves per SIMD; with more chunks per thread it ran at two).  Those partial
 // sums go to a scratch buffer, one row per workgroup, and a second small kernel adds them up in a fixed
 // order: deterministic, no atomics.
+// The backward kernel is bound by what it keeps in flight, not by its arithmetic: with 16-bit elements the next group of
+// rows is requested before the reduction of this one (float32 runs five waves per SIMD and gains nothing), weight and
+// bias come in one 16-byte load each, and a CU holds one workgroup of 1024 threads and so writes one row of partial sums.
+// Backward pass with its reduction, bf16, us before / after: [16384,2048] 87.2 / 62.9 (5.3 TB/s), [8192,1024] 33.9 / 22.6,
+// [32768,4096] 259 / 225 (6.0 TB/s), [32768,512] 42.0 / 34.7, [4096,8192] 85.5 / 65.1, [700,2048] 22.7 / 9.8.
 //
 // Per element, float32 throughout:
 //   forward   xh = (o - mean) rstd ; ln = xh w + b ; sg = 1 / (1 + exp(-g)) ; y = ln sg
@@ -27,9 +31,14 @@ namespace la {
 // Threads of a workgroup: TPR threads share a row; rows of one or two wavefronts travel four or two to a
 // workgroup of 256, wider rows take a workgroup of 256, 512 or 1024 threads to themselves.
 constexpr int ng_threads(int tpr) { return tpr >= 256 ? tpr : 256; }
+// The backward kernel with 16-bit elements: always 1024 threads (its registers leave a CU 16 wavefronts either way), so
+// that a CU leaves one row of partial column sums, not four.
+constexpr int ng_bwd_threads(int tpr, int elt) { return elt == 2 ? 1024 : ng_threads(tpr); }
 
 // both sums over the TPR threads of a row at once (every thread of the workgroup takes part)
-template <int TPR>
+// ONCE: the caller hands over another 32 floats of LDS on every other call, so that the next call's writes cannot meet
+// this one's reads and one barrier will do
+template <int TPR, bool ONCE = false>
 __device__ __forceinline__ void row_sum2(float& a, float& b, float* red) {
     if (TPR >= 128) {
         constexpr int NWV = TPR / 64;  // wavefronts per row
@@ -47,7 +56,7 @@ __device__ __forceinline__ void row_sum2(float& a, float& b, float* red) {
             a += red[w0 + i];
             b += red[16 + w0 + i];
         }
-        __syncthreads();
+        if (!ONCE) __syncthreads();
         return;
     }
 #pragma unroll
@@ -141,49 +150,69 @@ __global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_fwd_kernel(const T*
     }
 }
 
+typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));  // (the workspace need not be 16-byte aligned)
+
 // `part`: gridDim.x rows of [d weight | d bias] partial column sums, 2 * cols floats each.
 template <typename T, int NV, int TPR>
-__global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_bwd_kernel(const T* __restrict__ o, const T* __restrict__ g,
+__global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T))) void norm_gate_bwd_kernel(const T* __restrict__ o, const T* __restrict__ g,
                                                                   const T* __restrict__ w, const T* __restrict__ b,
                                                                   const float* __restrict__ mean, const float* __restrict__ rstd,
                                                                   const T* __restrict__ dy, T* __restrict__ d_o,
                                                                   T* __restrict__ d_g, float* __restrict__ part,
                                                                   int64_t rows, int cols) {
     constexpr int E = Pack16<T>::N;
-    constexpr int RPG = ng_threads(TPR) / TPR;
-    __shared__ float red[32];
+    constexpr int RPG = ng_bwd_threads(TPR, sizeof(T)) / TPR;
+    constexpr bool AHEAD = sizeof(T) == 2;
+    __shared__ float red[64];
     __shared__ float comb[RPG > 1 ? (RPG - 1) * TPR * NV * E * 2 : 1];  // column sums of the rows beside the first
     const int l = threadIdx.x % TPR;
     float wf[NV][E], bf[NV][E];  // this thread's columns of weight and bias
     float aw[NV][E], ab[NV][E];  // ... and of the column sums
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
+        // (one 16-byte load each: element by element every load waited for the one before it, 10 us per workgroup)
         const int c = (u * TPR + l) * E;
+        Pack16<T> pw, pb;
+        if (c < cols) {
+            pw = *reinterpret_cast<const Pack16<T>*>(w + c);
+            pb = *reinterpret_cast<const Pack16<T>*>(b + c);
+        }
 #pragma unroll
         for (int t = 0; t < E; ++t) {
-            wf[u][t] = c < cols ? (float)w[c + t] : 0.f;
-            bf[u][t] = c < cols ? (float)b[c + t] : 0.f;
+            wf[u][t] = c < cols ? (float)pw.v[t] : 0.f;
+            bf[u][t] = c < cols ? (float)pb.v[t] : 0.f;
             aw[u][t] = ab[u][t] = 0.f;
         }
     }
     const float inv = 1.0f / (float)cols;
-    for (int64_t row0 = (int64_t)blockIdx.x * RPG; row0 < rows; row0 += (int64_t)gridDim.x * RPG) {
+    // The next group of rows is requested as soon as the first pass has used up the packed registers of this one, so
+    // that its memory latency runs beside the reduction, the second pass and the stores.
+    const int64_t step = (int64_t)gridDim.x * RPG;
+    Pack16<T> po[NV], pg[NV], py[NV];
+    float mu_next = 0.f, rs_next = 0.f;
+    auto fetch = [&](int64_t row) __attribute__((always_inline)) {
+        if (row < rows) {
+            const int64_t at = row * (int64_t)cols;
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int c = (u * TPR + l) * E;
+                if (c < cols) {
+                    po[u] = load16(o + at + c);
+                    pg[u] = load16(g + at + c);
+                    py[u] = load16(dy + at + c);
+                }
+            }
+            mu_next = mean[row];
+            rs_next = rstd[row];
+        }
+    };
+    if (AHEAD) fetch((int64_t)blockIdx.x * RPG + threadIdx.x / TPR);
+    int turn = 0;
+    for (int64_t row0 = (int64_t)blockIdx.x * RPG; row0 < rows; row0 += step, turn ^= 1) {
         const int64_t row = row0 + threadIdx.x / TPR;
         const bool row_ok = row < rows;
-        const T* orow = o + row * (int64_t)cols;
-        const T* grow = g + row * (int64_t)cols;
-        const T* yrow = dy + row * (int64_t)cols;
-        Pack16<T> po[NV], pg[NV], py[NV];
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int c = (u * TPR + l) * E;
-            if (row_ok && c < cols) {
-                po[u] = load16(orow + c);
-                pg[u] = load16(grow + c);
-                py[u] = load16(yrow + c);
-            }
-        }
-        const float mu = row_ok ? mean[row] : 0.f, rs = row_ok ? rstd[row] : 0.f;
+        if (!AHEAD) fetch(row);
+        const float mu = mu_next, rs = rs_next;
         // Kept from the first pass for the second: xh, dln and 1 - sigmoid(g) (one exp and one
         // reciprocal per element in all; the kernel is close to its VALU budget, not only to HBM's).
         float xh[NV][E], dln[NV][E], cs[NV][E];
@@ -207,7 +236,8 @@ __global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_bwd_kernel(const T*
                 }
             }
         }
-        row_sum2<TPR>(s1, s2, red);
+        if (AHEAD) fetch(row + step);
+        row_sum2<TPR, true>(s1, s2, red + 32 * turn);
         const float k1 = s1 * inv * rs, k2 = s2 * inv * rs;
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
@@ -257,9 +287,9 @@ __global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_bwd_kernel(const T*
         const int c = (u * TPR + l) * E;
         if (c < cols) {
 #pragma unroll
-            for (int t = 0; t < E; ++t) {
-                prow[c + t] = aw[u][t];
-                prow[cols + c + t] = ab[u][t];
+            for (int t = 0; t < E; t += 4) {
+                *reinterpret_cast<Quad*>(prow + c + t) = Quad{aw[u][t], aw[u][t + 1], aw[u][t + 2], aw[u][t + 3]};
+                *reinterpret_cast<Quad*>(prow + cols + c + t) = Quad{ab[u][t], ab[u][t + 1], ab[u][t + 2], ab[u][t + 3]};
             }
         }
     }
@@ -331,30 +361,30 @@ static void ng_shape(int64_t chunks, bool backward, int* tpr, int* nv) {
 }
 
 // workgroups of a launch: enough to keep every CU's memory pipeline full, never more than row groups
-static int64_t ng_grid(int64_t rows, int tpr, bool backward) {
-    const int64_t threads = ng_threads(tpr), rpg = threads / tpr, groups = (rows + rpg - 1) / rpg;
+static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
+    const int64_t threads = backward ? ng_bwd_threads(tpr, elt) : ng_threads(tpr), rpg = threads / tpr, groups = (rows + rpg - 1) / rpg;
     if (!backward) return groups;  // nothing is carried from row to row: one group of rows per workgroup
     const int64_t cap = 4 * (int64_t)num_cus() * 256 / threads;  // ~16 wavefronts per CU
     return groups < cap ? groups : cap;
 }
 
-#define LA_NG_GO(KERNEL, NV, TPR, ...) hipLaunchKernelGGL((KERNEL<T, NV, TPR>), grid, dim3(ng_threads(TPR)), 0, st, __VA_ARGS__)
+#define LA_NG_GO(KERNEL, NV, TPR, THREADS, ...) hipLaunchKernelGGL((KERNEL<T, NV, TPR>), grid, dim3(THREADS), 0, st, __VA_ARGS__)
 #define LA_NG_DISPATCH_FWD(KERNEL, ...)                               \
     do {                                                              \
-        if (tpr == 64 && nv == 1) LA_NG_GO(KERNEL, 1, 64, __VA_ARGS__);       \
-        else if (tpr == 64 && nv == 2) LA_NG_GO(KERNEL, 2, 64, __VA_ARGS__);  \
-        else if (tpr == 64) LA_NG_GO(KERNEL, 4, 64, __VA_ARGS__);             \
-        else if (nv == 1) LA_NG_GO(KERNEL, 1, 256, __VA_ARGS__);              \
-        else if (nv == 2) LA_NG_GO(KERNEL, 2, 256, __VA_ARGS__);              \
-        else LA_NG_GO(KERNEL, 4, 256, __VA_ARGS__);                           \
+        if (tpr == 64 && nv == 1) LA_NG_GO(KERNEL, 1, 64, ng_threads(64), __VA_ARGS__);       \
+        else if (tpr == 64 && nv == 2) LA_NG_GO(KERNEL, 2, 64, ng_threads(64), __VA_ARGS__);  \
+        else if (tpr == 64) LA_NG_GO(KERNEL, 4, 64, ng_threads(64), __VA_ARGS__);             \
+        else if (nv == 1) LA_NG_GO(KERNEL, 1, 256, ng_threads(256), __VA_ARGS__);              \
+        else if (nv == 2) LA_NG_GO(KERNEL, 2, 256, ng_threads(256), __VA_ARGS__);              \
+        else LA_NG_GO(KERNEL, 4, 256, ng_threads(256), __VA_ARGS__);                           \
     } while (0)
 #define LA_NG_DISPATCH_BWD(KERNEL, ...)                               \
     do {                                                              \
-        if (tpr == 64) LA_NG_GO(KERNEL, 1, 64, __VA_ARGS__);          \
-        else if (tpr == 128) LA_NG_GO(KERNEL, 1, 128, __VA_ARGS__);   \
-        else if (tpr == 256) LA_NG_GO(KERNEL, 1, 256, __VA_ARGS__);   \
-        else if (tpr == 512) LA_NG_GO(KERNEL, 1, 512, __VA_ARGS__);   \
-        else LA_NG_GO(KERNEL, 1, 1024, __VA_ARGS__);                  \
+        if (tpr == 64) LA_NG_GO(KERNEL, 1, 64, ng_bwd_threads(64, sizeof(T)), __VA_ARGS__);          \
+        else if (tpr == 128) LA_NG_GO(KERNEL, 1, 128, ng_bwd_threads(128, sizeof(T)), __VA_ARGS__);   \
+        else if (tpr == 256) LA_NG_GO(KERNEL, 1, 256, ng_bwd_threads(256, sizeof(T)), __VA_ARGS__);   \
+        else if (tpr == 512) LA_NG_GO(KERNEL, 1, 512, ng_bwd_threads(512, sizeof(T)), __VA_ARGS__);   \
+        else LA_NG_GO(KERNEL, 1, 1024, ng_bwd_threads(1024, sizeof(T)), __VA_ARGS__);                  \
     } while (0)
 
 template <typename T>
@@ -363,7 +393,7 @@ static int ng_fwd(const void* o, const void* g, const void* w, const void* b, vo
     int tpr = 0, nv = 0;
     ng_shape(cols / (16 / (int64_t)sizeof(T)), false, &tpr, &nv);
     if (!nv) return LA_E_UNSUPPORTED;
-    const dim3 grid((unsigned)ng_grid(rows, tpr, false));
+    const dim3 grid((unsigned)ng_grid(rows, tpr, false, sizeof(T)));
     LA_NG_DISPATCH_FWD(norm_gate_fwd_kernel, static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
                    static_cast<const T*>(b), static_cast<T*>(y), mean, rstd, rows, (int)cols, eps);
     return (int)hipGetLastError();
@@ -376,7 +406,7 @@ static int ng_bwd(const void* o, const void* g, const void* w, const void* b, co
     int tpr = 0, nv = 0;
     ng_shape(cols / (16 / (int64_t)sizeof(T)), true, &tpr, &nv);
     if (!nv) return LA_E_UNSUPPORTED;
-    const dim3 grid((unsigned)ng_grid(rows, tpr, true));
+    const dim3 grid((unsigned)ng_grid(rows, tpr, true, sizeof(T)));
     LA_NG_DISPATCH_BWD(norm_gate_bwd_kernel, static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
                    static_cast<const T*>(b), mean, rstd, static_cast<const T*>(dy), static_cast<T*>(d_o), static_cast<T*>(d_g),
                    part, rows, (int)cols);
@@ -417,7 +447,7 @@ extern "C" size_t norm_gate_workspace_bytes(int64_t rows, int64_t cols, int dtyp
     if (rows <= 0 || !norm_gate_supported(cols, dtype)) return 0;
     int tpr = 0, nv = 0;
     la::ng_shape(cols / (dtype == LA_FP32 ? 4 : 8), true, &tpr, &nv);
-    return (size_t)la::ng_grid(rows, tpr, true) * 2 * (size_t)cols * sizeof(float);
+    return (size_t)la::ng_grid(rows, tpr, true, dtype == LA_FP32 ? 4 : 2) * 2 * (size_t)cols * sizeof(float);
 }
 
 extern "C" int norm_gate_fwd(const void* o, const void* g, const void* weight, const void* bias, void* y, float* mean,
