@@ -11,6 +11,8 @@ int sweep_silu(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t
                void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
 int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                    int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st);
+int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
+                      int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st);
 int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk,
                        int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
 int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv,
@@ -167,6 +169,10 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
         if (rc != LA_E_UNSUPPORTED) return rc;
     }
     if (d != e && dtype != LA_FP32) {
+        // few sequences: all three gradients in one launch
+        rc = sweep_bwd_once_de(io(dout, v, k, dq), io(v, dout, q, dk), io(k, q, dout, dv), s, b * h, h, n, d, e, dtype, ws.p,
+                               ws.bytes, opts, carried ? carried_us(e, cp) : 0.0, st);
+        if (rc != LA_E_UNSUPPORTED) return rc;
         // dQ and dK have one shape and opposite directions: with few sequences, one launch for the two
         rc = sweep_fwd_rev_once(io(dout, v, k, dq), io(v, dout, q, dk), s, b * h, h, n, e, d, dtype, ws.p, ws.bytes, opts, st);
         if (rc == LA_OK) return run(k, q, dout, dv, s, b * h, h, n, d, e, dtype, true, ws, opts, st);
@@ -400,6 +406,7 @@ static int static_scratch(void** out) {
 extern "C" int la_init(void) {
     int rc = la::prepare_plans();
     if (rc == LA_OK) rc = la::prepare_pipe();
+    if (rc == LA_OK) rc = la::prepare_trio();
     if (rc == LA_OK) rc = la::prepare_f32();
     if (rc == LA_OK) rc = la::prepare_srmsnorm();
     if (rc == LA_OK) rc = la::prepare_norm_gate();

@@ -12,6 +12,8 @@
 // decides, from the shape and the compute units of the device, how many columns of z / out a workgroup
 // takes (64 or 128), whether a long walk over few sequences is cut into chunks (from warm-up blocks, or
 // from scanned states in a workspace), and which sweeps of a backward pass share a launch.
+#include <algorithm>
+
 #include "la_sweep_common.h"
 #include "lightning_attn_hip.h"
 
@@ -527,6 +529,46 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
     }
     b.nfwd = part_grid(b.fwd);
     return sweep_pipe_both(b, dtype, st);
+}
+
+// The same with d != e (both up to 128), where the three sweeps have a CU for every 64-column workgroup: side by side
+// they take as long as the longest of them, and one launch replaces two or three (b6 h8 n1213 d128 e64 fp16:
+// la_bwd 50.7 -> 33 us).  LA_E_UNSUPPORTED otherwise.
+int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
+                      int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
+    if ((dtype != LA_BF16 && dtype != LA_FP16) || d > 128 || e > 128) return LA_E_UNSUPPORTED;
+    const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
+    if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
+    if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;
+    const int64_t cus = num_cus(), nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8;
+    const int64_t wgs_a = units8 * slices(e, d, 0) * 2, wgs = wgs_a + units8 * slices(d, e, 0);
+    if (forced == 0) {
+        if (wgs > cus) return LA_E_UNSUPPORTED;
+        const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
+        const size_t scratch = ws_ok ? ws_bytes : 0;
+        const double a_us = width_us(bh, n, e, d, 1, column_width(bh, n, e, d, 1, scratch, opts), scratch, opts);
+        const double v_us = width_us(bh, n, d, e, 1, column_width(bh, n, d, e, 1, scratch, opts), scratch, opts);
+        const double two = warm_up_frac(wgs_a, nblk) * (double)nblk * block_us(e, 0);  // dQ and dK sharing a launch
+        const double separate = std::min(two, (dq_us > 0.0 ? dq_us : a_us) + a_us) + v_us;
+        if (warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) >= separate) return LA_E_UNSUPPORTED;
+    }
+    SweepTrio t;
+    SweepPair* const ps[3] = {&t.dq, &t.dk, &t.dv};
+    const SweepIO* const ios[3] = {&dq, &dk, &dv};
+    for (int i = 0; i < 3; ++i) {
+        SweepPair& p = *ps[i];
+        p.nprod = 1;
+        p.a[0] = i < 2 ? make_args(*ios[i], s, bh, h, n, e, d) : make_args(*ios[i], s, bh, h, n, d, e);
+        plan_warm_up_chunks(wgs, nblk, opts.chunks, &p.a[0].nchunk, p.a[0].chunk_start);
+        p.a[1] = p.a[0];
+        p.wide = 0;
+        p.mode = kWarmUp;
+        p.chunk_len = 0;
+        p.state = nullptr;
+    }
+    t.ndq = part_grid(t.dq);
+    t.ndv = part_grid(t.dv);
+    return sweep_pipe_trio(t, dtype, st);
 }
 
 // The same for two sweeps of one shape and opposite directions (dQ and dK of a backward pass with

@@ -150,6 +150,14 @@ inline unsigned part_grid(const SweepPair& p) {
     return (unsigned)((p.a[0].bh + 7) / 8 * 8 * p.a[0].nslice * p.a[0].nchunk * p.nprod);
 }
 
+// The three sweeps of a backward pass with d != e in one launch (la_sweep_pipe_trio.hip): one sweep to a part, all in
+// 64-column workgroups and the same warm-up chunks.
+struct SweepTrio {
+    SweepPair dq, dk, dv;
+    unsigned ndq, ndv;  // workgroups of the dQ and dV parts (multiples of 8)
+};
+int sweep_pipe_trio(const SweepTrio& t, int dtype, hipStream_t st);
+
 // Count (up to 8) and first blocks, chunk_start[0 .. 8], of the warm-up chunks for a launch that would have
 // `wgs` workgroups with one chunk each, on a walk of nblk blocks; `forced` > 0 overrides the count.
 // `rho`: what a warm-up block costs of a full one; `min_blocks`: fewest blocks per chunk (on average).
@@ -188,10 +196,11 @@ int sweep_pipe(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 int sweep_pipe_apply(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 // One-time work per device, done ahead of the first launches: the dynamic LDS limits of every instantiation
-// of the pipelined kernels (la_sweep_pipe.hip) and of the float32 kernels (la_sweep_f32.hip), and the
+// of the pipelined kernels (la_sweep_pipe.hip, la_sweep_pipe_trio.hip) and of the float32 kernels (la_sweep_f32.hip), and the
 // device's compute-unit count (la_sweep.hip).
 int prepare_pipe();
 int prepare_f32();
+int prepare_trio();
 int prepare_plans();
 // Floats of one state slot: the feature dim as the kernel pads it (64, 128, 192 or 256) times the 64 or 128
 // columns of a workgroup.  Must agree with the kernels' own SF; the 128-column form pads feature dims up
