@@ -423,7 +423,7 @@ static SweepPair chunked(const SweepIO& io, const float* s, int64_t bh, int64_t 
 
 // Where the forward pass runs in chunks from scanned states and the state tile is square, the slots it leaves behind
 // serve the dQ sweep of the backward pass (same chunks, transposed states): no collect and scan launches there.
-// b1 h16 n32768 d128 without decay: dQ 60 + 8 + 97 us -> 97; fwd + bwd 491 -> 424 us.
+// b1 h16 n32768 d128 without decay: dQ 60 + 8 + 97 us -> 97; with the shared collect of dK + dV fwd + bwd 494 -> 416 us.
 // nchunk == 1: not for this shape.
 SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts) {
     const SavedPlan none = {1, 0, 0, 0, 0};
@@ -532,8 +532,9 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
 }
 
 // The same with d != e (both up to 128), where the three sweeps have a CU for every 64-column workgroup: side by side
-// they take as long as the longest of them, and one launch replaces two or three (b6 h8 n1213 d128 e64 fp16:
-// la_bwd 50.7 -> 33 us).  LA_E_UNSUPPORTED otherwise.
+// they take as long as the longest of them, and one launch replaces two or three (fwd + bwd of b2 h20 n2048 d128 e96
+// 124 -> 91 us, b1 h40 n6000 d128 e64 210 -> 194).  Beyond one workgroup per CU the sweeps would only queue behind each other.
+// LA_E_UNSUPPORTED otherwise.
 int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                       int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
     if ((dtype != LA_BF16 && dtype != LA_FP16) || d > 128 || e > 128) return LA_E_UNSUPPORTED;
