@@ -254,7 +254,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const int64_t it_end = cend;
     // the state slot of this workgroup's chunk: [unit][sweep][slice][chunk 0 .. nchunk-2][state waves' accumulators]
     constexpr size_t SF = (size_t)4 * NH * KT * 64 * 4;
-    const bool shared = NF == 1 && pair.shared;  // (forms with square tiles of state only)
+    // the forms whose tile of state is square, so that a sweep can start from another one's transposed state
+    constexpr bool TRANSPOSES = NF == 1 && 4 * NH == KT && !SILU;
+    const bool shared = TRANSPOSES && pair.shared;
     const size_t slot_set = shared ? (size_t)unit * nslice + slice : ((size_t)unit * nprod + sub % nprod) * nslice + slice;
     float* const slot0 = pair.state + slot_set * (size_t)(shared ? pair.nslot : nchunk - 1) * SF;
 
@@ -532,9 +534,6 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // the forms a forward pass that saves runs in, and the forms a pass that resumes runs in
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
-
-    // the forms whose tile of state is square, so that a sweep can start from another one's transposed state
-    constexpr bool TRANSPOSES = NF == 1 && 4 * NH == KT;
 
     f32x4 oacc[NH][4];  // state waves: the output tile of the block in progress, summed over the feature chunks
 
@@ -951,8 +950,8 @@ static int launch_one(const SweepPair& pair, hipStream_t st) {
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
     if (pair.mode == kResume && (!RESUMES || pair.nprod != 1)) return LA_E_UNSUPPORTED;
-    if (pair.shared && NF != 1) return LA_E_UNSUPPORTED;
-    if (pair.transposed && (NF != 1 || 4 * NH != DKP / 16 || a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
+    if (pair.shared && (NF != 1 || 4 * NH != DKP / 16 || SILU || a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
+    if (pair.transposed && !pair.shared) return LA_E_UNSUPPORTED;
     // every chunk's slot must exist
     if (pair.shared && (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot)) return LA_E_WORKSPACE;
     if (pair.save && (!SAVES || pair.nprod != 1 || pair.mode != kWarmUp || a.nchunk != 1)) return LA_E_UNSUPPORTED;
