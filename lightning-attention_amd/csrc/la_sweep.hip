@@ -221,7 +221,13 @@ static bool own_choices(const Opts& o) {
     return o.chunks == 0 && o.scan == LA_OPT_AUTO && o.wide == LA_OPT_AUTO && o.paired == LA_OPT_AUTO;
 }
 
-// dK + dV with d == e from scanned states that are collected once for both: dV carries Q^T dO, dK its transpose dO^T Q.
+// dK + dV with d == e from scanned states that are collected once for both: dK carries dO^T Q, dV its transpose Q^T dO.
+// It is dK's that is collected: there the decay factors, and with them the rounding to 16 bits, fall on Q, and dO stays as
+// it is.  In fp16 numbers below 6e-5 lose bits, and gradients get that small where activations do not.  Error (2-norm,
+// against 64 bits) of dK / dV, fp16, b1 h16 n8192 d128 with decay: separate sweeps - dK's states for both - dV's for both
+//     dO of 1e-5:  3.77e-4 / 1.70e-3   3.77e-4 / 1.61e-3   6.46e-4 / 1.70e-3
+//     Q of 1e-4:   3.54e-4 / 3.32e-4   3.54e-4 / 3.35e-4   (of 1e-5: dV 3.77e-4, 6.45e-4)
+// From Q of 1e-3 and dO of 1e-4 up, and in bf16 at any magnitude, all three agree to three digits.
 // `nchunk` chunks of `chunk_len` blocks per sweep, collected as `ncollect` chunks of chunk_len / mul blocks (one
 // sweep collects, so there are CUs for mul times as many chunks).  nchunk == 1: not for this shape.
 struct SharedPlan {
@@ -424,6 +430,8 @@ static SweepPair chunked(const SweepIO& io, const float* s, int64_t bh, int64_t 
 // Where the forward pass runs in chunks from scanned states and the state tile is square, the slots it leaves behind
 // serve the dQ sweep of the backward pass (same chunks, transposed states): no collect and scan launches there.
 // b1 h16 n32768 d128 without decay: dQ 60 + 8 + 97 us -> 97; with the shared collect of dK + dV fwd + bwd 494 -> 416 us.
+// dQ's own states would round K times the decay factors, these round V times them: the same error to three digits from V of
+// 1e-3 up and in bf16 at any magnitude; fp16 with V of 1e-4 3.33e-4 / 3.38e-4, of 1e-5 (where O is off by 1.7e-3) 3.79e-4 / 8.66e-4.
 // nchunk == 1: not for this shape.
 SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts) {
     const SavedPlan none = {1, 0, 0, 0, 0};
@@ -461,9 +469,9 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
     const SharedPlan sh = dk == dv && ws_ok ? plan_shared(bh, n, dk, ws_bytes, opts) : SharedPlan{1, 0, 0, 1, 0, 0.0};
     SweepPair p;
     if (sh.nchunk > 1) {
-        // io0 (dK) and io1 (dV) have y and z swapped: io1's states, and for io0 their transposes
+        // io0 (dK) and io1 (dV) have y and z swapped: io0's states, and for io1 their transposes
         const int width = square_width(dk, dv);
-        p = chunked(io1, s, bh, h, n, dk, dv, width, sh.ncollect, sh.chunk_len / sh.mul, static_cast<float*>(ws));
+        p = chunked(io0, s, bh, h, n, dk, dv, width, sh.ncollect, sh.chunk_len / sh.mul, static_cast<float*>(ws));
         const int rc = sweep_pipe_collect(p, dtype, reverse, st);
         if (rc != LA_OK) return rc;
         p = chunked(io0, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws));
@@ -472,7 +480,7 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
         p.shared = 1;
         p.nslot = sh.ncollect - 1;
         p.slot_mul = sh.mul;
-        p.transposed = 1;
+        p.transposed = 2;
         return sweep_pipe_apply(p, dtype, reverse, st);
     }
     p.nprod = 2;
