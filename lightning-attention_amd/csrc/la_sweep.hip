@@ -236,21 +236,25 @@ struct SharedPlan {
     double us;
 };
 // In place of a collect of both sweeps it always pays (b1 h16 n32768 d128 without decay: collect + scan 105 + 7 -> 63 + 8
-// us).  Against two single walks that fill the chip in 64-column workgroups - which are then bound by the memory system and
-// take 1.95 us per block, not the 1.4 of block_us - the two extra launches have to be earned back: fwd + bwd at 64
-// sequences of d128, without / with: n = 1600 104 / 110 us, 2048 134 / 139, 4096 302 / 291, 16384 887 / 855.
+// us).  Against two single walks in 64-column workgroups that take more than half of the chip - bound by the memory system
+// then, and slower than block_us says - the two extra launches have to be earned back.  With three chunks per sweep (33 .. 40
+// sequences) that takes 40 blocks; with two (41 .. 64 sequences) the walk is only halved, and it takes about 96.  la_bwd
+// of d128 with a carried dQ, dK + dV paired / shared, us, at 41 - 48 - 64 sequences:
+//     n = 3584  113 / 117 - 116 / 123 - 153 / 162     n = 5120  154 / 153 - 160 / 162 - 191 / 189
+//     n = 6144  183 / 181 - 192 / 191 - 227 / 226     n = 16384  470 / 448 - 502 / 489 - 623 / 580
+// `us` is what sweep_bwd_once weighs its own launch by, so without a shared plan it is by block_us as there.
 static SharedPlan plan_shared(int64_t bh, int64_t n, int64_t d, size_t scratch, const Opts& opts) {
     const int own_width = column_width(bh, n, d, d, 2, scratch, opts), width = square_width(d, d);
     const int64_t nblk = (n + 63) / 64, cus = num_cus(), units8 = (bh + 7) / 8 * 8;
-    SharedPlan none = {1, 0, 0, 1, 0, width_us(bh, n, d, d, 2, own_width, scratch, opts)};
-    if (own_width == 0 && d > 64 && d <= 128 && units8 * slices(d, d, 0) * 4 > cus) none.us *= 1.95 / 1.4;
+    const SharedPlan none = {1, 0, 0, 1, 0, width_us(bh, n, d, d, 2, own_width, scratch, opts)};
+    const bool crowded = own_width == 0 && d > 64 && d <= 128 && units8 * slices(d, d, 0) * 4 > cus;
     if (width < 0 || !own_choices(opts)) return none;
     const ScanPlan own = plan_scan(bh, n, d, d, 2, own_width, opts);
     const bool scanned = own.nchunk > 1 && own.bytes <= scratch;
     int64_t c = cus / (2 * units8);
     if (c > nblk / 4) c = nblk / 4;
     if (c > 32) c = 32;
-    if (c < 2 || bh > 65535) return none;
+    if (c < 2 || bh > 65535 || (crowded && c == 2 && nblk < 96)) return none;
     int64_t mul = cus / (units8 * c);
     if (mul > 2) mul = 2;
     SharedPlan pl;
@@ -262,7 +266,7 @@ static SharedPlan plan_shared(int64_t bh, int64_t n, int64_t d, size_t scratch, 
     if (pl.nchunk < 2) return none;
     pl.bytes = (size_t)bh * (size_t)(pl.ncollect - 1) * pipe_state_floats((int)d, width) * sizeof(float);
     pl.us = (0.5 * (double)len + (double)pl.chunk_len) * block_us(d, width) + 16.0 + 10.0 + (scanned ? 0.0 : 10.0);
-    return pl.us < none.us && pl.bytes <= scratch ? pl : none;
+    return pl.us < none.us * (crowded ? 1.95 / 1.4 : 1.0) && pl.bytes <= scratch ? pl : none;
 }
 
 // Workspace the kernels can use for one launch of nprod sweeps (0: none).
@@ -513,8 +517,10 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
         const double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) +
                                 plan_shared(bh, n, d, scratch, opts).us;
         // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
-        const double rounds = wgs > cus ? 2.0 : 1.0;
-        if (rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) >= separate) return LA_E_UNSUPPORTED;
+        // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
+        // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
+        const double rounds = wgs > cus ? 2.0 : 1.0, launch = wgs > cus ? 1.5 : 0.0;
+        if (rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) >= separate + launch) return LA_E_UNSUPPORTED;
     }
     SweepBoth b;
     b.fwd.nprod = 1;

@@ -1,0 +1,21 @@
+"""The planner's choices where they are close, by the launches that a call is mapped onto (no GPU; 256 compute units)."""
+import pytest
+
+from launch_routes import routes
+
+BF16 = 0
+
+
+@pytest.mark.parametrize("d", [104, 128])
+def test_backward_of_41_to_64_sequences(d):
+    """One launch of 64-column workgroups would take two rounds here (la_bwd, b*h = 48, n = 2048, d = 128: 97 us); dQ, then dK + dV
+    paired, take 87.  Shared states only on longer walks; up to 40 sequences one launch is one round."""
+    got = routes([(bh, n, d, d, BF16) for bh in (33, 40, 41, 48, 56, 64) for n in (256, 512, 1024, 1600, 2048, 3072, 3584, 5120, 8192)])
+    for (bh, n, *_), r in got.items():
+        if bh <= 40:
+            assert ("once" in r["bwd"]) == (n <= 5120), (bh, n, r)
+        elif n == 256:
+            assert "once" in r["bwd"], (bh, n, r)  # (19.3 against 19.9)
+        else:
+            assert "once" not in r["bwd"] and ("shared" in r["bwd"]) == (n == 8192), (bh, n, r)
+            assert n == 8192 or "sweep rev warm w0 x2 c1;" in r["bwd"], (bh, n, r)
