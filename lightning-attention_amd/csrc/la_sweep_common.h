@@ -119,11 +119,6 @@ struct SweepPair {
     int mode;
     int chunk_len;
     float* state;
-    // kApply from states that another launch over the same tensors collected: `shared` says that there is one set of
-    // slots per unit and slice for all sweeps of the launch, nslot slots to a set, chunk c starting from slot
-    // c * slot_mul - 1; bit i of `transposed`: sweep i has y and z in swapped roles, its state is the transpose of
-    // the collected one (square tiles of state only: feature dim as padded == columns of a workgroup).
-    int shared = 0, nslot = 0, slot_mul = 1, transposed = 0;
     // Forward walk in one piece (pipelined kernel, 64-column workgroups): after every save_len blocks but the
     // last the state is also written to `save`, per unit (number of such boundaries) row-major dk x dv float
     // matrices.  The sweep (x', y' = z, z' = y) then has exactly the transposed state at those boundaries
@@ -134,6 +129,11 @@ struct SweepPair {
     // x, y and z are pre-activations: the kernel applies SiLU to them as it loads them (forward sweeps of
     // the pipelined kernel at feature dims up to 128)
     int silu = 0;
+    // kApply from states that another launch over the same tensors collected: `shared` says that there is one set of
+    // slots per unit and slice for all sweeps of the launch, nslot slots to a set, chunk c starting from slot
+    // c * slot_mul - 1; bit i of `transposed`: sweep i has y and z in swapped roles, its state is the transpose of
+    // the collected one (square tiles of state only: feature dim as padded == columns of a workgroup).
+    int shared = 0, nslot = 0, slot_mul = 1, transposed = 0;
 };
 
 // One launch can also carry sweeps of both directions: the whole backward pass when d == e, dQ walking

@@ -70,7 +70,10 @@ struct PipeLds {
 // `bid`: number of the workgroup within its part of the launch.
 // SILU: x, y and z pass through SiLU on their way from memory into LDS (the attention block's activation on
 // q, k, v, examples/module/tnl_attn.py:51-54, fused into the forward pass).
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
+// SHARED: a kApply launch from shared or transposed slots (SweepPair::shared); an instantiation of its own, because the slot
+// arithmetic and the transposed load cost every other launch of the form 1 - 2 % (la_bwd of b1 h88 n8192 d64 e40 205.2 us
+// with them, 202.2 without; la_fwd of b1 h8 n113 d64 6.68 / 6.53).
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
 __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const unsigned bid) {
     typedef Mma<T> M;
     typedef typename M::V8 V8;
@@ -254,11 +257,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const int64_t it_end = cend;
     // the state slot of this workgroup's chunk: [unit][sweep][slice][chunk 0 .. nchunk-2][state waves' accumulators]
     constexpr size_t SF = (size_t)4 * NH * KT * 64 * 4;
-    // the forms whose tile of state is square, so that a sweep can start from another one's transposed state
-    constexpr bool TRANSPOSES = NF == 1 && 4 * NH == KT && !SILU;
-    const bool shared = TRANSPOSES && pair.shared;
-    const size_t slot_set = shared ? (size_t)unit * nslice + slice : ((size_t)unit * nprod + sub % nprod) * nslice + slice;
-    float* const slot0 = pair.state + slot_set * (size_t)(shared ? pair.nslot : nchunk - 1) * SF;
+    static_assert(!SHARED || (NF == 1 && 4 * NH == KT && !SILU), "only a square tile of state can be another sweep's transposed one");
+    const size_t slot_set = SHARED ? (size_t)unit * nslice + slice : ((size_t)unit * nprod + sub % nprod) * nslice + slice;
+    float* const slot0 = pair.state + slot_set * (size_t)(SHARED ? pair.nslot : nchunk - 1) * SF;
 
     u32x4 xrA[XC], yrA[XC], zrA[ZC], xrB[XC], yrB[XC], zrB[ZC];
 
@@ -848,9 +849,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
         // this lane's part of a state slot: [wave][slab][tile][lane] accumulator quartets
         const size_t lane_slot = ((size_t)w * NH * KT * 64 + lane) * 4;
         const bool resume = mode == kApply && chunk > 0;
-        const float* const slot = slot0 + (size_t)(shared ? chunk * pair.slot_mul - 1 : chunk - 1) * SF;
+        const float* const slot = slot0 + (size_t)(SHARED ? chunk * pair.slot_mul - 1 : chunk - 1) * SF;
         const float* const src = slot + lane_slot;
-        if constexpr (TRANSPOSES) {
+        if constexpr (SHARED) {
             if (resume && ((pair.transposed >> (sub % nprod)) & 1)) {
                 // state[k][c] = slot[c][k]: tile (kt; NH w + h) is the transpose of the slot's tile (NH w + h; kt)
 #pragma unroll
@@ -911,9 +912,9 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     }
 }
 
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
 __global__ __launch_bounds__(512, 1) void la_sweep_pipe_kernel(SweepPair pair) {
-    sweep_pipe_body<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>(pair, blockIdx.x);
+    sweep_pipe_body<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>(pair, blockIdx.x);
 }
 
 // Forward-walking and backward-walking sweeps in one launch (SweepBoth).
@@ -924,21 +925,21 @@ __global__ __launch_bounds__(512, 1) void la_sweep_pipe_both_kernel(SweepBoth bo
 }
 
 // What a kernel instantiation needs once per device before its first launch (its dynamic LDS limit raised).
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
 static int prep_one() {
     constexpr size_t lds = PipeLds<DKP, NF, NH>::bytes(sizeof(T));
     static_assert(lds <= 160 * 1024, "LDS budget");
     static unsigned char lds_allowed[kMaxDevices];
-    return allow_lds(la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>, lds, lds_allowed);
+    return allow_lds(la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>, lds, lds_allowed);
 }
 
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
 static int launch_one(const SweepPair& pair, hipStream_t st) {
     const SweepArgs& a = pair.a[0];
     constexpr size_t lds = PipeLds<DKP, NF, NH>::bytes(sizeof(T));
-    auto kern = la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>;
-    if (const int e = prep_one<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>()) return e;
-    if (SILU != (pair.silu != 0)) return LA_E_UNSUPPORTED;
+    auto kern = la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>;
+    if (const int e = prep_one<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>()) return e;
+    if (SILU != (pair.silu != 0) || SHARED != (pair.shared != 0)) return LA_E_UNSUPPORTED;
     const int units8 = (a.bh + 7) / 8 * 8;
     // the slice width the host chose must be one this instantiation's LDS slot and state waves hold
     if (a.zw <= 0 || a.zw > 64 * NH || a.zw % (16 * NH)) return LA_E_UNSUPPORTED;
@@ -950,10 +951,10 @@ static int launch_one(const SweepPair& pair, hipStream_t st) {
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
     if (pair.mode == kResume && (!RESUMES || pair.nprod != 1)) return LA_E_UNSUPPORTED;
-    if (pair.shared && (NF != 1 || 4 * NH != DKP / 16 || SILU || a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
-    if (pair.transposed && !pair.shared) return LA_E_UNSUPPORTED;
+    if (SHARED && (a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
+    if (pair.transposed && !SHARED) return LA_E_UNSUPPORTED;
     // every chunk's slot must exist
-    if (pair.shared && (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot)) return LA_E_WORKSPACE;
+    if (SHARED && (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot)) return LA_E_WORKSPACE;
     if (pair.save && (!SAVES || pair.nprod != 1 || pair.mode != kWarmUp || a.nchunk != 1)) return LA_E_UNSUPPORTED;
     const unsigned grid = (unsigned)(units8 * a.nslice * a.nchunk * pair.nprod);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, pair);
@@ -997,6 +998,12 @@ static int prep_family() {
     LA_P(false, false, false) LA_P(false, false, true) LA_P(false, true, false) LA_P(false, true, true)
     LA_P(true, false, false) LA_P(true, false, true) LA_P(true, true, false) LA_P(true, true, true)
 #undef LA_P
+    if constexpr (NF == 1 && 4 * NH == DKP / 16) {
+#define LA_P(R, D, S) if (!e) e = prep_one<T, DKP, NF, NH, R, D, S, false, true>();
+        LA_P(false, false, false) LA_P(false, false, true) LA_P(false, true, false) LA_P(false, true, true)
+        LA_P(true, false, false) LA_P(true, false, true) LA_P(true, true, false) LA_P(true, true, true)
+#undef LA_P
+    }
     if constexpr (NH == 1) {
 #define LA_P(D, S) if (!e) e = prep_both_one<T, DKP, NF, D, S>();
         LA_P(false, false) LA_P(false, true) LA_P(true, false) LA_P(true, true)
