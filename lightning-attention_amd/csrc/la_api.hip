@@ -14,7 +14,7 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
 int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                       int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st);
 int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk,
-                       int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
+                       int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st);
 int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv,
            int dtype, bool reverse, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st);
 size_t sweep_workspace_bytes(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int dtype, const Opts& opts);
@@ -162,19 +162,20 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
     const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : kNoPlan;
     const SavedPlan cp = sv.p && sv.carry && pl.nchunk <= 1 ? plan_carry(b * h, n, d, e, dtype, opts) : kNoPlan;
     const bool carried = saved_usable(sv, cp);
+    const double dq_us = carried ? carried_us(e, cp) : 0.0;  // (0: dQ by its own plan)
     if (d == e && dtype != LA_FP32) {
         // few sequences: all three gradients in one launch, side by side (LA_E_UNSUPPORTED: not this time)
         rc = sweep_bwd_once(io(dout, v, k, dq), io(v, dout, q, dk), io(k, q, dout, dv), s, b * h, h, n, d, dtype, ws.p,
-                            ws.bytes, opts, carried ? carried_us(e, cp) : 0.0, st);
+                            ws.bytes, opts, dq_us, st);
         if (rc != LA_E_UNSUPPORTED) return rc;
     }
     if (d != e && dtype != LA_FP32) {
         // few sequences: all three gradients in one launch
         rc = sweep_bwd_once_de(io(dout, v, k, dq), io(v, dout, q, dk), io(k, q, dout, dv), s, b * h, h, n, d, e, dtype, ws.p,
-                               ws.bytes, opts, carried ? carried_us(e, cp) : 0.0, st);
+                               ws.bytes, opts, dq_us, st);
         if (rc != LA_E_UNSUPPORTED) return rc;
         // dQ and dK have one shape and opposite directions: with few sequences, one launch for the two
-        rc = sweep_fwd_rev_once(io(dout, v, k, dq), io(v, dout, q, dk), s, b * h, h, n, e, d, dtype, ws.p, ws.bytes, opts, st);
+        rc = sweep_fwd_rev_once(io(dout, v, k, dq), io(v, dout, q, dk), s, b * h, h, n, e, d, dtype, ws.p, ws.bytes, opts, dq_us, st);
         if (rc == LA_OK) return run(k, q, dout, dv, s, b * h, h, n, d, e, dtype, true, ws, opts, st);
         if (rc != LA_E_UNSUPPORTED) return rc;
     }

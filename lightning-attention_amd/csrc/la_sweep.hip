@@ -545,6 +545,29 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
     return sweep_pipe_both(b, dtype, st);
 }
 
+// dQ and dK of a backward pass with d != e (one shape: both contract over dk = e and produce dv = d columns): in one launch
+// of 64-column workgroups, or one after the other, and the estimated time of the better way.
+// dq_us > 0: what the dQ sweep alone would take from states the forward pass left.
+// (together: up to three rounds of workgroups; where each sweep alone leaves its last round mostly empty, the two need
+// fewer rounds - d192 e128 b*h = 96, 288 workgroups a sweep: la_bwd 0.215 against 0.261 ms at n = 2048; d256 e128 b*h = 80:
+// 0.229 against 0.274.  A carried dQ has to be estimated a fifth faster: with 41 .. 64 sequences all launches wait for
+// the memory system and the estimates flatter the one that reads more.  la_bwd together / carried, us, d128 e96: b*h = 24, n =
+// 6016 155 / 138 (estimates 101 / 70); 48, 4096 155 / 163 (90 / 82); 48, 8192 282 / 270 (179 / 138); 56, 6016 227 / 244
+// (132 / 131); 64, 12288 476 / 504 (269 / 236).)
+struct DqDkPlan {
+    bool together;
+    double us;
+};
+static DqDkPlan plan_dq_dk(int64_t bh, int64_t n, int64_t dk, int64_t dv, size_t scratch, const Opts& opts, double dq_us) {
+    const int64_t cus = num_cus(), nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, 0) * 2;
+    const int64_t rounds = (wgs + cus - 1) / cus;
+    const double own = width_us(bh, n, dk, dv, 1, column_width(bh, n, dk, dv, 1, scratch, opts), scratch, opts);
+    const double two = (rounds > 1 ? (double)rounds : warm_up_frac(wgs, nblk)) * (double)nblk * block_us(dk, 0);
+    const double apart = (dq_us > 0.0 ? dq_us : own) + own;
+    const bool together = rounds <= 3 && two < 2.0 * own && !(dq_us > 0.0 && apart < 0.8 * two);
+    return {together, together ? two : apart};
+}
+
 // The same with d != e (both up to 128), where the three sweeps have a CU for every 64-column workgroup: side by side
 // they take as long as the longest of them, and one launch replaces two or three (fwd + bwd of b2 h20 n2048 d128 e96
 // 124 -> 91 us, b1 h40 n6000 d128 e64 210 -> 194).  Beyond one workgroup per CU the sweeps would only queue behind each other.
@@ -556,15 +579,13 @@ int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, c
     if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
     if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;
     const int64_t cus = num_cus(), nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8;
-    const int64_t wgs_a = units8 * slices(e, d, 0) * 2, wgs = wgs_a + units8 * slices(d, e, 0);
+    const int64_t wgs = units8 * (slices(e, d, 0) * 2 + slices(d, e, 0));
     if (forced == 0) {
         if (wgs > cus) return LA_E_UNSUPPORTED;
         const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
         const size_t scratch = ws_ok ? ws_bytes : 0;
-        const double a_us = width_us(bh, n, e, d, 1, column_width(bh, n, e, d, 1, scratch, opts), scratch, opts);
         const double v_us = width_us(bh, n, d, e, 1, column_width(bh, n, d, e, 1, scratch, opts), scratch, opts);
-        const double two = warm_up_frac(wgs_a, nblk) * (double)nblk * block_us(e, 0);  // dQ and dK sharing a launch
-        const double separate = std::min(two, (dq_us > 0.0 ? dq_us : a_us) + a_us) + v_us;
+        const double separate = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us).us + v_us;
         if (warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) >= separate) return LA_E_UNSUPPORTED;
     }
     SweepTrio t;
@@ -588,26 +609,17 @@ int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, c
 
 // The same for two sweeps of one shape and opposite directions (dQ and dK of a backward pass with
 // d != e: both contract over e and produce d columns): one launch where separate launches are not estimated
-// faster (they fit on the chip together, or share rounds of workgroups); LA_E_UNSUPPORTED otherwise.
+// faster (they fit on the chip together, or share rounds of workgroups); LA_E_UNSUPPORTED otherwise.  `fwd` is the sweep
+// that dq_us is about.
 int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk,
-                       int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, hipStream_t st) {
+                       int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
     if (dtype != LA_BF16 && dtype != LA_FP16) return LA_E_UNSUPPORTED;
     const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
     if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
     if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, nslice = (dv + 63) / 64;
-    const int64_t wgs = (bh + 7) / 8 * 8 * nslice * 2;
     if (forced == 0) {
-        // (up to three rounds of workgroups: where each sweep alone leaves its last round mostly empty, the two
-        // together need fewer rounds - d192 e128 b*h = 96, 288 workgroups a sweep: la_bwd 0.215 against 0.261 ms at
-        // n = 2048; d256 e128 b*h = 80: 0.229 against 0.274)
-        if (wgs > 3 * cus) return LA_E_UNSUPPORTED;
         const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-        const size_t scratch = ws_ok ? ws_bytes : 0;
-        const double separate = 2.0 * width_us(bh, n, dk, dv, 1, column_width(bh, n, dk, dv, 1, scratch, opts), scratch, opts);
-        const int64_t rounds = (wgs + cus - 1) / cus;
-        const double share = rounds > 1 ? (double)rounds : warm_up_frac(wgs, nblk);
-        if (share * (double)nblk * block_us(dk, false) >= separate) return LA_E_UNSUPPORTED;
+        if (!plan_dq_dk(bh, n, dk, dv, ws_ok ? ws_bytes : 0, opts, dq_us).together) return LA_E_UNSUPPORTED;
     }
     SweepBoth b;
     b.fwd.nprod = b.rev.nprod = 1;

@@ -19,3 +19,15 @@ def test_backward_of_41_to_64_sequences(d):
         else:
             assert "once" not in r["bwd"] and ("shared" in r["bwd"]) == (n == 8192), (bh, n, r)
             assert n == 8192 or "sweep rev warm w0 x2 c1;" in r["bwd"], (bh, n, r)
+
+
+@pytest.mark.parametrize("d, e", [(128, 96), (96, 128)])
+def test_carried_dq_is_weighed_by_every_other_form(d, e):
+    """d != e, states carried from the forward pass: la_bwd in one launch for dQ + dK, against a carried dQ, takes 155 / 138 us at
+    b*h = 24, n = 6016, 282 / 270 at 48, 8192, but 155 / 163 at 48, 4096 and 238 / 265 at 64, 6016."""
+    got = routes([(bh, n, d, e, BF16) for bh, n in ((24, 5120), (24, 6016), (32, 7168), (48, 8192), (48, 4096), (56, 6016), (64, 6016), (64, 12288))])
+    for (bh, n, *_), r in got.items():
+        if bh == 48 and n == 4096 or bh > 48:
+            assert r["bwd"].startswith("dq+dk"), (bh, n, r)
+        else:
+            assert r["bwd"].startswith(("apply apply w1 x1", "trio")), (bh, n, r)
