@@ -28,7 +28,7 @@ int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int
                    float* carry, const SavedPlan& pl, hipStream_t st);
 int sweep_carried(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                   const float* carry, const SavedPlan& pl, hipStream_t st);
-double carried_us(int64_t e, const SavedPlan& pl);
+double kept_us(int64_t n, int64_t e, const SavedPlan& pl);
 int prepare_srmsnorm();   // srmsnorm.hip
 int prepare_norm_gate();  // norm_gate.hip
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
@@ -162,7 +162,7 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
     const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : kNoPlan;
     const SavedPlan cp = sv.p && sv.carry && pl.nchunk <= 1 ? plan_carry(b * h, n, d, e, dtype, opts) : kNoPlan;
     const bool carried = saved_usable(sv, cp);
-    const double dq_us = carried ? carried_us(e, cp) : 0.0;  // (0: dQ by its own plan)
+    const double dq_us = carried ? kept_us(n, e, cp) : saved_usable(sv, pl) ? kept_us(n, e, pl) : 0.0;  // (0: dQ by its own plan)
     if (d == e && dtype != LA_FP32) {
         // few sequences: all three gradients in one launch, side by side (LA_E_UNSUPPORTED: not this time)
         rc = sweep_bwd_once(io(dout, v, k, dq), io(v, dout, q, dk), io(k, q, dout, dv), s, b * h, h, n, d, dtype, ws.p,

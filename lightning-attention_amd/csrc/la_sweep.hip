@@ -459,8 +459,13 @@ int sweep_carried(const SweepIO& io, const float* s, int64_t bh, int64_t h, int6
     p.transposed = 1;
     return sweep_pipe_apply(p, dtype, false, st);
 }
-// Estimated duration (us) of that launch.
-double carried_us(int64_t e, const SavedPlan& pl) { return (double)pl.chunk_len * block_us(e, pl.dq_width); }
+// Estimated duration (us) of the dQ sweep from what the forward pass left by plan_saved or plan_carry; 0: leave it out of the account.
+// (Left out: plain matrices on walks below 40 blocks, where with 65 .. 80 sequences at d 97 .. 128 one launch of almost two rounds is
+// still as fast: fwd + bwd of b1 h80 n1792 d128 131 us without states, 136 with; h72 n2560 179 / 179.5, n8192 545 / 528.)
+double kept_us(int64_t n, int64_t e, const SavedPlan& pl) {
+    const bool matrices = pl.fwd_width != pl.dq_width;
+    return matrices && (n + 63) / 64 < 40 ? 0.0 : (double)pl.chunk_len * block_us(e, pl.dq_width);
+}
 
 // Two sweeps of the same shape and direction in one launch.
 int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv,

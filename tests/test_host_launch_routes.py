@@ -31,3 +31,11 @@ def test_carried_dq_is_weighed_by_every_other_form(d, e):
             assert r["bwd"].startswith("dq+dk"), (bh, n, r)
         else:
             assert r["bwd"].startswith(("apply apply w1 x1", "trio")), (bh, n, r)
+
+
+def test_saved_matrices_are_weighed_by_the_one_launch_form():
+    """65 .. 80 sequences at d = 128: the forward pass leaves matrices, and from 40 blocks on the backward pass starts dQ from them
+    rather than running everything in one launch (fwd + bwd of b*h = 72: n = 8192 528 / 549 us, n = 32768 2108 / 2246)."""
+    got = routes([(bh, n, 128, 128, BF16) for bh in (65, 72, 80) for n in (2560, 4096, 32768)])
+    for key, r in got.items():
+        assert "saving" in r["fwd"] and "sweep resume" in r["bwd"], (key, r)
