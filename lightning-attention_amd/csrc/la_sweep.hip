@@ -519,8 +519,12 @@ int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, cons
         // what the separate launches would take, by the estimates behind their own plans
         const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
         const size_t scratch = ws_ok ? ws_bytes : 0;
-        const double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) +
-                                plan_shared(bh, n, d, scratch, opts).us;
+        const SharedPlan sh = plan_shared(bh, n, d, scratch, opts);
+        double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
+        // Short rows and a shared plan of two chunks per sweep: more than the last-level cache holds, the separate launches
+        // take as long as their twelve passes over a tensor (this launch: ten), not as long as their blocks.  la_bwd of d64, separate /
+        // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
+        if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.4e6);
         // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
         // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
         // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
