@@ -593,8 +593,17 @@ int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, c
         if (wgs > cus) return LA_E_UNSUPPORTED;
         const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
         const size_t scratch = ws_ok ? ws_bytes : 0;
-        const double v_us = width_us(bh, n, d, e, 1, column_width(bh, n, d, e, 1, scratch, opts), scratch, opts);
-        const double separate = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us).us + v_us;
+        const int v_width = column_width(bh, n, d, e, 1, scratch, opts);
+        const DqDkPlan q = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us);
+        double separate = q.us + width_us(bh, n, d, e, 1, v_width, scratch, opts);
+        // Rows of d above 96 against rows of e = 49 .. 64, chunked: block_us is 11 % too long for the two sweeps over e, and a scanned dV takes
+        // 5 us less than estimated (10 with up to 8 sequences).  la_bwd of e64, one launch / dQ + dK and dV, us, d128: b*h = 8, n = 4096 60 / 62,
+        // 5120 74 / 71, 6016 86 / 80; 16, 4096 65 / 68, 6016 92 / 90; 24, 6016 103 / 107, 8192 138 / 135, 16384 278 / 254.  Rows of
+        // d = 97 .. 112 only with up to 8 sequences (d104: 8, 5120 74 / 71, but 24, 8192 142 / 151), narrower ones nowhere (e40: 8, 6016 73 / 79).
+        if (d > 96 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d > 112 || units8 == 8)) {
+            const ScanPlan v = plan_scan(bh, n, d, e, 1, v_width, opts);
+            separate -= 0.11 * q.us + (v.nchunk > 1 && v.bytes <= scratch ? (units8 == 8 ? 10.0 : 5.0) : 0.0);
+        }
         if (warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) >= separate) return LA_E_UNSUPPORTED;
     }
     SweepTrio t;

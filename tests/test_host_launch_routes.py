@@ -47,3 +47,11 @@ def test_long_walks_of_short_rows_read_no_more_than_they_must():
     got = routes([(bh, n, d, d, BF16) for bh, n, d in ((64, 24576, 64), (64, 65536, 64), (56, 49152, 64), (52, 49152, 64), (41, 32768, 64), (64, 65536, 40))])
     for (bh, n, d, *_), r in got.items():
         assert ("once" in r["bwd"]) == (d == 64 and bh > 41), (bh, n, d, r)
+
+
+def test_one_launch_for_three_sweeps_of_different_rows():
+    """d = 128, e = 64: three sweeps in one launch where that measures faster than dQ + dK in one and dV scanned."""
+    got = routes([(bh, n, 128, 64, BF16) for bh, n in ((8, 2048), (8, 4096), (16, 2048), (16, 4096), (24, 6016), (40, 16384))])
+    assert all(r["bwd"].startswith("trio") for r in got.values()), got
+    got = routes([(bh, n, 128, 64, BF16) for bh, n in ((1, 5120), (8, 5120), (8, 6016), (16, 6016), (24, 12288), (24, 16384))])
+    assert all(r["bwd"].startswith("dq+dk") for r in got.values()), got
