@@ -23,6 +23,7 @@ int sweep_saving(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64
                  float* save, int save_len, int width, hipStream_t st);
 int sweep_resumed(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                   const float* saved, int nchunk, int chunk_len, int width, hipStream_t st);
+bool reads_kept(int64_t bh, int64_t n, int64_t d, int64_t e, const SavedPlan& pl, const Opts& opts);
 SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts);
 int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                    float* carry, const SavedPlan& pl, hipStream_t st);
@@ -323,7 +324,8 @@ extern "C" size_t la_carry_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int
     const la::Opts& o = opts ? *opts : la::kAuto;
     if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
     const la::SavedPlan pl = la::plan_saved(b * h, n, d, e, dtype, o);
-    return pl.nchunk > 1 ? pl.bytes : la::plan_carry(b * h, n, d, e, dtype, o).bytes;
+    if (pl.nchunk > 1) return la::reads_kept(b * h, n, d, e, pl, o) ? pl.bytes : 0;
+    return la::plan_carry(b * h, n, d, e, dtype, o).bytes;
 }
 
 namespace la {

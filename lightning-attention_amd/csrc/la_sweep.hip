@@ -431,19 +431,23 @@ static SweepPair chunked(const SweepIO& io, const float* s, int64_t bh, int64_t 
     return p;
 }
 
+bool reads_kept(int64_t bh, int64_t n, int64_t d, int64_t e, const SavedPlan& pl, const Opts& opts);  // (below)
+
 // Where the forward pass runs in chunks from scanned states and the state tile is square, the slots it leaves behind
 // serve the dQ sweep of the backward pass (same chunks, transposed states): no collect and scan launches there.
 // b1 h16 n32768 d128 without decay: dQ 60 + 8 + 97 us -> 97; with the shared collect of dK + dV fwd + bwd 494 -> 416 us.
 // dQ's own states would round K times the decay factors, these round V times them: the same error to three digits from V of
 // 1e-3 up and in bf16 at any magnitude; fp16 with V of 1e-4 3.33e-4 / 3.38e-4, of 1e-5 (where O is off by 1.7e-3) 3.79e-4 / 8.66e-4.
-// nchunk == 1: not for this shape.
+// nchunk == 1: not for this shape, or nothing the backward pass would read.
 SavedPlan plan_carry(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, const Opts& opts) {
     const SavedPlan none = {1, 0, 0, 0, 0};
     const int width = square_width(d, e);
     if ((dtype != LA_BF16 && dtype != LA_FP16) || width < 0 || !own_choices(opts)) return none;
     if (column_width(bh, n, d, e, 1, (size_t)-1, opts) != width) return none;
     const ScanPlan pl = plan_scan(bh, n, d, e, 1, width, opts);
-    return pl.nchunk > 1 ? SavedPlan{pl.nchunk, pl.chunk_len, pl.bytes, width, width} : none;
+    if (pl.nchunk < 2) return none;
+    const SavedPlan got = {pl.nchunk, pl.chunk_len, pl.bytes, width, width};
+    return reads_kept(bh, n, d, e, got, opts) ? got : none;
 }
 // The forward sweep by that plan, its slots in `carry`.
 int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
@@ -498,39 +502,44 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
     return launch_planned(p, bh, n, dk, dv, dtype, reverse, ws, ws_bytes, opts, st);
 }
 
+// What the launch options say about every sweep of a backward pass in one launch: -1 never, 1 whenever possible, 0 where estimated faster.
+static int once_forced(const Opts& opts) {
+    if (opts.once == LA_OPT_OFF || opts.paired == LA_OPT_OFF) return -1;
+    if (opts.once == LA_OPT_ON) return 1;
+    return opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL ? -1 : 0;  // wider workgroups asked for
+}
+static size_t usable_bytes(const void* ws, size_t ws_bytes) { return ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0 ? ws_bytes : 0; }
+
 // The three sweeps of a backward pass with d == e (dQ forward; dK, dV reverse, paired) in ONE launch,
 // where that is the faster way: they fit on the chip together, so they run side by side, each cut into
-// the warm-up chunks the CUs left over allow.  Results are bit-identical to separate launches.
-// Returns LA_E_UNSUPPORTED when separate launches are to be used (they are estimated faster - scanned
-// chunk states on a long walk -, or the sweeps fill the chip anyway).  opts.once = LA_OPT_OFF / LA_OPT_ON:
-// never / whenever possible.  dq_us > 0: what the dQ sweep alone would take from states the forward pass left.
+// the warm-up chunks the CUs left over allow.  Results are bit-identical to separate launches of warm-up chunks
+// (states that separate launches scan, share or carry are summed in another order).
+// Not where separate launches are to be used (they are estimated faster - scanned chunk states on a long walk -, or the
+// sweeps fill the chip anyway).  dq_us > 0: what the dQ sweep alone would take from states the forward pass left.
+static bool once_chosen(int64_t bh, int64_t n, int64_t d, size_t scratch, const Opts& opts, double dq_us) {
+    if (const int forced = once_forced(opts)) return forced > 0;
+    const int64_t cus = num_cus(), nblk = (n + 63) / 64, nslice = (d + 63) / 64;
+    const int64_t wgs = (bh + 7) / 8 * 8 * nslice * 3;  // one chunk each
+    // (up to two rounds of workgroups: on a short walk one launch of twice as many 64-column workgroups as
+    // there are CUs still beats two launches - b1 h48 n2048 d192: la_bwd 0.138 against 0.162 ms)
+    if (wgs > 2 * cus) return false;
+    // what the separate launches would take, by the estimates behind their own plans
+    const SharedPlan sh = plan_shared(bh, n, d, scratch, opts);
+    double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
+    // Short rows and a shared plan of two chunks per sweep: more than the last-level cache holds, the separate launches
+    // take as long as their twelve passes over a tensor (this launch: ten), not as long as their blocks.  la_bwd of d64, separate /
+    // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
+    if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.4e6);
+    // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
+    // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
+    // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
+    const double rounds = wgs > cus ? 2.0 : 1.0, launch = wgs > cus ? 1.5 : 0.0;
+    return rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) < separate + launch;
+}
 int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                    int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
     if (dtype != LA_BF16 && dtype != LA_FP16) return LA_E_UNSUPPORTED;
-    const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
-    if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
-    if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;  // wider workgroups asked for
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, nslice = (d + 63) / 64;
-    const int64_t wgs = (bh + 7) / 8 * 8 * nslice * 3;  // one chunk each
-    if (forced == 0) {
-        // (up to two rounds of workgroups: on a short walk one launch of twice as many 64-column workgroups as
-        // there are CUs still beats two launches - b1 h48 n2048 d192: la_bwd 0.138 against 0.162 ms)
-        if (wgs > 2 * cus) return LA_E_UNSUPPORTED;
-        // what the separate launches would take, by the estimates behind their own plans
-        const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-        const size_t scratch = ws_ok ? ws_bytes : 0;
-        const SharedPlan sh = plan_shared(bh, n, d, scratch, opts);
-        double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
-        // Short rows and a shared plan of two chunks per sweep: more than the last-level cache holds, the separate launches
-        // take as long as their twelve passes over a tensor (this launch: ten), not as long as their blocks.  la_bwd of d64, separate /
-        // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
-        if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.4e6);
-        // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
-        // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
-        // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
-        const double rounds = wgs > cus ? 2.0 : 1.0, launch = wgs > cus ? 1.5 : 0.0;
-        if (rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) >= separate + launch) return LA_E_UNSUPPORTED;
-    }
+    if (!once_chosen(bh, n, d, usable_bytes(ws, ws_bytes), opts, dq_us)) return LA_E_UNSUPPORTED;
     SweepBoth b;
     b.fwd.nprod = 1;
     b.fwd.a[0] = make_args(dq, s, bh, h, n, d, d);
@@ -580,32 +589,30 @@ static DqDkPlan plan_dq_dk(int64_t bh, int64_t n, int64_t dk, int64_t dv, size_t
 // The same with d != e (both up to 128), where the three sweeps have a CU for every 64-column workgroup: side by side
 // they take as long as the longest of them, and one launch replaces two or three (fwd + bwd of b2 h20 n2048 d128 e96
 // 124 -> 91 us, b1 h40 n6000 d128 e64 210 -> 194).  Beyond one workgroup per CU the sweeps would only queue behind each other.
-// LA_E_UNSUPPORTED otherwise.
+static int64_t trio_wgs(int64_t bh, int64_t d, int64_t e) { return (bh + 7) / 8 * 8 * (slices(e, d, 0) * 2 + slices(d, e, 0)); }
+static bool trio_chosen(int64_t bh, int64_t n, int64_t d, int64_t e, size_t scratch, const Opts& opts, double dq_us) {
+    if (d > 128 || e > 128) return false;
+    if (const int forced = once_forced(opts)) return forced > 0;
+    const int64_t cus = num_cus(), nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8, wgs = trio_wgs(bh, d, e);
+    if (wgs > cus) return false;
+    const int v_width = column_width(bh, n, d, e, 1, scratch, opts);
+    const DqDkPlan q = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us);
+    double separate = q.us + width_us(bh, n, d, e, 1, v_width, scratch, opts);
+    // Rows of d above 96 against rows of e = 49 .. 64, chunked: block_us is 11 % too long for the two sweeps over e, and a scanned dV takes
+    // 5 us less than estimated (10 with up to 8 sequences).  la_bwd of e64, one launch / dQ + dK and dV, us, d128: b*h = 8, n = 4096 60 / 62,
+    // 5120 74 / 71, 6016 86 / 80; 16, 4096 65 / 68, 6016 92 / 90; 24, 6016 103 / 107, 8192 138 / 135, 16384 278 / 254.  Rows of
+    // d = 97 .. 112 only with up to 8 sequences (d104: 8, 5120 74 / 71, but 24, 8192 142 / 151), narrower ones nowhere (e40: 8, 6016 73 / 79).
+    if (d > 96 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d > 112 || units8 == 8)) {
+        const ScanPlan v = plan_scan(bh, n, d, e, 1, v_width, opts);
+        separate -= 0.11 * q.us + (v.nchunk > 1 && v.bytes <= scratch ? (units8 == 8 ? 10.0 : 5.0) : 0.0);
+    }
+    return warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) < separate;
+}
 int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                       int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
-    if ((dtype != LA_BF16 && dtype != LA_FP16) || d > 128 || e > 128) return LA_E_UNSUPPORTED;
-    const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
-    if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
-    if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8;
-    const int64_t wgs = units8 * (slices(e, d, 0) * 2 + slices(d, e, 0));
-    if (forced == 0) {
-        if (wgs > cus) return LA_E_UNSUPPORTED;
-        const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-        const size_t scratch = ws_ok ? ws_bytes : 0;
-        const int v_width = column_width(bh, n, d, e, 1, scratch, opts);
-        const DqDkPlan q = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us);
-        double separate = q.us + width_us(bh, n, d, e, 1, v_width, scratch, opts);
-        // Rows of d above 96 against rows of e = 49 .. 64, chunked: block_us is 11 % too long for the two sweeps over e, and a scanned dV takes
-        // 5 us less than estimated (10 with up to 8 sequences).  la_bwd of e64, one launch / dQ + dK and dV, us, d128: b*h = 8, n = 4096 60 / 62,
-        // 5120 74 / 71, 6016 86 / 80; 16, 4096 65 / 68, 6016 92 / 90; 24, 6016 103 / 107, 8192 138 / 135, 16384 278 / 254.  Rows of
-        // d = 97 .. 112 only with up to 8 sequences (d104: 8, 5120 74 / 71, but 24, 8192 142 / 151), narrower ones nowhere (e40: 8, 6016 73 / 79).
-        if (d > 96 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d > 112 || units8 == 8)) {
-            const ScanPlan v = plan_scan(bh, n, d, e, 1, v_width, opts);
-            separate -= 0.11 * q.us + (v.nchunk > 1 && v.bytes <= scratch ? (units8 == 8 ? 10.0 : 5.0) : 0.0);
-        }
-        if (warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) >= separate) return LA_E_UNSUPPORTED;
-    }
+    if (dtype != LA_BF16 && dtype != LA_FP16) return LA_E_UNSUPPORTED;
+    if (!trio_chosen(bh, n, d, e, usable_bytes(ws, ws_bytes), opts, dq_us)) return LA_E_UNSUPPORTED;
+    const int64_t nblk = (n + 63) / 64, wgs = trio_wgs(bh, d, e);
     SweepTrio t;
     SweepPair* const ps[3] = {&t.dq, &t.dk, &t.dv};
     const SweepIO* const ios[3] = {&dq, &dk, &dv};
@@ -627,18 +634,16 @@ int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, c
 
 // The same for two sweeps of one shape and opposite directions (dQ and dK of a backward pass with
 // d != e: both contract over e and produce d columns): one launch where separate launches are not estimated
-// faster (they fit on the chip together, or share rounds of workgroups); LA_E_UNSUPPORTED otherwise.  `fwd` is the sweep
+// faster (they fit on the chip together, or share rounds of workgroups).  `fwd` is the sweep
 // that dq_us is about.
+static bool pair_chosen(int64_t bh, int64_t n, int64_t dk, int64_t dv, size_t scratch, const Opts& opts, double dq_us) {
+    if (const int forced = once_forced(opts)) return forced > 0;
+    return plan_dq_dk(bh, n, dk, dv, scratch, opts, dq_us).together;
+}
 int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk,
                        int64_t dv, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
     if (dtype != LA_BF16 && dtype != LA_FP16) return LA_E_UNSUPPORTED;
-    const int forced = opts.once == LA_OPT_ON ? 1 : opts.once == LA_OPT_OFF ? -1 : 0;
-    if (forced < 0 || opts.paired == LA_OPT_OFF) return LA_E_UNSUPPORTED;
-    if (forced == 0 && (opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL)) return LA_E_UNSUPPORTED;
-    if (forced == 0) {
-        const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0;
-        if (!plan_dq_dk(bh, n, dk, dv, ws_ok ? ws_bytes : 0, opts, dq_us).together) return LA_E_UNSUPPORTED;
-    }
+    if (!pair_chosen(bh, n, dk, dv, usable_bytes(ws, ws_bytes), opts, dq_us)) return LA_E_UNSUPPORTED;
     SweepBoth b;
     b.fwd.nprod = b.rev.nprod = 1;
     b.fwd.a[0] = make_args(fwd, s, bh, h, n, dk, dv);
@@ -655,6 +660,15 @@ int sweep_fwd_rev_once(const SweepIO& fwd, const SweepIO& rev, const float* s, i
     }
     b.nfwd = part_grid(b.fwd);
     return sweep_pipe_both(b, dtype, st);
+}
+
+// Whether a backward pass with all the workspace it can use starts its dQ sweep from what the forward pass leaves by `pl`: that is,
+// whether dQ is a launch of its own.
+bool reads_kept(int64_t bh, int64_t n, int64_t d, int64_t e, const SavedPlan& pl, const Opts& opts) {
+    const double dq_us = kept_us(n, e, pl);
+    const size_t scratch = (size_t)-1;
+    if (d == e) return !once_chosen(bh, n, d, scratch, opts, dq_us);
+    return !trio_chosen(bh, n, d, e, scratch, opts, dq_us) && !pair_chosen(bh, n, e, d, scratch, opts, dq_us);
 }
 
 }  // namespace la

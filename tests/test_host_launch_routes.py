@@ -55,3 +55,17 @@ def test_one_launch_for_three_sweeps_of_different_rows():
     assert all(r["bwd"].startswith("trio") for r in got.values()), got
     got = routes([(bh, n, 128, 64, BF16) for bh, n in ((1, 5120), (8, 5120), (8, 6016), (16, 6016), (24, 12288), (24, 16384))])
     assert all(r["bwd"].startswith("dq+dk") for r in got.values()), got
+
+
+def test_what_is_kept_is_read():
+    """The forward pass leaves states (up to 21 MB a layer, for as long as the graph lives) only where the backward pass starts its dQ
+    sweep from them."""
+    pairs = ((128, 128), (104, 104), (96, 96), (64, 64), (40, 40), (192, 192), (128, 96), (72, 128), (64, 40), (192, 160), (128, 64))
+    lengths = (64, 512, 1024, 1600, 2048, 3072, 4096, 6016, 8192, 12288, 16384, 24576, 37888, 65536)
+    shapes = [(bh, n, d, e, BF16) for d, e in pairs for bh in (1, 8, 16, 24, 32, 40, 48, 56, 64, 72, 80, 88, 96, 128, 160) for n in lengths]
+    kept = 0
+    for once in (0, 1, 2):
+        for key, r in routes(shapes, once=once).items():
+            assert bool(r["kept"]) == ("carried" in r["bwd"] or "resume" in r["bwd"]), (once, key, r)
+            kept += bool(r["kept"])
+    assert kept > 500
