@@ -6,8 +6,8 @@
 //
 // Same data movement as the SimpleRMSNorm kernels: a row of o, g (and dy) is read once with 16-byte
 // non-temporal loads into registers, reduced, and the results written once.  TPR threads share a row:
-// 64, 128, 256, 512 or 1024, with as many rows side by side as the workgroup has room for.  The forward kernel takes one group of rows per workgroup and fetches weight and
-// bias from the caches.  The backward kernel walks the rows with a grid stride and gives every thread one
+// 64, 128, 256, 512 or 1024, with as many rows side by side as the workgroup has room for.  The forward kernel takes one
+// group of rows per workgroup and fetches weight and bias from the caches.  The backward kernel walks the rows with a grid stride and gives every thread one
 // 16-byte chunk of the row: a thread always holds the same columns, so weight and bias stay in registers
 // as floats and the column sums (d weight, d bias) are accumulated in registers over all rows a thread
 // sees (117 registers: four waves per SIMD; with more chunks per thread it ran at two).  Those partial
@@ -15,9 +15,13 @@
 // order: deterministic, no atomics.
 // The backward kernel is bound by what it keeps in flight, not by its arithmetic: with 16-bit elements the next group of
 // rows is requested before the reduction of this one (float32 runs five waves per SIMD and gains nothing), weight and
-// bias come in one 16-byte load each, and a CU holds one workgroup of 1024 threads and so writes one row of partial sums.
+// bias come in one 16-byte load each, and a CU holds one workgroup of 1024 threads and so writes one row of partial sums
+// (rows of up to 2048 elements: of four, up to 4096 of two; wider rows had such workgroups already).  Few short rows take
+// workgroups of 256 threads, a pass and a CU each: us with 1024 / with 256, bf16: [16,64] 7.2 / 6.0, [512,256] 8.0 / 6.4,
+// [1024,512] 8.3 / 7.1, [512,1024] 8.2 / 7.8.
 // Backward pass with its reduction, bf16, us before / after: [16384,2048] 87.2 / 62.9 (5.3 TB/s), [8192,1024] 33.9 / 22.6,
-// [32768,4096] 259 / 225 (6.0 TB/s), [32768,512] 42.0 / 34.7, [4096,8192] 85.5 / 65.1, [700,2048] 22.7 / 9.8.
+// [32768,4096] 259 / 225 (6.0 TB/s), [32768,512] 42.0 / 34.7, [4096,8192] 85.5 / 65.1, [700,2048] 22.7 / 9.8.  float32 has the
+// vector loads alone: [16384,4096] 252 / 236, [1024,1024] 17.4 / 14.7, [16,64] the same; one shape is slower, [16384,64] 13.2 / 14.5.
 //
 // Per element, float32 throughout:
 //   forward   xh = (o - mean) rstd ; ln = xh w + b ; sg = 1 / (1 + exp(-g)) ; y = ln sg
@@ -31,9 +35,11 @@ namespace la {
 // Threads of a workgroup: TPR threads share a row; rows of one or two wavefronts travel four or two to a
 // workgroup of 256, wider rows take a workgroup of 256, 512 or 1024 threads to themselves.
 constexpr int ng_threads(int tpr) { return tpr >= 256 ? tpr : 256; }
-// The backward kernel with 16-bit elements: always 1024 threads (its registers leave a CU 16 wavefronts either way), so
-// that a CU leaves one row of partial column sums, not four.
-constexpr int ng_bwd_threads(int tpr, int elt) { return elt == 2 ? 1024 : ng_threads(tpr); }
+// The backward kernel with 16-bit elements: 1024 threads (its registers leave a CU 16 wavefronts either way), so that a CU
+// leaves one row of partial column sums, not one per workgroup.  `few`: rows of one or two wavefronts, so few that workgroups of 256
+// threads get a CU and one pass each (ng_few): there is nothing to add up over passes then, and the rows of a 1024-thread
+// workgroup, added up one after the other, are what it waits for.
+constexpr int ng_bwd_threads(int tpr, int elt, bool few) { return elt == 2 && !few ? 1024 : ng_threads(tpr); }
 
 // both sums over the TPR threads of a row at once (every thread of the workgroup takes part)
 // ONCE: the caller hands over another 32 floats of LDS on every other call, so that the next call's writes cannot meet
@@ -153,15 +159,15 @@ __global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_fwd_kernel(const T*
 typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));  // (the workspace need not be 16-byte aligned)
 
 // `part`: gridDim.x rows of [d weight | d bias] partial column sums, 2 * cols floats each.
-template <typename T, int NV, int TPR>
-__global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T))) void norm_gate_bwd_kernel(const T* __restrict__ o, const T* __restrict__ g,
+template <typename T, int NV, int TPR, bool FEW = false>
+__global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate_bwd_kernel(const T* __restrict__ o, const T* __restrict__ g,
                                                                   const T* __restrict__ w, const T* __restrict__ b,
                                                                   const float* __restrict__ mean, const float* __restrict__ rstd,
                                                                   const T* __restrict__ dy, T* __restrict__ d_o,
                                                                   T* __restrict__ d_g, float* __restrict__ part,
                                                                   int64_t rows, int cols) {
     constexpr int E = Pack16<T>::N;
-    constexpr int RPG = ng_bwd_threads(TPR, sizeof(T)) / TPR;
+    constexpr int RPG = ng_bwd_threads(TPR, sizeof(T), FEW) / TPR;
     constexpr bool AHEAD = sizeof(T) == 2;
     __shared__ float red[64];
     __shared__ float comb[RPG > 1 ? (RPG - 1) * TPR * NV * E * 2 : 1];  // column sums of the rows beside the first
@@ -360,9 +366,15 @@ static void ng_shape(int64_t chunks, bool backward, int* tpr, int* nv) {
     }
 }
 
+// backward, 16-bit rows of up to 1024 elements: at most one group of rows of a 256-thread workgroup per CU
+static bool ng_few(int64_t rows, int tpr, int elt) {
+    const int64_t rpg = ng_threads(tpr) / tpr;
+    return elt == 2 && tpr <= 128 && (rows + rpg - 1) / rpg <= num_cus();
+}
+
 // workgroups of a launch: enough to keep every CU's memory pipeline full, never more than row groups
 static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
-    const int64_t threads = backward ? ng_bwd_threads(tpr, elt) : ng_threads(tpr), rpg = threads / tpr, groups = (rows + rpg - 1) / rpg;
+    const int64_t threads = backward ? ng_bwd_threads(tpr, elt, ng_few(rows, tpr, elt)) : ng_threads(tpr), rpg = threads / tpr, groups = (rows + rpg - 1) / rpg;
     if (!backward) return groups;  // nothing is carried from row to row: one group of rows per workgroup
     const int64_t cap = 4 * (int64_t)num_cus() * 256 / threads;  // ~16 wavefronts per CU
     return groups < cap ? groups : cap;
@@ -378,13 +390,18 @@ static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
         else if (nv == 2) LA_NG_GO(KERNEL, 2, 256, ng_threads(256), __VA_ARGS__);              \
         else LA_NG_GO(KERNEL, 4, 256, ng_threads(256), __VA_ARGS__);                           \
     } while (0)
-#define LA_NG_DISPATCH_BWD(KERNEL, ...)                               \
+#define LA_NG_BWD(TPR, FEW, ...) hipLaunchKernelGGL((norm_gate_bwd_kernel<T, 1, TPR, FEW>), grid, dim3(ng_bwd_threads(TPR, sizeof(T), FEW)), 0, st, __VA_ARGS__)
+#define LA_NG_DISPATCH_BWD(...)                                       \
     do {                                                              \
-        if (tpr == 64) LA_NG_GO(KERNEL, 1, 64, ng_bwd_threads(64, sizeof(T)), __VA_ARGS__);          \
-        else if (tpr == 128) LA_NG_GO(KERNEL, 1, 128, ng_bwd_threads(128, sizeof(T)), __VA_ARGS__);   \
-        else if (tpr == 256) LA_NG_GO(KERNEL, 1, 256, ng_bwd_threads(256, sizeof(T)), __VA_ARGS__);   \
-        else if (tpr == 512) LA_NG_GO(KERNEL, 1, 512, ng_bwd_threads(512, sizeof(T)), __VA_ARGS__);   \
-        else LA_NG_GO(KERNEL, 1, 1024, ng_bwd_threads(1024, sizeof(T)), __VA_ARGS__);                  \
+        constexpr bool kFew = sizeof(T) == 2;                         \
+        const bool few = ng_few(rows, tpr, sizeof(T));                \
+        if (tpr == 64 && few) LA_NG_BWD(64, kFew, __VA_ARGS__);       \
+        else if (tpr == 128 && few) LA_NG_BWD(128, kFew, __VA_ARGS__); \
+        else if (tpr == 64) LA_NG_BWD(64, false, __VA_ARGS__);        \
+        else if (tpr == 128) LA_NG_BWD(128, false, __VA_ARGS__);      \
+        else if (tpr == 256) LA_NG_BWD(256, false, __VA_ARGS__);      \
+        else if (tpr == 512) LA_NG_BWD(512, false, __VA_ARGS__);      \
+        else LA_NG_BWD(1024, false, __VA_ARGS__);                     \
     } while (0)
 
 template <typename T>
@@ -407,7 +424,7 @@ static int ng_bwd(const void* o, const void* g, const void* w, const void* b, co
     ng_shape(cols / (16 / (int64_t)sizeof(T)), true, &tpr, &nv);
     if (!nv) return LA_E_UNSUPPORTED;
     const dim3 grid((unsigned)ng_grid(rows, tpr, true, sizeof(T)));
-    LA_NG_DISPATCH_BWD(norm_gate_bwd_kernel, static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
+    LA_NG_DISPATCH_BWD(static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
                    static_cast<const T*>(b), mean, rstd, static_cast<const T*>(dy), static_cast<T*>(d_o), static_cast<T*>(d_g),
                    part, rows, (int)cols);
     int rc = (int)hipGetLastError();
@@ -419,6 +436,7 @@ static int ng_bwd(const void* o, const void* g, const void* w, const void* b, co
 }
 #undef LA_NG_DISPATCH_FWD
 #undef LA_NG_DISPATCH_BWD
+#undef LA_NG_BWD
 #undef LA_NG_GO
 
 static int ng_check(int64_t rows, int64_t cols, int dtype) {

@@ -29,3 +29,20 @@ def test_row_counts_around_a_pass(cols, side, dtype):
         want = oracle.norm_gate_fwd_bwd(o, g, w, b, dy, 1e-5, torch.float64)
         for name, a, r in zip(("y", "d_o", "d_g", "d_weight", "d_bias"), got, want):
             assert rel_norm(a.detach().cpu(), r) < lim, (rows, name, rel_norm(a.detach().cpu(), r))
+
+
+@pytest.mark.parametrize("cols,side", [(64, 4), (200, 4), (512, 4), (520, 2), (1024, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_row_counts_around_the_small_workgroups(cols, side, dtype):
+    """16-bit rows of one or two wavefronts: workgroups of 256 threads up to one group of rows per CU (256), of 1024 beyond."""
+    lim = {torch.bfloat16: 5e-3, torch.float16: 1e-3}[dtype]
+    for rows in (1, side - 1, side, side + 1, 255 * side + 1, 256 * side, 256 * side + 1):
+        g_ = torch.Generator().manual_seed(rows + cols)
+        o, g, dy = ((torch.randn(rows, cols, generator=g_) * 2).to(dtype) for _ in range(3))
+        w, b = (torch.randn(cols, generator=g_).to(dtype) for _ in range(2))
+        leaves = [t.cuda().requires_grad_() for t in (o, g, w, b)]
+        y = norm_gate(*leaves, 1e-5)
+        got = (y,) + torch.autograd.grad(y, leaves, dy.cuda())
+        want = oracle.norm_gate_fwd_bwd(o, g, w, b, dy, 1e-5, torch.float64)
+        for name, a, r in zip(("y", "d_o", "d_g", "d_weight", "d_bias"), got, want):
+            assert rel_norm(a.detach().cpu(), r) < lim, (rows, name, rel_norm(a.detach().cpu(), r))
