@@ -26,9 +26,9 @@ def _recorder():
     return out
 
 
-def routes(shapes, lib=LIB, decay=True, once=0):
-    """`once`: that launch option (0: none given)."""
-    ask = json.dumps({"recorder": _recorder(), "lib": lib, "decay": decay, "once": once, "shapes": [list(s) for s in shapes]})
+def routes(shapes, lib=LIB, decay=True, once=0, workspace=True):
+    """`once`: that launch option (0: none given); `workspace`: whether the backward pass gets what it asks for, or none."""
+    ask = json.dumps({"recorder": _recorder(), "lib": lib, "decay": decay, "once": once, "workspace": workspace, "shapes": [list(s) for s in shapes]})
     r = subprocess.run([sys.executable, os.path.abspath(__file__)], input=ask, capture_output=True, text=True, check=True)
     return {tuple(k): v for k, v in json.loads(r.stdout)}
 
@@ -54,6 +54,7 @@ def _main():
         kept = L.la_carry_bytes(*dims, op)
         w0, w1 = (L.la_workspace_bytes_opts(i, *dims, op) for i in (0, 1))
         got = {"kept": kept, "ws": w1}
+        w1 = w1 if ask["workspace"] else 0
         w0 = 0 if kept else w0
         assert L.la_fwd_carry(p[0], p[1], p[2], s, p[3], None, *dims, p[9] if w0 else None, w0, op, p[10] if kept else None, kept, None) == 0
         got["fwd"] = rec.recorded().decode()

@@ -358,8 +358,9 @@ def test_backward_in_one_launch(b, h, n, d, decay):
 @pytest.mark.parametrize("decay", [True, False])
 def test_dq_and_dk_in_one_launch(b, h, n, d, e, decay):
     """With d != e the dQ sweep (walking forward) and the dK sweep (walking backward) have one shape
-    and, with few sequences, share a launch; dV follows.  once=False / True as above; same numbers,
-    bit for bit, on plain and token-major tensors."""
+    and, with few sequences, share a launch; dV follows - up to 128 features in the same launch, as far as
+    once=True goes (test_gpu_bwd_trio.py has the rows where the library's own choice is the shared launch of the
+    two).  once=False / True as above; same numbers, bit for bit, on plain and token-major tensors."""
     g = torch.Generator().manual_seed(n + d + e)
     q, k = ((torch.randn(b, n, h, d, generator=g) * 0.7).bfloat16().to(DEV) for _ in range(2))
     v, do = (torch.randn(b, n, h, e, generator=g).bfloat16().to(DEV) for _ in range(2))

@@ -5,7 +5,9 @@ transposes of those states, and dK + dV from states collected once (dK from thei
   chunks: states summed in the same order, operands rounded to the tensors' dtype in the other role: a few 1e-3 in the
   2-norm, as for la_bwd_saved) and with the formula on a few sequences;
 * carry and workspace start as NaN: every slot that is read was written;
-* too few bytes of carry: exactly la_bwd_opts."""
+* too few bytes of carry: exactly la_bwd_opts;
+* an altered carry shows in dQ after its first chunk and nowhere else, and shared states in the workspace: the launches under
+  test are the ones that ran (which ones a shape takes: tests/test_host_launch_routes.py)."""
 import ctypes
 
 import pytest
@@ -27,7 +29,8 @@ CASES = [
     (1, 16, 8192, 128, 128, torch.bfloat16, True, False),
     (1, 13, 9057, 128, 128, torch.bfloat16, True, False),   # ragged, a short last chunk, units short of a multiple of 8
     (2, 12, 6400, 96, 120, torch.float16, True, False),    # d != e: dQ alone
-    (4, 16, 4096, 128, 128, torch.bfloat16, True, True),   # projection layout; dK + dV: two chunks, four collected
+    (4, 16, 4096, 128, 128, torch.bfloat16, True, True),   # projection layout; dK + dV in single walks
+    (4, 16, 6400, 128, 128, torch.bfloat16, True, True),   # projection layout; dK + dV: two chunks, four collected
     (3, 15, 6113, 72, 72, torch.bfloat16, False, True),    # no decay, d off the tiles
     (1, 16, 16384, 64, 64, torch.bfloat16, True, False),   # 64-column workgroups
     (1, 9, 9001, 48, 40, torch.float16, False, False),
@@ -94,6 +97,101 @@ def test_gradients_from_carried_states(b, h, n, d, e, dtype, decay, token_major)
     for name, a, r in zip(("o", "dq", "dk", "dv"), [o] + got, want):
         assert_close_scaled(a[-1:, sel], r, 2e-2, 2e-2, "carried %s" % name)
         assert rel_norm(a[-1:, sel], r) < 1e-2, (name, rel_norm(a[-1:, sel], r))
+
+
+def _prepared(b, h, n, d, e, dtype, decay, token_major):
+    """Forward pass done; backward(workspace bytes, carry) -> dq, dk, dv; the carry, the workspace and the bytes it may have."""
+    L = _lib.lib()
+    code = CODE[dtype]
+    g = torch.Generator(device="cuda").manual_seed(n)
+
+    def mk(c):
+        t = torch.randn(b, n, h, c, generator=g, device="cuda") if token_major else torch.randn(b, h, n, c, generator=g, device="cuda")
+        return t.to(dtype).transpose(1, 2) if token_major else t.to(dtype)
+
+    q, k, v, do = mk(d), mk(d), mk(e), mk(e)
+    s = _build_slope_tensor(h).float().cuda().contiguous() if decay else None
+    st = torch.cuda.current_stream().cuda_stream
+    nbytes, wb = L.la_carry_bytes(b, h, n, d, e, code, None), L.la_workspace_bytes(1, b, h, n, d, e, code)
+    assert nbytes > 0
+    carry = torch.empty(nbytes // 4, device="cuda")
+    ws = torch.full((max(wb, 16) // 4,), float("nan"), device="cuda")
+    o = torch.empty_like(v)
+    rc = L.la_fwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr() if decay else None, o.data_ptr(), _strides(q, k, v, o), b, h, n, d, e, code, None, 0, None,
+                        carry.data_ptr(), nbytes, st)
+    assert rc == 0, L.la_error_string(rc)
+
+    def backward(ws_bytes, cr):
+        gr = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        rc = L.la_bwd_carry(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr() if decay else None, do.data_ptr(), *(t.data_ptr() for t in gr), _strides(q, k, v, do, *gr),
+                            b, h, n, d, e, code, ws.data_ptr() if ws_bytes else None, ws_bytes, None, cr.data_ptr(), nbytes, st)
+        assert rc == 0, L.la_error_string(rc)
+        return gr
+
+    return backward, carry, ws, wb
+
+
+@pytest.mark.parametrize("b, h, n, d, e, dtype, decay, token_major", CASES)
+def test_the_launches_under_test_run(b, h, n, d, e, dtype, decay, token_major):
+    backward, carry, ws, wb = _prepared(b, h, n, d, e, dtype, decay, token_major)
+    got = backward(wb, carry)
+    shared = d == e and (b, n) in ((1, 8192), (1, 9057), (1, 16384), (4, 6400))
+    assert torch.isfinite(ws).any().item() == (shared or d != e)  # (d != e: dK and dV scan states of their own)
+    other = backward(wb, torch.zeros_like(carry))
+    assert torch.equal(got[1], other[1]) and torch.equal(got[2], other[2])
+    same = (got[0] == other[0]).all(-1).all(0).all(0)  # per token
+    chunk = int((~same).nonzero()[0])
+    assert same[:chunk].all() and chunk % 64 == 0 and 0 < chunk < n and not same[chunk:chunk + 64].any()
+
+
+@pytest.mark.parametrize("b, h, n, d", [(1, 16, 8192, 128), (4, 16, 6400, 128)])
+@pytest.mark.parametrize("given", [0, 4096])
+def test_carried_dq_without_a_backward_workspace(b, h, n, d, given):
+    """No workspace, or one too small for the states of dK + dV: dQ from the carry as ever, dK and dV from warm-up blocks or single walks."""
+    backward, carry, ws, wb = _prepared(b, h, n, d, d, torch.bfloat16, True, False)
+    full, got = backward(wb, carry), None
+    ws.fill_(float("nan"))
+    got = backward(given, carry)
+    assert not torch.isfinite(ws).any()
+    assert torch.equal(got[0], full[0])
+    for a, c in zip(got[1:], full[1:]):
+        assert rel_norm(a, c.float()) < 3e-3
+
+
+def test_carried_states_in_a_captured_step():
+    """The operators under HIP graph capture, carry and workspaces in the graph's own memory: three replays over new inputs, eager work
+    of the same kind and synchronisations between them, each equal to the eager result."""
+    b, h, n, d = 1, 16, 4096, 128
+    assert _lib.lib().la_carry_bytes(b, h, n, d, d, 0, None) > 0
+    s = _build_slope_tensor(h).float().cuda()
+    fresh = lambda: [torch.randn(b, h, n, d, device="cuda", dtype=torch.bfloat16) for _ in range(4)]  # noqa: E731
+    q, k, v, do = fresh()
+    ts = [t.requires_grad_() for t in (q, k, v)]
+
+    def step(ts, do):
+        o = lightning_attn_func(*ts, s)
+        return (o,) + torch.autograd.grad(o, ts, do)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(ts, do)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step(ts, do)
+    for _ in range(3):
+        new = fresh()
+        with torch.no_grad():
+            for t, x in zip(ts + [do], new):
+                t.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = step([t.clone().requires_grad_() for t in new[:3]], new[3])
+        torch.cuda.synchronize()
+        for a, c in zip(out, want):
+            assert torch.equal(a, c)
 
 
 def test_carried_states_through_autograd_twice():

@@ -69,3 +69,16 @@ def test_what_is_kept_is_read():
             assert bool(r["kept"]) == ("carried" in r["bwd"] or "resume" in r["bwd"]), (once, key, r)
             kept += bool(r["kept"])
     assert kept > 500
+
+
+def test_shapes_that_the_gpu_tests_mean_a_launch_by():
+    """What tests/test_gpu_bwd_trio.py and tests/test_gpu_carried_states.py take their shapes to run."""
+    pairs = [(48, 130, 128, 96), (48, 700, 96, 128), (41, 513, 72, 128), (88, 200, 64, 40), (128, 65, 32, 64)]
+    for key, r in routes([p + (BF16,) for p in pairs]).items():
+        assert r["bwd"].startswith("dq+dk warm w0") and "sweep rev warm" in r["bwd"], (key, r)
+    carried = {(16, 8192, 128, 128, 0): 8, (13, 9057, 128, 128, 0): 8, (64, 6400, 128, 128, 0): 2, (16, 16384, 64, 64, 0): 8, (64, 4096, 128, 128, 0): 0,
+               (45, 6113, 72, 72, 0): 0, (24, 6400, 96, 120, 1): 0, (9, 9001, 48, 40, 1): 0}
+    for key, r in routes(carried).items():
+        assert "carried" in r["bwd"] and ("x2 c%d shared" % carried[key] in r["bwd"] if carried[key] else "shared" not in r["bwd"]), (key, r)
+    for key, r in routes([(16, 8192, 128, 128, 0), (64, 6400, 128, 128, 0)], workspace=False).items():
+        assert "carried" in r["bwd"] and "sweep rev warm" in r["bwd"], (key, r)
