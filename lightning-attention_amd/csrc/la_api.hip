@@ -88,7 +88,6 @@ static int check_opts(const Opts& o) {
     if (o.wide != LA_OPT_AUTO && o.wide != LA_OPT_OFF && o.wide != LA_OPT_ON && o.wide != LA_OPT_ALL) return LA_E_SHAPE;
     return LA_OK;
 }
-static const Opts kAuto = {0, LA_OPT_AUTO, LA_OPT_AUTO, LA_OPT_AUTO, LA_OPT_AUTO};
 
 // pointer and strides of one tensor with `cols` features per row
 static int check_tensor(const Tensor& t, int64_t b, int64_t h, int64_t n, int64_t cols, int dtype) {
@@ -231,7 +230,7 @@ extern "C" int la_supported(int64_t d, int64_t e, int dtype) {
 
 extern "C" size_t la_workspace_bytes_opts(int which, int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype,
                                           const la_launch_opts* opts) {
-    const la::Opts& o = opts ? *opts : la::kAuto;
+    const la::Opts o = la::planning(opts);
     // nothing for empty tensors and for shapes the entry points reject
     if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
     using la::sweep_workspace_bytes;
@@ -254,7 +253,7 @@ static int fwd_saved(const void* q, const void* k, const void* v, const float* s
                      int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace, size_t ws_bytes,
                      const la_launch_opts* opts, const Saved& sv, void* stream) {
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
-    const la::Opts& op = opts ? *opts : la::kAuto;
+    const la::Opts op = la::planning(opts);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
     using la::strided;
@@ -289,7 +288,7 @@ extern "C" int la_fwd_silu(const void* q, const void* k, const void* v, const fl
     if (la_supported(d, e, dtype) && !la_fwd_silu_supported(d, e, dtype)) return LA_E_UNSUPPORTED;
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
     const la::Saved none = {nullptr, 0, false};
-    const la::Opts& op = opts ? *opts : la::kAuto;
+    const la::Opts op = la::planning(opts);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
     using la::strided;
@@ -307,21 +306,21 @@ extern "C" int la_fwd_opts(const void* q, const void* k, const void* v, const fl
 
 extern "C" size_t la_saved_state_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype,
                                        const la_launch_opts* opts) {
-    const la::Opts& o = opts ? *opts : la::kAuto;
+    const la::Opts o = la::planning(opts);
     if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
     return la::plan_saved(b * h, n, d, e, dtype, o).bytes;
 }
 
 extern "C" int64_t la_saved_state_interval(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype,
                                            const la_launch_opts* opts) {
-    const la::Opts& o = opts ? *opts : la::kAuto;
+    const la::Opts o = la::planning(opts);
     if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
     const la::SavedPlan pl = la::plan_saved(b * h, n, d, e, dtype, o);
     return pl.nchunk > 1 ? (int64_t)pl.chunk_len * 64 : 0;
 }
 
 extern "C" size_t la_carry_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, const la_launch_opts* opts) {
-    const la::Opts& o = opts ? *opts : la::kAuto;
+    const la::Opts o = la::planning(opts);
     if (b <= 0 || n <= 0 || la::check_dims(b, h, n, d, e, dtype) != LA_OK || la::check_opts(o) != LA_OK) return 0;
     const la::SavedPlan pl = la::plan_saved(b * h, n, d, e, dtype, o);
     if (pl.nchunk > 1) return la::reads_kept(b * h, n, d, e, pl, o) ? pl.bytes : 0;
@@ -333,7 +332,7 @@ static int bwd_from(const void* q, const void* k, const void* v, const float* s,
                     const int64_t* strides, int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, void* workspace,
                     size_t ws_bytes, const la_launch_opts* opts, const Saved& sv, void* stream) {
     const la::Scratch ws = {workspace, workspace ? ws_bytes : 0};
-    const la::Opts& op = opts ? *opts : la::kAuto;
+    const la::Opts op = la::planning(opts);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     using la::dense;
     using la::strided;

@@ -26,8 +26,7 @@ int prepare_plans() { return num_cus() > 0 ? 0 : (int)hipErrorInvalidDevice; }
 // rebuild their incoming state themselves.  A warm-up block costs about half a full block, so
 // chunk lengths shrink geometrically (len_c ~ (1 - rho)^c, rho = 0.5) to make all workgroups
 // finish together.  The caller's launch options can override the count.
-static int64_t warm_up_chunks(int64_t wgs, int64_t nblk, int64_t min_blocks = 4) {
-    const int64_t cus = num_cus();
+static int64_t warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int64_t min_blocks = 4) {
     int64_t c = 1;
     if (wgs * 2 <= cus && nblk >= 2 * min_blocks) {
         c = cus / wgs;
@@ -36,8 +35,8 @@ static int64_t warm_up_chunks(int64_t wgs, int64_t nblk, int64_t min_blocks = 4)
     return c > 8 ? 8 : c < 1 ? 1 : c;
 }
 
-void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start /* [9] */, double rho, int64_t min_blocks) {
-    int64_t c = forced > 0 ? forced : warm_up_chunks(wgs, nblk, min_blocks);
+void plan_warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start /* [9] */, double rho, int64_t min_blocks) {
+    int64_t c = forced > 0 ? forced : warm_up_chunks(cus, wgs, nblk, min_blocks);
     if (c > 8) c = 8;
     if (c > nblk) c = nblk;
     if (c < 1) c = 1;
@@ -60,7 +59,7 @@ void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int
 }
 
 static void choose_chunks(SweepArgs& a, int nprod, const Opts& opts) {
-    plan_warm_up_chunks((int64_t)((a.bh + 7) / 8 * 8) * a.nslice * nprod, (a.n + 63) / 64, opts.chunks, &a.nchunk, a.chunk_start);
+    plan_warm_up_chunks(opts.cus, (int64_t)((a.bh + 7) / 8 * 8) * a.nslice * nprod, (a.n + 63) / 64, opts.chunks, &a.nchunk, a.chunk_start);
 }
 
 static SweepArgs make_args(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv) {
@@ -100,21 +99,21 @@ static double block_us(int64_t dk, int width) {
 // Column slices per sequence: 64 columns each, or 128, or one slice.
 static int64_t wide_slices(int64_t dv) { return (dv + 127) / 128; }
 static int64_t slices(int64_t dk, int64_t dv, int width) { return width == 2 ? 1 : width ? wide_slices(dv) : (dv + 63) / 64; }
-static double warm_up_frac(int64_t wgs, int64_t nblk) {
+static double warm_up_frac(int64_t wgs, int64_t nblk, const Opts& opts) {
     static const double frac[9] = {1.0, 1.0, 0.77, 0.71, 0.68, 0.67, 0.66, 0.66, 0.66};
-    return frac[warm_up_chunks(wgs, nblk)];
+    return frac[warm_up_chunks(opts.cus, wgs, nblk)];
 }
-static double warm_up_us(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int wide) {
+static double warm_up_us(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int wide, const Opts& opts) {
     const int64_t nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, wide) * nprod;
-    return warm_up_frac(wgs, nblk) * (double)nblk * block_us(dk, wide);
+    return warm_up_frac(wgs, nblk, opts) * (double)nblk * block_us(dk, wide);
 }
 
 static ScanPlan plan_scan(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int wide, const Opts& opts) {
-    const ScanPlan none = {1, 0, 0, warm_up_us(bh, n, dk, dv, nprod, wide)};
+    const ScanPlan none = {1, 0, 0, warm_up_us(bh, n, dk, dv, nprod, wide, opts)};
     ScanPlan pl = none;
     if (opts.scan == LA_OPT_OFF) return none;
     const int forced = opts.chunks;
-    const int64_t nblk = (n + 63) / 64, cus = num_cus();
+    const int64_t nblk = (n + 63) / 64, cus = opts.cus;
     const int64_t nslice = slices(dk, dv, wide);
     const int64_t wgs = (bh + 7) / 8 * 8 * nslice * nprod;
     int64_t c = 1;
@@ -138,10 +137,10 @@ static ScanPlan plan_scan(int64_t bh, int64_t n, int64_t dk, int64_t dv, int npr
 // Estimated duration (us) of one launch of nprod sweeps in workgroups of width code `width`, by the figures
 // above: rounds of workgroups where they fill the chip, else the better of the two chunk plans.
 static double width_us(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod, int width, size_t scratch, const Opts& opts) {
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, width) * nprod;
+    const int64_t cus = opts.cus, nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, width) * nprod;
     if (wgs * 2 > cus) return (double)((wgs + cus - 1) / cus) * (double)nblk * block_us(dk, width);
     const ScanPlan pl = plan_scan(bh, n, dk, dv, nprod, width, opts);
-    return pl.nchunk > 1 && pl.bytes <= scratch ? pl.us : warm_up_us(bh, n, dk, dv, nprod, width);
+    return pl.nchunk > 1 && pl.bytes <= scratch ? pl.us : warm_up_us(bh, n, dk, dv, nprod, width, opts);
 }
 
 // The pipelined kernel can give each workgroup 128 columns of z / out instead of 64: the score tile
@@ -163,14 +162,14 @@ static bool wide_columns(int64_t bh, int64_t n, int64_t dk, int64_t dv, int npro
         const int64_t ws = wide_slices(dv), ns = (dv + 63) / 64;
         if (ws >= ns) return false;
         if (opts.wide != LA_OPT_AUTO) return opts.wide == LA_OPT_ON;
-        const int64_t cus = num_cus(), units = (bh + 7) / 8 * 8 * nprod, wide = units * ws, narrow = units * ns;
+        const int64_t cus = opts.cus, units = (bh + 7) / 8 * 8 * nprod, wide = units * ws, narrow = units * ns;
         if (narrow <= cus) return width_us(bh, n, dk, dv, nprod, 1, scratch, opts) < 0.9 * width_us(bh, n, dk, dv, nprod, 0, scratch, opts);
         return (wide + cus - 1) / cus * 7 < (narrow + cus - 1) / cus * 5;
     }
     if (dv <= 64 || dv > 128) return false;
     if (opts.wide != LA_OPT_AUTO) return opts.wide == LA_OPT_ON;
     if (dk <= 64) return false;  // the 128-column form pads the feature dim to 128
-    const int64_t cus = num_cus(), wide = (bh + 7) / 8 * 8 * nprod, narrow = 2 * wide;
+    const int64_t cus = opts.cus, wide = (bh + 7) / 8 * 8 * nprod, narrow = 2 * wide;
     if (narrow <= cus) {
         // Every 64-column workgroup gets a CU of its own.  With so few of them that a long walk is cut
         // into chunks from scanned states, rather half as many workgroups of 128 columns and twice the chunks
@@ -179,7 +178,7 @@ static bool wide_columns(int64_t bh, int64_t n, int64_t dk, int64_t dv, int npro
         // empty - d = e = 96, b*h = 96: la_fwd 0.321 against 0.359 ms at n = 16384, la_bwd 0.78 against 0.82)
         if (narrow * 2 > cus) return dv <= 96;
         const ScanPlan w = plan_scan(bh, n, dk, dv, nprod, true, opts), nw = plan_scan(bh, n, dk, dv, nprod, false, opts);
-        return w.nchunk > 1 && w.bytes <= scratch && w.us < (nw.bytes <= scratch ? nw.us : warm_up_us(bh, n, dk, dv, nprod, false));
+        return w.nchunk > 1 && w.bytes <= scratch && w.us < (nw.bytes <= scratch ? nw.us : warm_up_us(bh, n, dk, dv, nprod, false, opts));
     }
     return (wide + cus - 1) / cus * 5 < (narrow + cus - 1) / cus * 4;
 }
@@ -245,7 +244,7 @@ struct SharedPlan {
 // `us` is what sweep_bwd_once weighs its own launch by, so without a shared plan it is by block_us as there.
 static SharedPlan plan_shared(int64_t bh, int64_t n, int64_t d, size_t scratch, const Opts& opts) {
     const int own_width = column_width(bh, n, d, d, 2, scratch, opts), width = square_width(d, d);
-    const int64_t nblk = (n + 63) / 64, cus = num_cus(), units8 = (bh + 7) / 8 * 8;
+    const int64_t nblk = (n + 63) / 64, cus = opts.cus, units8 = (bh + 7) / 8 * 8;
     const SharedPlan none = {1, 0, 0, 1, 0, width_us(bh, n, d, d, 2, own_width, scratch, opts)};
     const bool crowded = own_width == 0 && d > 64 && d <= 128 && units8 * slices(d, d, 0) * 4 > cus;
     if (width < 0 || !own_choices(opts)) return none;
@@ -342,7 +341,7 @@ SavedPlan plan_saved(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, con
     const bool big = d > 128 && d <= 192 && e > 128 && e <= 192;
     if (!big && (d <= 64 || d > 128 || e > 128)) return none;
     if (opts.chunks != 0 || opts.wide == LA_OPT_ON || opts.wide == LA_OPT_ALL || opts.scan == LA_OPT_ON) return none;
-    const int64_t nblk = (n + 63) / 64, cus = num_cus(), units8 = (bh + 7) / 8 * 8;
+    const int64_t nblk = (n + 63) / 64, cus = opts.cus, units8 = (bh + 7) / 8 * 8;
     // Short sequences: writing the states and starting from them costs what the wider workgroups save
     // (b4 h32 d128 fwd+bwd, with / without: n = 512 0.060 / 0.056 ms, 1024 0.097 / 0.096, 2048 0.176 / 0.181, 4096
     // 0.341 / 0.357; d = 192: n = 1024 0.160 / 0.158, 2048 0.319 / 0.332).
@@ -351,7 +350,7 @@ SavedPlan plan_saved(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, con
     // the forward pass as planned: that width, one walk per sequence
     if (column_width(bh, n, d, e, 1, (size_t)-1, opts) != fwd_width) return none;
     if (plan_scan(bh, n, d, e, 1, fwd_width, opts).nchunk > 1) return none;
-    if (warm_up_chunks(units8 * slices(d, e, fwd_width), nblk) > 1) return none;
+    if (warm_up_chunks(opts.cus, units8 * slices(d, e, fwd_width), nblk) > 1) return none;
     // dQ: one workgroup of that width per sequence and chunk
     int64_t c = cus / units8;
     if (c > nblk / 4) c = nblk / 4;
@@ -366,7 +365,7 @@ SavedPlan plan_saved(int64_t bh, int64_t n, int64_t d, int64_t e, int dtype, con
     const ScanPlan own = plan_scan(bh, n, e, d, 1, wide, opts);
     const int64_t own_wgs = units8 * slices(e, d, wide);
     const double own_us = own.nchunk > 1 ? own.us
-                          : own_wgs * 2 <= cus ? warm_up_us(bh, n, e, d, 1, wide)
+                          : own_wgs * 2 <= cus ? warm_up_us(bh, n, e, d, 1, wide, opts)
                                                : (double)((own_wgs + cus - 1) / cus) * (double)nblk * block_us(e, wide);
     if ((double)pl.chunk_len * block_us(e, dq_width) >= own_us) return none;
     pl.bytes = (size_t)bh * (size_t)(pl.nchunk - 1) * (size_t)(d * e) * sizeof(float);
@@ -518,7 +517,7 @@ static size_t usable_bytes(const void* ws, size_t ws_bytes) { return ws && (rein
 // sweeps fill the chip anyway).  dq_us > 0: what the dQ sweep alone would take from states the forward pass left.
 static bool once_chosen(int64_t bh, int64_t n, int64_t d, size_t scratch, const Opts& opts, double dq_us) {
     if (const int forced = once_forced(opts)) return forced > 0;
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, nslice = (d + 63) / 64;
+    const int64_t cus = opts.cus, nblk = (n + 63) / 64, nslice = (d + 63) / 64;
     const int64_t wgs = (bh + 7) / 8 * 8 * nslice * 3;  // one chunk each
     // (up to two rounds of workgroups: on a short walk one launch of twice as many 64-column workgroups as
     // there are CUs still beats two launches - b1 h48 n2048 d192: la_bwd 0.138 against 0.162 ms)
@@ -534,7 +533,7 @@ static bool once_chosen(int64_t bh, int64_t n, int64_t d, size_t scratch, const 
     // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
     // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
     const double rounds = wgs > cus ? 2.0 : 1.0, launch = wgs > cus ? 1.5 : 0.0;
-    return rounds * warm_up_frac(wgs, nblk) * (double)nblk * block_us(d, false) < separate + launch;
+    return rounds * warm_up_frac(wgs, nblk, opts) * (double)nblk * block_us(d, false) < separate + launch;
 }
 int sweep_bwd_once(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                    int64_t d, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
@@ -577,10 +576,10 @@ struct DqDkPlan {
     double us;
 };
 static DqDkPlan plan_dq_dk(int64_t bh, int64_t n, int64_t dk, int64_t dv, size_t scratch, const Opts& opts, double dq_us) {
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, 0) * 2;
+    const int64_t cus = opts.cus, nblk = (n + 63) / 64, wgs = (bh + 7) / 8 * 8 * slices(dk, dv, 0) * 2;
     const int64_t rounds = (wgs + cus - 1) / cus;
     const double own = width_us(bh, n, dk, dv, 1, column_width(bh, n, dk, dv, 1, scratch, opts), scratch, opts);
-    const double two = (rounds > 1 ? (double)rounds : warm_up_frac(wgs, nblk)) * (double)nblk * block_us(dk, 0);
+    const double two = (rounds > 1 ? (double)rounds : warm_up_frac(wgs, nblk, opts)) * (double)nblk * block_us(dk, 0);
     const double apart = (dq_us > 0.0 ? dq_us : own) + own;
     const bool together = rounds <= 3 && two < 2.0 * own && !(dq_us > 0.0 && apart < 0.8 * two);
     return {together, together ? two : apart};
@@ -593,7 +592,7 @@ static int64_t trio_wgs(int64_t bh, int64_t d, int64_t e) { return (bh + 7) / 8 
 static bool trio_chosen(int64_t bh, int64_t n, int64_t d, int64_t e, size_t scratch, const Opts& opts, double dq_us) {
     if (d > 128 || e > 128) return false;
     if (const int forced = once_forced(opts)) return forced > 0;
-    const int64_t cus = num_cus(), nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8, wgs = trio_wgs(bh, d, e);
+    const int64_t cus = opts.cus, nblk = (n + 63) / 64, units8 = (bh + 7) / 8 * 8, wgs = trio_wgs(bh, d, e);
     if (wgs > cus) return false;
     const int v_width = column_width(bh, n, d, e, 1, scratch, opts);
     const DqDkPlan q = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us);
@@ -606,7 +605,7 @@ static bool trio_chosen(int64_t bh, int64_t n, int64_t d, int64_t e, size_t scra
         const ScanPlan v = plan_scan(bh, n, d, e, 1, v_width, opts);
         separate -= 0.11 * q.us + (v.nchunk > 1 && v.bytes <= scratch ? (units8 == 8 ? 10.0 : 5.0) : 0.0);
     }
-    return warm_up_frac(wgs, nblk) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) < separate;
+    return warm_up_frac(wgs, nblk, opts) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) < separate;
 }
 int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, const float* s, int64_t bh, int64_t h, int64_t n,
                       int64_t d, int64_t e, int dtype, void* ws, size_t ws_bytes, const Opts& opts, double dq_us, hipStream_t st) {
@@ -620,7 +619,7 @@ int sweep_bwd_once_de(const SweepIO& dq, const SweepIO& dk, const SweepIO& dv, c
         SweepPair& p = *ps[i];
         p.nprod = 1;
         p.a[0] = i < 2 ? make_args(*ios[i], s, bh, h, n, e, d) : make_args(*ios[i], s, bh, h, n, d, e);
-        plan_warm_up_chunks(wgs, nblk, opts.chunks, &p.a[0].nchunk, p.a[0].chunk_start);
+        plan_warm_up_chunks(opts.cus, wgs, nblk, opts.chunks, &p.a[0].nchunk, p.a[0].chunk_start);
         p.a[1] = p.a[0];
         p.wide = 0;
         p.mode = kWarmUp;

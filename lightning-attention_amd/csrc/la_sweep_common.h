@@ -5,8 +5,17 @@
 
 namespace la {
 
-// How the caller wants a call mapped onto launches (all zero: the library's own choices).
-typedef la_launch_opts Opts;
+// How the caller wants a call mapped onto launches (all zero: the library's own choices), and the compute units it is planned
+// for, asked once per call: a plan looks at them some forty times, and asking which device is current costs 0.1 us.
+struct Opts : la_launch_opts {
+    int64_t cus;
+};
+inline Opts planning(const la_launch_opts* given) {
+    Opts o;
+    static_cast<la_launch_opts&>(o) = given ? *given : la_launch_opts{0, LA_OPT_AUTO, LA_OPT_AUTO, LA_OPT_AUTO, LA_OPT_AUTO};
+    o.cus = num_cus();
+    return o;
+}
 
 // Where the (batch, head, token) rows of a tensor start, in elements; the feature dim is contiguous.
 // A plain (b, h, n, d) tensor has {h*n*d, n*d, d}; a (b, n, h, d) projection output viewed as
@@ -159,10 +168,10 @@ struct SweepTrio {
 int sweep_pipe_trio(const SweepTrio& t, int dtype, hipStream_t st);
 
 // Count (up to 8) and first blocks, chunk_start[0 .. 8], of the warm-up chunks for a launch that would have
-// `wgs` workgroups with one chunk each, on a walk of nblk blocks; `forced` > 0 overrides the count.
+// `wgs` workgroups with one chunk each, on a walk of nblk blocks and `cus` compute units; `forced` > 0 overrides the count.
 // `rho`: what a warm-up block costs of a full one; `min_blocks`: fewest blocks per chunk (on average).
 // Defined in la_sweep.hip.
-void plan_warm_up_chunks(int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start, double rho = 0.5, int64_t min_blocks = 4);
+void plan_warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start, double rho = 0.5, int64_t min_blocks = 4);
 
 // Raises a kernel's dynamic LDS limit above the 64 KB default, once per kernel and device (the call is
 // not free and the limit stays).  `done` is the instantiation's own flag array, one entry per device.

@@ -453,7 +453,7 @@ int sweep_f32(const void* x, const void* y, const void* z, void* out, const floa
               int64_t n, int64_t dk, int64_t dv, bool reverse, int chunks, hipStream_t st) {
     if (dk > 128) return LA_E_UNSUPPORTED;
     SweepArgsF32 a = make_args_f32(x, y, z, out, s, bh, h, n, dk, dv);
-    plan_warm_up_chunks((bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
+    plan_warm_up_chunks(num_cus(), (bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
     return reverse ? launch_dir_f32<true>(a, st) : launch_dir_f32<false>(a, st);
 }
 
@@ -466,7 +466,7 @@ int sweep_f32_bwd_once(const void* q, const void* k, const void* v, const void* 
     t.a[0] = make_args_f32(dout, v, k, dq, s, bh, h, n, d, d);
     t.a[1] = make_args_f32(v, dout, q, dk, s, bh, h, n, d, d);
     t.a[2] = make_args_f32(k, q, dout, dv, s, bh, h, n, d, d);
-    plan_warm_up_chunks((bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, chunks, &t.a[0].nchunk, t.a[0].chunk_start, kWarmCost, kMinBlocks);
+    plan_warm_up_chunks(num_cus(), (bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, chunks, &t.a[0].nchunk, t.a[0].chunk_start, kWarmCost, kMinBlocks);
     for (int i = 1; i < 3; ++i) {
         t.a[i].nchunk = t.a[0].nchunk;
         for (int j = 0; j < 9; ++j) t.a[i].chunk_start[j] = t.a[0].chunk_start[j];
