@@ -457,7 +457,6 @@ int sweep_carrying(const SweepIO& io, const float* s, int64_t bh, int64_t h, int
 int sweep_carried(const SweepIO& io, const float* s, int64_t bh, int64_t h, int64_t n, int64_t dk, int64_t dv, int dtype,
                   const float* carry, const SavedPlan& pl, hipStream_t st) {
     SweepPair p = chunked(io, s, bh, h, n, dk, dv, pl.dq_width, pl.nchunk, pl.chunk_len, const_cast<float*>(carry));
-    p.shared = 1;
     p.nslot = pl.nchunk - 1;
     p.transposed = 1;
     return sweep_pipe_apply(p, dtype, false, st);
@@ -489,7 +488,6 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
         p = chunked(io0, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws));
         p.a[1] = chunked(io1, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws)).a[0];
         p.nprod = 2;
-        p.shared = 1;
         p.nslot = sh.ncollect - 1;
         p.slot_mul = sh.mul;
         p.transposed = 2;

@@ -121,7 +121,8 @@ struct SweepPair {
     //             into the state at the start of each chunk.
     //   kResume   a single launch: it starts from `state`, which an earlier sweep over the same y and z in
     //             swapped roles has left behind (`save` below).
-    // In the three latter modes the chunks are chunk_len blocks long (a[0].chunk_start is not used).  kCollect /
+    //   kShared   like kApply, from slots with a layout of their own (`nslot` below).
+    // In the four latter modes the chunks are chunk_len blocks long (a[0].chunk_start is not used).  kCollect /
     // kApply: `state` holds, per (unit, sweep, slice), nchunk - 1 slots of the state waves' accumulators.
     // kResume: per unit nchunk - 1 plain row-major matrices of dv x dk floats, matrix c - 1 being the
     // transpose of the state chunk c starts from (pipelined kernel, 128-column workgroups, one sweep).
@@ -138,11 +139,11 @@ struct SweepPair {
     // x, y and z are pre-activations: the kernel applies SiLU to them as it loads them (forward sweeps of
     // the pipelined kernel at feature dims up to 128)
     int silu = 0;
-    // kApply from states that another launch over the same tensors collected: `shared` says that there is one set of
-    // slots per unit and slice for all sweeps of the launch, nslot slots to a set, chunk c starting from slot
-    // c * slot_mul - 1; bit i of `transposed`: sweep i has y and z in swapped roles, its state is the transpose of
-    // the collected one (square tiles of state only: feature dim as padded == columns of a workgroup).
-    int shared = 0, nslot = 0, slot_mul = 1, transposed = 0;
+    // kShared: as kApply, from states that another launch over the same tensors collected.  One set of nslot slots per unit and
+    // slice for all sweeps of the launch, chunk c starting from slot c * slot_mul - 1; bit i of `transposed`: sweep i has y and
+    // z in swapped roles, its state is the transpose of the collected one (square tiles of state only: feature dim as
+    // padded == columns of a workgroup).  nslot == 0 elsewhere.
+    int nslot = 0, slot_mul = 1, transposed = 0;
 };
 
 // One launch can also carry sweeps of both directions: the whole backward pass when d == e, dQ walking
@@ -199,9 +200,9 @@ struct SavedPlan {
 
 // Launches the single-barrier pipelined kernel (feature dim up to 256); defined in la_sweep_pipe.hip.
 // n, dk, dv, h, bh, nslice and the chunking must agree between the two sweeps of a pair.
-enum { kWarmUp = 0, kCollect = 1, kApply = 2, kResume = 3 };
+enum { kWarmUp = 0, kCollect = 1, kApply = 2, kResume = 3, kShared = 4 };
 int sweep_pipe(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
-// The middle and the last of the three launches behind kCollect, for a launch whose states are shared.
+// The first two and the last of the three launches behind kCollect, for a launch whose states are shared.
 int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 int sweep_pipe_apply(const SweepPair& p, int dtype, bool reverse, hipStream_t st);
 // One-time work per device, done ahead of the first launches: the dynamic LDS limits of every instantiation

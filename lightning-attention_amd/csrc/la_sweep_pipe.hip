@@ -24,14 +24,6 @@ static int launch_dir(const SweepPair& pair, hipStream_t st) {
         }
         return LA_E_UNSUPPORTED;
     }
-    if (pair.shared) {
-#define LA_GT2(DKP, NH, DENSE) (decay ? launch_one<T, DKP, 1, NH, REVERSE, true, DENSE, false, true>(pair, st) : launch_one<T, DKP, 1, NH, REVERSE, false, DENSE, false, true>(pair, st))
-#define LA_GT(DKP, NH) (dense ? LA_GT2(DKP, NH, true) : LA_GT2(DKP, NH, false))
-        if (pair.wide) return LA_GT(128, 2);
-        return a.dk <= 64 ? LA_GT(64, 1) : LA_E_UNSUPPORTED;
-#undef LA_GT
-#undef LA_GT2
-    }
     if (pair.wide) return LA_GO(128, 2);  // 128 columns per workgroup (nslice counts those)
     if (a.dk <= 64) return LA_GO(64, 1);
     return LA_GO(128, 1);
@@ -146,7 +138,7 @@ int sweep_pipe(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
 }
 
 int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
-    if (!p.state || p.chunk_len < 1 || p.a[0].nchunk < 2 || p.shared) return LA_E_WORKSPACE;
+    if (!p.state || p.chunk_len < 1 || p.a[0].nchunk < 2 || p.nslot) return LA_E_WORKSPACE;
     SweepPair q = p;
     q.mode = kCollect;
     const int rc = launch_any(q, dtype, reverse, st);
@@ -156,7 +148,7 @@ int sweep_pipe_collect(const SweepPair& p, int dtype, bool reverse, hipStream_t 
 int sweep_pipe_apply(const SweepPair& p, int dtype, bool reverse, hipStream_t st) {
     if (!p.state || p.chunk_len < 1 || p.a[0].nchunk < 2) return LA_E_WORKSPACE;
     SweepPair q = p;
-    q.mode = kApply;
+    q.mode = p.nslot ? kShared : kApply;
     return launch_any(q, dtype, reverse, st);
 }
 

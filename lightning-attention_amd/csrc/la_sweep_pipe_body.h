@@ -70,10 +70,12 @@ struct PipeLds {
 // `bid`: number of the workgroup within its part of the launch.
 // SILU: x, y and z pass through SiLU on their way from memory into LDS (the attention block's activation on
 // q, k, v, examples/module/tnl_attn.py:51-54, fused into the forward pass).
-// SHARED: a kApply launch from shared or transposed slots (SweepPair::shared); an instantiation of its own, because the slot
-// arithmetic and the transposed load cost every other launch of the form 1 - 2 % (la_bwd of b1 h88 n8192 d64 e40 205.2 us
-// with them, 202.2 without; la_fwd of b1 h8 n113 d64 6.68 / 6.53).
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
+// SHARES: the launch may be a kShared one.  Only the kernel of one sweep or pair ever is: in the kernels that hold several
+// bodies its code costs 1.5 % (la_bwd of b1 h88 n8192 d64 e40 205.2 us with it, 202.2 without).  As instantiations of their own
+// kShared launches would find their code cold, 0.5 - 1 us each: 2.6 % on fwd + bwd of b1 h8 n22291 d64 (99.1 -> 101.7 us).  Its
+// fields are read where such a launch needs them: ahead of the walk they are 0.15 us of every launch (b1 h8 n113 d64
+// 6.45 -> 6.60 us).
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARES = false>
 __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const unsigned bid) {
     typedef Mma<T> M;
     typedef typename M::V8 V8;
@@ -257,9 +259,8 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const int64_t it_end = cend;
     // the state slot of this workgroup's chunk: [unit][sweep][slice][chunk 0 .. nchunk-2][state waves' accumulators]
     constexpr size_t SF = (size_t)4 * NH * KT * 64 * 4;
-    static_assert(!SHARED || (NF == 1 && 4 * NH == KT && !SILU), "only a square tile of state can be another sweep's transposed one");
-    const size_t slot_set = SHARED ? (size_t)unit * nslice + slice : ((size_t)unit * nprod + sub % nprod) * nslice + slice;
-    float* const slot0 = pair.state + slot_set * (size_t)(SHARED ? pair.nslot : nchunk - 1) * SF;
+    static_assert(!SHARES || (NF == 1 && 4 * NH == KT && !SILU), "only a square tile of state can be another sweep's transposed one");
+    float* const slot0 = pair.state + ((((size_t)unit * nprod + sub % nprod) * nslice + slice) * (size_t)(nchunk - 1)) * SF;
 
     u32x4 xrA[XC], yrA[XC], zrA[ZC], xrB[XC], yrB[XC], zrB[ZC];
 
@@ -848,21 +849,25 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     auto init_state = [&]() __attribute__((always_inline)) {
         // this lane's part of a state slot: [wave][slab][tile][lane] accumulator quartets
         const size_t lane_slot = ((size_t)w * NH * KT * 64 + lane) * 4;
-        const bool resume = mode == kApply && chunk > 0;
-        const float* const slot = slot0 + (size_t)(SHARED ? chunk * pair.slot_mul - 1 : chunk - 1) * SF;
-        const float* const src = slot + lane_slot;
-        if constexpr (SHARED) {
-            if (resume && ((pair.transposed >> (sub % nprod)) & 1)) {
-                // state[k][c] = slot[c][k]: tile (kt; NH w + h) is the transpose of the slot's tile (NH w + h; kt)
+        bool resume = mode == kApply && chunk > 0;
+        const float* src = slot0 + (size_t)(chunk - 1) * SF + lane_slot;
+        if constexpr (SHARES) {
+            if (mode == kShared && chunk > 0) {
+                const float* const slot = pair.state + (((size_t)unit * nslice + slice) * (size_t)pair.nslot + (size_t)(chunk * pair.slot_mul - 1)) * SF;
+                if ((pair.transposed >> (sub % nprod)) & 1) {
+                    // state[k][c] = slot[c][k]: tile (kt; NH w + h) is the transpose of the slot's tile (NH w + h; kt)
 #pragma unroll
-                for (int h = 0; h < NH; ++h)
+                    for (int h = 0; h < NH; ++h)
 #pragma unroll
-                    for (int kt = 0; kt < KT; ++kt) {
-                        const float* const m = slot + (size_t)(kt * KT + NH * w + h) * 256 + ((r >> 2) * 16 + 4 * g) * 4 + (r & 3);
+                        for (int kt = 0; kt < KT; ++kt) {
+                            const float* const m = slot + (size_t)(kt * KT + NH * w + h) * 256 + ((r >> 2) * 16 + 4 * g) * 4 + (r & 3);
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) st[h][kt][v] = m[4 * v];
-                    }
-                return;
+                            for (int v = 0; v < 4; ++v) st[h][kt][v] = m[4 * v];
+                        }
+                    return;
+                }
+                resume = true;
+                src = slot + lane_slot;
             }
         }
 #pragma unroll
@@ -912,9 +917,13 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     }
 }
 
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
+// the forms whose tile of state is square
+template <int DKP, int NF, int NH>
+constexpr bool kSquare = NF == 1 && 4 * NH == DKP / 16;
+
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
 __global__ __launch_bounds__(512, 1) void la_sweep_pipe_kernel(SweepPair pair) {
-    sweep_pipe_body<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>(pair, blockIdx.x);
+    sweep_pipe_body<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, kSquare<DKP, NF, NH> && !SILU>(pair, blockIdx.x);
 }
 
 // Forward-walking and backward-walking sweeps in one launch (SweepBoth).
@@ -925,36 +934,38 @@ __global__ __launch_bounds__(512, 1) void la_sweep_pipe_both_kernel(SweepBoth bo
 }
 
 // What a kernel instantiation needs once per device before its first launch (its dynamic LDS limit raised).
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
 static int prep_one() {
     constexpr size_t lds = PipeLds<DKP, NF, NH>::bytes(sizeof(T));
     static_assert(lds <= 160 * 1024, "LDS budget");
     static unsigned char lds_allowed[kMaxDevices];
-    return allow_lds(la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>, lds, lds_allowed);
+    return allow_lds(la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>, lds, lds_allowed);
 }
 
-template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false, bool SHARED = false>
+template <typename T, int DKP, int NF, int NH, bool REVERSE, bool DECAY, bool DENSE, bool SILU = false>
 static int launch_one(const SweepPair& pair, hipStream_t st) {
     const SweepArgs& a = pair.a[0];
     constexpr size_t lds = PipeLds<DKP, NF, NH>::bytes(sizeof(T));
-    auto kern = la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>;
-    if (const int e = prep_one<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU, SHARED>()) return e;
-    if (SILU != (pair.silu != 0) || SHARED != (pair.shared != 0)) return LA_E_UNSUPPORTED;
+    auto kern = la_sweep_pipe_kernel<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>;
+    if (const int e = prep_one<T, DKP, NF, NH, REVERSE, DECAY, DENSE, SILU>()) return e;
+    if (SILU != (pair.silu != 0)) return LA_E_UNSUPPORTED;
     const int units8 = (a.bh + 7) / 8 * 8;
     // the slice width the host chose must be one this instantiation's LDS slot and state waves hold
     if (a.zw <= 0 || a.zw > 64 * NH || a.zw % (16 * NH)) return LA_E_UNSUPPORTED;
     // the state slots the host sized must be the ones this instantiation reads and writes
-    if ((pair.mode == kCollect || pair.mode == kApply) && pipe_state_floats(a.dk, pair.wide) != (size_t)4 * NH * (DKP / 16) * 64 * 4)
+    if ((pair.mode == kCollect || pair.mode == kApply || pair.mode == kShared) && pipe_state_floats(a.dk, pair.wide) != (size_t)4 * NH * (DKP / 16) * 64 * 4)
         return LA_E_WORKSPACE;
     if (pair.wide != NH - 1) return LA_E_UNSUPPORTED;
     // the plain-matrix forms of the state exist in two instantiations only
     constexpr bool SAVES = !REVERSE && ((NH == 1 && NF == 1) || (NH == 2 && NF == 2));
     constexpr bool RESUMES = !REVERSE && ((NH == 2 && NF == 1) || (NH == 3 && NF == 2));
     if (pair.mode == kResume && (!RESUMES || pair.nprod != 1)) return LA_E_UNSUPPORTED;
-    if (SHARED && (a.nslice != 1 || pair.mode != kApply)) return LA_E_UNSUPPORTED;
-    if (pair.transposed && !SHARED) return LA_E_UNSUPPORTED;
-    // every chunk's slot must exist
-    if (SHARED && (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot)) return LA_E_WORKSPACE;
+    if ((pair.mode == kShared) != (pair.nslot > 0) || (pair.transposed && pair.mode != kShared)) return LA_E_UNSUPPORTED;
+    if (pair.mode == kShared) {
+        if (!kSquare<DKP, NF, NH> || SILU || a.nslice != 1) return LA_E_UNSUPPORTED;
+        // every chunk's slot must exist
+        if (pair.slot_mul < 1 || (int64_t)(a.nchunk - 1) * pair.slot_mul > pair.nslot) return LA_E_WORKSPACE;
+    }
     if (pair.save && (!SAVES || pair.nprod != 1 || pair.mode != kWarmUp || a.nchunk != 1)) return LA_E_UNSUPPORTED;
     const unsigned grid = (unsigned)(units8 * a.nslice * a.nchunk * pair.nprod);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, pair);
@@ -998,12 +1009,6 @@ static int prep_family() {
     LA_P(false, false, false) LA_P(false, false, true) LA_P(false, true, false) LA_P(false, true, true)
     LA_P(true, false, false) LA_P(true, false, true) LA_P(true, true, false) LA_P(true, true, true)
 #undef LA_P
-    if constexpr (NF == 1 && 4 * NH == DKP / 16) {
-#define LA_P(R, D, S) if (!e) e = prep_one<T, DKP, NF, NH, R, D, S, false, true>();
-        LA_P(false, false, false) LA_P(false, false, true) LA_P(false, true, false) LA_P(false, true, true)
-        LA_P(true, false, false) LA_P(true, false, true) LA_P(true, true, false) LA_P(true, true, true)
-#undef LA_P
-    }
     if constexpr (NH == 1) {
 #define LA_P(D, S) if (!e) e = prep_both_one<T, DKP, NF, D, S>();
         LA_P(false, false) LA_P(false, true) LA_P(true, false) LA_P(true, true)

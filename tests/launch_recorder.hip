@@ -10,11 +10,11 @@ namespace {
 std::string log_;
 
 void note(const char* what, const la::SweepPair& p, bool reverse) {
-    static const char* const modes[] = {"warm", "scan", "apply", "resume"};
+    static const char* const modes[] = {"warm", "scan", "apply", "resume", "shared"};
     char t[200];
     snprintf(t, sizeof(t), "%s %s%s w%d x%d c%d", what, reverse ? "rev " : "", modes[p.mode], p.wide, p.nprod, p.a[0].nchunk);
     log_ += t;
-    if (p.shared) log_ += p.nprod == 2 ? " shared" : " carried";
+    if (p.nslot) log_ += p.nprod == 2 ? " shared" : " carried";
     if (p.save) log_ += " saving";
     log_ += ";";
 }
