@@ -488,7 +488,7 @@ int sweep2(const SweepIO& io0, const SweepIO& io1, const float* s, int64_t bh, i
         p = chunked(io0, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws));
         p.a[1] = chunked(io1, s, bh, h, n, dk, dv, width, sh.nchunk, sh.chunk_len, static_cast<float*>(ws)).a[0];
         p.nprod = 2;
-        p.nslot = sh.ncollect - 1;
+            p.nslot = sh.ncollect - 1;
         p.slot_mul = sh.mul;
         p.transposed = 2;
         return sweep_pipe_apply(p, dtype, reverse, st);
@@ -595,13 +595,22 @@ static bool trio_chosen(int64_t bh, int64_t n, int64_t d, int64_t e, size_t scra
     const int v_width = column_width(bh, n, d, e, 1, scratch, opts);
     const DqDkPlan q = plan_dq_dk(bh, n, e, d, scratch, opts, dq_us);
     double separate = q.us + width_us(bh, n, d, e, 1, v_width, scratch, opts);
-    // Rows of d above 96 against rows of e = 49 .. 64, chunked: block_us is 11 % too long for the two sweeps over e, and a scanned dV takes
-    // 5 us less than estimated (10 with up to 8 sequences).  la_bwd of e64, one launch / dQ + dK and dV, us, d128: b*h = 8, n = 4096 60 / 62,
-    // 5120 74 / 71, 6016 86 / 80; 16, 4096 65 / 68, 6016 92 / 90; 24, 6016 103 / 107, 8192 138 / 135, 16384 278 / 254.  Rows of
-    // d = 97 .. 112 only with up to 8 sequences (d104: 8, 5120 74 / 71, but 24, 8192 142 / 151), narrower ones nowhere (e40: 8, 6016 73 / 79).
-    if (d > 96 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d > 112 || units8 == 8)) {
-        const ScanPlan v = plan_scan(bh, n, d, e, 1, v_width, opts);
-        separate -= 0.11 * q.us + (v.nchunk > 1 && v.bytes <= scratch ? (units8 == 8 ? 10.0 : 5.0) : 0.0);
+    // Where long rows meet short ones (64 and less) the separate launches are quicker than estimated with few sequences: a sweep
+    // scanned in 64-column workgroups by 10 us with up to 8, by 5 with more, two chunked sweeps over e = 49 .. 64 by 11 %.
+    // la_bwd of e64, one launch / dQ + dK and dV, us, d128: b*h = 8, n = 4096 60 / 62, 5120 74 / 71, 6016 86 / 80; 16, 4096 65 / 68, 6016
+    // 92 / 90; 24, 6016 103 / 107, 8192 138 / 135, 16384 278 / 254; d96: 10, 8192 123 / 108; 18, 10240 169 / 160 (not so d = 97 .. 112 beyond 8
+    // sequences, d104: 24, 8192 142 / 151, nor narrower e, d128 e40: 8, 6016 73 / 79).  One launch / apart, d64 e128: 2, 6016 88 / 74; 8, 4096
+    // 62 / 72, 6016 88 / 81; 10, 8192 120 / 110; 24, 12288 204 / 208; d40 e96: 2, 6016 77 / 70; 8, 6016 77 / 80; 16, 8192 106 / 109.
+    auto scanned = [&](int64_t dk, int64_t dv, int width) {
+        const ScanPlan pl = plan_scan(bh, n, dk, dv, 1, width, opts);
+        return width == 0 && pl.nchunk > 1 && pl.bytes <= scratch ? 1.0 : 0.0;
+    };
+    const double each = units8 == 8 ? 10.0 : 5.0;
+    if (d <= 64 && e > 64 && units8 <= 16 && (e > 96 || bh <= 4)) {
+        separate -= each * scanned(d, e, v_width);
+        if (!q.together) separate -= 2.0 * each * scanned(e, d, column_width(bh, n, e, d, 1, scratch, opts));
+    } else if (d > 64 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d <= 96 || d > 112 || units8 == 8)) {
+        separate -= 0.11 * q.us + each * scanned(d, e, v_width);
     }
     return warm_up_frac(wgs, nblk, opts) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) < separate;
 }

@@ -53,8 +53,13 @@ def test_one_launch_for_three_sweeps_of_different_rows():
     """d = 128, e = 64: three sweeps in one launch where that measures faster than dQ + dK in one and dV scanned."""
     got = routes([(bh, n, 128, 64, BF16) for bh, n in ((8, 2048), (8, 4096), (16, 2048), (16, 4096), (24, 6016), (40, 16384))])
     assert all(r["bwd"].startswith("trio") for r in got.values()), got
-    got = routes([(bh, n, 128, 64, BF16) for bh, n in ((1, 5120), (8, 5120), (8, 6016), (16, 6016), (24, 12288), (24, 16384))])
+    got = routes([(bh, n, 128, 64, BF16) for bh, n in ((1, 5120), (8, 5120), (8, 6016), (16, 6016), (24, 12288), (24, 16384))] +
+                 [(2, 6509, 80, 64, BF16), (10, 8192, 96, 64, BF16), (18, 10240, 80, 64, BF16)])
     assert all(r["bwd"].startswith("dq+dk") for r in got.values()), got
+    got = routes([(8, 4096, 64, 128, BF16), (24, 12288, 64, 128, BF16), (48, 16384, 64, 128, BF16), (24, 8192, 104, 64, BF16), (16, 8192, 40, 96, BF16), (8, 6016, 40, 96, BF16)])
+    assert all(r["bwd"].startswith("trio") for r in got.values()), got
+    got = routes([(2, 6016, 64, 128, BF16), (8, 6016, 64, 128, BF16), (10, 8192, 64, 128, BF16), (2, 6016, 40, 96, BF16)])
+    assert all("trio" not in r["bwd"] and r["bwd"].count("scan") == 3 for r in got.values()), got
 
 
 def test_what_is_kept_is_read():
