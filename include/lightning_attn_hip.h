@@ -218,7 +218,8 @@ int la_bwd_saved(const void *q, const void *k, const void *v, const float *s, co
  * the forward pass runs in chunks from scanned states (few long sequences) and the dQ sweep has the same chunks - the
  * state slots the forward pass works with anyway.  The contents of `carry` are opaque: la_bwd_carry must be given what
  * la_fwd_carry left for the same tensors, shapes and options on the same device; it only reads it.
- * la_carry_bytes: bytes to provide (16-byte aligned), 0 where nothing would be kept.  With carry == NULL or too few
+ * la_carry_bytes: bytes to provide (16-byte aligned), 0 where nothing would be kept or a backward pass with the workspace
+ * it asks for would not read it.  With carry == NULL or too few
  * bytes the calls are la_fwd_opts and la_bwd_opts; where bytes are provided la_fwd_carry needs no workspace.
  */
 size_t la_carry_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int64_t e, int dtype, const la_launch_opts *opts);
