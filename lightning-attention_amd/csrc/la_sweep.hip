@@ -525,8 +525,8 @@ static bool once_chosen(int64_t bh, int64_t n, int64_t d, size_t scratch, const 
     double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
     // Short rows and a shared plan of two chunks per sweep: more than the last-level cache holds, the separate launches
     // take as long as their twelve passes over a tensor (this launch: ten), not as long as their blocks.  la_bwd of d64, separate /
-    // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
-    if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.4e6);
+    // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 56, 24576 397 / 363; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
+    if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.1e6);
     // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
     // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
     // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
@@ -611,6 +611,8 @@ static bool trio_chosen(int64_t bh, int64_t n, int64_t d, int64_t e, size_t scra
         if (!q.together) separate -= 2.0 * each * scanned(e, d, column_width(bh, n, e, d, 1, scratch, opts));
     } else if (d > 64 && e > 48 && e <= 64 && q.together && units8 * slices(e, d, 0) * 4 <= cus && (d <= 96 || d > 112 || units8 == 8)) {
         separate -= 0.11 * q.us + each * scanned(d, e, v_width);
+    } else if (d > 64 && e <= 48 && q.together && units8 * slices(e, d, 0) * 4 <= cus && wgs * 2 > cus) {
+        separate -= each * scanned(d, e, v_width);  // (two chunks against none: d128 e40: 32, 3072 66 / 68, 4096 88 / 84)
     }
     return warm_up_frac(wgs, nblk, opts) * (double)nblk * std::max(block_us(d, 0), block_us(e, 0)) < separate;
 }
