@@ -520,13 +520,14 @@ static bool once_chosen(int64_t bh, int64_t n, int64_t d, size_t scratch, const 
     // (up to two rounds of workgroups: on a short walk one launch of twice as many 64-column workgroups as
     // there are CUs still beats two launches - b1 h48 n2048 d192: la_bwd 0.138 against 0.162 ms)
     if (wgs > 2 * cus) return false;
+    // 45 .. 64 sequences of d = 49 .. 64: one round of up to 192 workgroups, ten passes over a tensor, and by then as near to what the
+    // memory system gives as the twelve passes of carried and shared states in fewer blocks.  la_bwd of d64, one launch / those, us:
+    // 48 sequences n = 8192 119 / 123, 16384 235 / 230, 49152 692 / 728; 52, 24576 350 / 370; 56, 24576 360 / 397; 64, 65536 1065 / 1175.
+    // (Not so 41 sequences, n = 32768 465 / 436, nor narrower rows: 64 of d40, n = 65536, 936 / 855.)
+    if (d > 48 && d <= 64 && bh > 44 && bh <= 64) return true;
     // what the separate launches would take, by the estimates behind their own plans
     const SharedPlan sh = plan_shared(bh, n, d, scratch, opts);
-    double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
-    // Short rows and a shared plan of two chunks per sweep: more than the last-level cache holds, the separate launches
-    // take as long as their twelve passes over a tensor (this launch: ten), not as long as their blocks.  la_bwd of d64, separate /
-    // one launch, us: 64 sequences n = 24576 435 / 403, 65536 1175 / 1065; 56, 24576 397 / 363; 52, 49152 760 / 712; 48, 32768 466 / 471; 41, 32768 436 / 465.
-    if (d <= 64 && sh.nchunk == 2) separate = std::max(separate, (12.0 * (double)(bh * n * d) * 2.0 - 512e6) / 4.1e6);
+    const double separate = (dq_us > 0.0 ? dq_us : width_us(bh, n, d, d, 1, column_width(bh, n, d, d, 1, scratch, opts), scratch, opts)) + sh.us;
     // here: the longest workgroup of 3 * wgs/3 * c warm-up chunked ones, or two rounds of single walks
     // (of which the second starts while the first ends, where a second launch would wait for it: la_bwd in one / two
     // launches, b1 h48 d128 n = 256 19.0 / 19.9 us, n = 512 31.5 / 29.5; h32 d192 n = 256 23.4 / 24.4, n = 512 40.1 / 38.3)
