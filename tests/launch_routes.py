@@ -15,9 +15,12 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "lightning-attention_amd", "lightning_attn", "_C", "liblightning_attn_hip.so")
 
 
+_folder = tempfile.TemporaryDirectory(prefix="la_routes_")  # (gone when this process ends)
+
+
 @functools.lru_cache(None)
 def _recorder():
-    out = os.path.join(tempfile.mkdtemp(prefix="la_routes_"), "recorder.so")
+    out = os.path.join(_folder.name, "recorder.so")
     hipcc = os.environ.get("HIPCC") or "/opt/rocm/bin/hipcc"
     subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-fPIC", "-shared", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                     "-packed-fp32-ops", "-Wno-unknown-warning-option", "-I", os.path.join(ROOT, "include"), "-I",
