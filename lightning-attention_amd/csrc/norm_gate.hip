@@ -6,8 +6,11 @@
 //
 // Same data movement as the SimpleRMSNorm kernels: a row of o, g (and dy) is read once with 16-byte
 // non-temporal loads into registers, reduced, and the results written once.  TPR threads share a row:
-// 64, 128, 256, 512 or 1024, with as many rows side by side as the workgroup has room for.  The forward kernel takes one
-// group of rows per workgroup and fetches weight and bias from the caches.  The backward kernel walks the rows with a grid stride and gives every thread one
+// 8, 16, 32, 64, 128, 256, 512 or 1024, with as many rows side by side as the workgroup has room for.  The
+// forward kernel takes one group of rows per workgroup and fetches weight and bias from the caches; it is bound by memory, once
+// nothing waits between its reductions: us, before weight and bias came along with the row and before short rows shared a
+// wavefront / now, bf16: [16384,2048] 38.3 / 33.0 (6.1 TB/s), [4096,8192] 39.6 / 36.0, [16384,1024] 19.0 / 17.1, [700,2048] 6.0 / 4.6,
+// [131072,64] 49.3 / 10.1, [40000,200] 19.1 / 11.7; float32 [16384,1024] 37.6 / 31.9, [131072,64] 41.1 / 16.9.  The backward kernel walks the rows with a grid stride and gives every thread one
 // 16-byte chunk of the row: a thread always holds the same columns, so weight and bias stay in registers
 // as floats and the column sums (d weight, d bias) are accumulated in registers over all rows a thread
 // sees (117 registers: four waves per SIMD; with more chunks per thread it ran at two).  Those partial
@@ -21,7 +24,7 @@
 // [1024,512] 8.3 / 7.1, [512,1024] 8.2 / 7.8.
 // Backward pass with its reduction, bf16, us before / after: [16384,2048] 87.2 / 62.9 (5.3 TB/s), [8192,1024] 33.9 / 22.6,
 // [32768,4096] 259 / 225 (6.0 TB/s), [32768,512] 42.0 / 34.7, [4096,8192] 85.5 / 65.1, [700,2048] 22.7 / 9.8.  float32 has the
-// vector loads alone: [16384,4096] 252 / 236, [1024,1024] 17.4 / 14.7, [16,64] the same; one shape is slower, [16384,64] 13.2 / 14.5.
+// vector loads alone: [16384,4096] 252 / 236, [1024,1024] 17.4 / 14.7, [16,64] the same.
 //
 // Per element, float32 throughout:
 //   forward   xh = (o - mean) rstd ; ln = xh w + b ; sg = 1 / (1 + exp(-g)) ; y = ln sg
@@ -66,7 +69,7 @@ __device__ __forceinline__ void row_sum2(float& a, float& b, float* red) {
         return;
     }
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
+    for (int m = TPR / 2; m >= 1; m >>= 1) {
         a += __shfl_xor(a, m, 64);
         b += __shfl_xor(b, m, 64);
     }
@@ -84,74 +87,92 @@ __global__ __launch_bounds__(ng_threads(TPR)) void norm_gate_fwd_kernel(const T*
                                                                   T* __restrict__ y, float* __restrict__ mean,
                                                                   float* __restrict__ rstd, int64_t rows, int cols, float eps) {
     constexpr int E = Pack16<T>::N;
-    constexpr int RPG = ng_threads(TPR) / TPR;  // rows a workgroup holds at a time
+    constexpr int RPG = ng_threads(TPR) / TPR;  // rows a workgroup holds
     __shared__ float red[32];
     const int l = threadIdx.x % TPR;
     const float inv = 1.0f / (float)cols;
-    for (int64_t row0 = (int64_t)blockIdx.x * RPG; row0 < rows; row0 += (int64_t)gridDim.x * RPG) {
-        const int64_t row = row0 + threadIdx.x / TPR;
-        const bool row_ok = row < rows;
-        const T* orow = o + row * (int64_t)cols;
-        const T* grow = g + row * (int64_t)cols;
-        T* yrow = y + row * (int64_t)cols;
-        Pack16<T> po[NV], pg[NV];
+    const int64_t row = (int64_t)blockIdx.x * RPG + threadIdx.x / TPR;
+    const bool row_ok = row < rows;
+    const T* orow = o + row * (int64_t)cols;
+    const T* grow = g + row * (int64_t)cols;
+    T* yrow = y + row * (int64_t)cols;
+    // weight and bias come from the caches (every row reads the same cols elements).  Requested along with the row, so that
+    // the last pass does not wait for them - but for float32 rows of several wavefronts, where the registers cost more
+    // ([32768,4096] 259 / 268 us).
+    constexpr bool EARLY = sizeof(T) == 2 || TPR <= 64;
+    Pack16<T> po[NV], pg[NV], pw[NV], pb[NV];
+    auto affine = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
             const int c = (u * TPR + l) * E;
             if (row_ok && c < cols) {
-                po[u] = load16(orow + c);
-                pg[u] = load16(grow + c);
+                pw[u] = *reinterpret_cast<const Pack16<T>*>(w + c);
+                pb[u] = *reinterpret_cast<const Pack16<T>*>(b + c);
             }
         }
-        float s = 0.f, dummy = 0.f;
+    };
 #pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int c = (u * TPR + l) * E;
-            if (row_ok && c < cols) {
+    for (int u = 0; u < NV; ++u) {
+        const int c = (u * TPR + l) * E;
+        if (row_ok && c < cols) {
+            po[u] = load16(orow + c);
+            pg[u] = load16(grow + c);
+        }
+    }
+    if (EARLY) affine();
+    float s = 0.f, dummy = 0.f;
 #pragma unroll
-                for (int t = 0; t < E; ++t) s += (float)po[u].v[t];
+    for (int u = 0; u < NV; ++u) {
+        const int c = (u * TPR + l) * E;
+        if (row_ok && c < cols) {
+#pragma unroll
+            for (int t = 0; t < E; ++t) s += (float)po[u].v[t];
+        }
+    }
+    row_sum2<TPR>(s, dummy, red);
+    const float mu = s * inv;
+    // only the packed inputs live across the reductions: the passes convert them again
+#pragma unroll
+    for (int u = 0; u < NV; ++u) forget(po[u]);
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = (u * TPR + l) * E;
+        if (row_ok && c < cols) {
+#pragma unroll
+            for (int t = 0; t < E; ++t) {
+                const float dlt = (float)po[u].v[t] - mu;
+                ss += dlt * dlt;
             }
         }
-        row_sum2<TPR>(s, dummy, red);
-        const float mu = s * inv;
-        // only the packed inputs live across the reductions: the passes convert them again
+    }
+    row_sum2<TPR>(ss, dummy, red);
+    const float rs = 1.0f / sqrtf(ss * inv + eps);
 #pragma unroll
-        for (int u = 0; u < NV; ++u) forget(po[u]);
-        float ss = 0.f;
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int c = (u * TPR + l) * E;
-            if (row_ok && c < cols) {
-#pragma unroll
-                for (int t = 0; t < E; ++t) {
-                    const float dlt = (float)po[u].v[t] - mu;
-                    ss += dlt * dlt;
-                }
-            }
+    for (int u = 0; u < NV; ++u) {
+        forget(po[u]);
+        forget(pg[u]);
+        if (EARLY) {
+            forget(pw[u]);
+            forget(pb[u]);
         }
-        row_sum2<TPR>(ss, dummy, red);
-        const float rs = 1.0f / sqrtf(ss * inv + eps);
+    }
+    if (!EARLY) affine();
+    if (l == 0 && row_ok) {
+        mean[row] = mu;
+        rstd[row] = rs;
+    }
 #pragma unroll
-        for (int u = 0; u < NV; ++u) forget(po[u]);
-        if (l == 0 && row_ok) {
-            mean[row] = mu;
-            rstd[row] = rs;
-        }
+    for (int u = 0; u < NV; ++u) {
+        const int c = (u * TPR + l) * E;
+        if (row_ok && c < cols) {
+            Pack16<T> out;
 #pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int c = (u * TPR + l) * E;
-            if (row_ok && c < cols) {
-                // weight and bias come from the caches (every row reads the same cols elements)
-                const Pack16<T> pw = *reinterpret_cast<const Pack16<T>*>(w + c);
-                const Pack16<T> pb = *reinterpret_cast<const Pack16<T>*>(b + c);
-                Pack16<T> out;
-#pragma unroll
-                for (int t = 0; t < E; ++t) {
-                    const float ln = ((float)po[u].v[t] - mu) * rs * (float)pw.v[t] + (float)pb.v[t];
-                    out.v[t] = (T)(ln * sigmoidf((float)pg[u].v[t]));
-                }
-                store16(yrow + c, out);
+            for (int t = 0; t < E; ++t) {
+                const float ln = ((float)po[u].v[t] - mu) * rs * (float)pw[u].v[t] + (float)pb[u].v[t];
+                out.v[t] = (T)(ln * sigmoidf((float)pg[u].v[t]));
             }
+            store16(yrow + c, out);
         }
     }
 }
@@ -169,8 +190,9 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
     constexpr int E = Pack16<T>::N;
     constexpr int RPG = ng_bwd_threads(TPR, sizeof(T), FEW) / TPR;
     constexpr bool AHEAD = sizeof(T) == 2;
+    constexpr int SIDE = TPR < 64 ? RPG * TPR / 64 : RPG;  // column sums to add up once the rows of a wavefront are
     __shared__ float red[64];
-    __shared__ float comb[RPG > 1 ? (RPG - 1) * TPR * NV * E * 2 : 1];  // column sums of the rows beside the first
+    __shared__ float comb[SIDE > 1 ? (SIDE - 1) * TPR * NV * E * 2 : 1];  // column sums of the rows beside the first
     const int l = threadIdx.x % TPR;
     float wf[NV][E], bf[NV][E];  // this thread's columns of weight and bias
     float aw[NV][E], ab[NV][E];  // ... and of the column sums
@@ -263,9 +285,24 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
         }
     }
     // column sums of this workgroup: the thread groups of its rows hold the same columns and are
-    // added up in row order first
-    if (RPG > 1) {
-        const int grp = threadIdx.x / TPR;
+    // added up in a fixed order first, those of a wavefront by shuffles
+    if (TPR < 64) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int t = 0; t < E; ++t)
+#pragma unroll
+                for (int m = TPR; m < 64; m *= 2) {
+                    aw[u][t] += __shfl_xor(aw[u][t], m, 64);
+                    ab[u][t] += __shfl_xor(ab[u][t], m, 64);
+                }
+        if ((threadIdx.x & 63) >= TPR) {
+            if (SIDE > 1) __syncthreads();
+            return;
+        }
+    }
+    if (SIDE > 1) {
+        const int grp = threadIdx.x / (TPR < 64 ? 64 : TPR);
         if (grp > 0) {
 #pragma unroll
             for (int u = 0; u < NV; ++u)
@@ -278,7 +315,7 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
         __syncthreads();
         if (grp > 0) return;
 #pragma unroll
-        for (int k = 0; k < RPG - 1; ++k)
+        for (int k = 0; k < SIDE - 1; ++k)
 #pragma unroll
             for (int u = 0; u < NV; ++u)
 #pragma unroll
@@ -345,19 +382,22 @@ __global__ __launch_bounds__(kRedCols * kRedGroups) void norm_gate_reduce_kernel
 }
 
 // Threads per row and 16-byte chunks per thread for rows of `chunks` chunks (nv = 0: too wide).  The
-// forward kernel holds little per column and gives a wavefront rows of up to 512 chunks; the backward
+// forward kernel holds little per column and gives a wavefront rows of up to 256 chunks, or several short ones; the backward
 // kernel carries weight, bias and two column sums per column and spreads rows over the workgroup earlier.
-static void ng_shape(int64_t chunks, bool backward, int* tpr, int* nv) {
+static void ng_shape(int64_t rows, int64_t chunks, bool backward, int* tpr, int* nv) {
     *nv = 0;
     if (backward) {
         // one chunk per thread: the kernel keeps ~7 floats per element of a thread's columns
         if (chunks > 1024) return;
         *nv = 1;
-        *tpr = chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : chunks <= 512 ? 512 : 1024;
+        // short rows share a wavefront where a row to a wavefront would take more than one pass (us, bf16, a row to a wavefront / shared:
+        // [131072,64] 63.6 / 20.8, [16384,64] 14.0 / 9.8, [40000,200] 27.4 / 21.0; but [1,64] 4.9 / 5.7, [512,256] 6.0 / 6.5)
+        const bool many = rows > 16 * (int64_t)num_cus();
+        *tpr = many && chunks <= 8 ? 8 : many && chunks <= 16 ? 16 : many && chunks <= 32 ? 32 : chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : chunks <= 512 ? 512 : 1024;
         return;
     }
     if (chunks <= 64 * 4) {
-        *tpr = 64;
+        *tpr = chunks <= 8 ? 8 : chunks <= 16 ? 16 : chunks <= 32 ? 32 : 64;
         *nv = 1;
         while (64 * *nv < chunks) *nv *= 2;
     } else if (chunks <= 256 * 4) {
@@ -383,7 +423,10 @@ static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
 #define LA_NG_GO(KERNEL, NV, TPR, THREADS, ...) hipLaunchKernelGGL((KERNEL<T, NV, TPR>), grid, dim3(THREADS), 0, st, __VA_ARGS__)
 #define LA_NG_DISPATCH_FWD(KERNEL, ...)                               \
     do {                                                              \
-        if (tpr == 64 && nv == 1) LA_NG_GO(KERNEL, 1, 64, ng_threads(64), __VA_ARGS__);       \
+        if (tpr == 8) LA_NG_GO(KERNEL, 1, 8, ng_threads(8), __VA_ARGS__);                     \
+        else if (tpr == 16) LA_NG_GO(KERNEL, 1, 16, ng_threads(16), __VA_ARGS__);             \
+        else if (tpr == 32) LA_NG_GO(KERNEL, 1, 32, ng_threads(32), __VA_ARGS__);             \
+        else if (tpr == 64 && nv == 1) LA_NG_GO(KERNEL, 1, 64, ng_threads(64), __VA_ARGS__);  \
         else if (tpr == 64 && nv == 2) LA_NG_GO(KERNEL, 2, 64, ng_threads(64), __VA_ARGS__);  \
         else if (tpr == 64) LA_NG_GO(KERNEL, 4, 64, ng_threads(64), __VA_ARGS__);             \
         else if (nv == 1) LA_NG_GO(KERNEL, 1, 256, ng_threads(256), __VA_ARGS__);              \
@@ -395,8 +438,14 @@ static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
     do {                                                              \
         constexpr bool kFew = sizeof(T) == 2;                         \
         const bool few = ng_few(rows, tpr, sizeof(T));                \
-        if (tpr == 64 && few) LA_NG_BWD(64, kFew, __VA_ARGS__);       \
+        if (tpr == 8 && few) LA_NG_BWD(8, kFew, __VA_ARGS__);         \
+        else if (tpr == 16 && few) LA_NG_BWD(16, kFew, __VA_ARGS__);  \
+        else if (tpr == 32 && few) LA_NG_BWD(32, kFew, __VA_ARGS__);  \
+        else if (tpr == 64 && few) LA_NG_BWD(64, kFew, __VA_ARGS__);  \
         else if (tpr == 128 && few) LA_NG_BWD(128, kFew, __VA_ARGS__); \
+        else if (tpr == 8) LA_NG_BWD(8, false, __VA_ARGS__);          \
+        else if (tpr == 16) LA_NG_BWD(16, false, __VA_ARGS__);        \
+        else if (tpr == 32) LA_NG_BWD(32, false, __VA_ARGS__);        \
         else if (tpr == 64) LA_NG_BWD(64, false, __VA_ARGS__);        \
         else if (tpr == 128) LA_NG_BWD(128, false, __VA_ARGS__);      \
         else if (tpr == 256) LA_NG_BWD(256, false, __VA_ARGS__);      \
@@ -408,7 +457,7 @@ template <typename T>
 static int ng_fwd(const void* o, const void* g, const void* w, const void* b, void* y, float* mean, float* rstd, int64_t rows,
                   int64_t cols, float eps, hipStream_t st) {
     int tpr = 0, nv = 0;
-    ng_shape(cols / (16 / (int64_t)sizeof(T)), false, &tpr, &nv);
+    ng_shape(rows, cols / (16 / (int64_t)sizeof(T)), false, &tpr, &nv);
     if (!nv) return LA_E_UNSUPPORTED;
     const dim3 grid((unsigned)ng_grid(rows, tpr, false, sizeof(T)));
     LA_NG_DISPATCH_FWD(norm_gate_fwd_kernel, static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
@@ -421,7 +470,7 @@ static int ng_bwd(const void* o, const void* g, const void* w, const void* b, co
                   const void* dy, void* d_o, void* d_g, void* dweight, void* dbias, float* part, int64_t rows, int64_t cols,
                   hipStream_t st) {
     int tpr = 0, nv = 0;
-    ng_shape(cols / (16 / (int64_t)sizeof(T)), true, &tpr, &nv);
+    ng_shape(rows, cols / (16 / (int64_t)sizeof(T)), true, &tpr, &nv);
     if (!nv) return LA_E_UNSUPPORTED;
     const dim3 grid((unsigned)ng_grid(rows, tpr, true, sizeof(T)));
     LA_NG_DISPATCH_BWD(static_cast<const T*>(o), static_cast<const T*>(g), static_cast<const T*>(w),
@@ -464,7 +513,7 @@ extern "C" int norm_gate_supported(int64_t cols, int dtype) {
 extern "C" size_t norm_gate_workspace_bytes(int64_t rows, int64_t cols, int dtype) {
     if (rows <= 0 || !norm_gate_supported(cols, dtype)) return 0;
     int tpr = 0, nv = 0;
-    la::ng_shape(cols / (dtype == LA_FP32 ? 4 : 8), true, &tpr, &nv);
+    la::ng_shape(rows, cols / (dtype == LA_FP32 ? 4 : 8), true, &tpr, &nv);
     return (size_t)la::ng_grid(rows, tpr, true, dtype == LA_FP32 ? 4 : 2) * 2 * (size_t)cols * sizeof(float);
 }
 

@@ -46,3 +46,21 @@ def test_row_counts_around_the_small_workgroups(cols, side, dtype):
         want = oracle.norm_gate_fwd_bwd(o, g, w, b, dy, 1e-5, torch.float64)
         for name, a, r in zip(("y", "d_o", "d_g", "d_weight", "d_bias"), got, want):
             assert rel_norm(a.detach().cpu(), r) < lim, (rows, name, rel_norm(a.detach().cpu(), r))
+
+
+@pytest.mark.parametrize("cols", [8, 64, 72, 128, 136, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_short_rows_side_by_side(cols, dtype):
+    """Rows of up to 32 chunks of 16 bytes: 8, 4 or 2 of them to a wavefront - always in the forward pass, beyond 16 rows per CU
+    (4096) in the backward pass; the last workgroup of a launch with one row, all but one or all of them."""
+    lim = {torch.bfloat16: 5e-3, torch.float16: 1e-3, torch.float32: 2e-5}[dtype]
+    for rows in (1, 31, 32, 33, 4096, 4097, 8193, 32768, 65537):
+        g_ = torch.Generator().manual_seed(rows + cols)
+        o, g, dy = ((torch.randn(rows, cols, generator=g_) * 2).to(dtype) for _ in range(3))
+        w, b = (torch.randn(cols, generator=g_).to(dtype) for _ in range(2))
+        leaves = [t.cuda().requires_grad_() for t in (o, g, w, b)]
+        y = norm_gate(*leaves, 1e-5)
+        got = (y,) + torch.autograd.grad(y, leaves, dy.cuda())
+        want = oracle.norm_gate_fwd_bwd(o, g, w, b, dy, 1e-5, torch.float64)
+        for name, a, r in zip(("y", "d_o", "d_g", "d_weight", "d_bias"), got, want):
+            assert rel_norm(a.detach().cpu(), r) < lim, (rows, name, rel_norm(a.detach().cpu(), r))
