@@ -23,9 +23,10 @@ int prepare_plans() { return num_cus() > 0 ? 0 : (int)hipErrorInvalidDevice; }
 
 // Sequence chunks per (batch, head, slice).  With few sequences a single sweep per sequence
 // leaves most of the 256 CUs idle; the walk is then cut into up to 8 chunks whose workgroups
-// rebuild their incoming state themselves.  A warm-up block costs about half a full block, so
-// chunk lengths shrink geometrically (len_c ~ (1 - rho)^c, rho = 0.5) to make all workgroups
-// finish together.  The caller's launch options can override the count.
+// rebuild their incoming state themselves.  A warm-up block costs about a third of a full block, half of one where two chunks a
+// sequence fill the chip, so chunk lengths shrink geometrically (len_c ~ (1 - rho)^c) to make all workgroups
+// finish together (two chunks, rho 0.36 / 0.5: b4 h32 n1024 d64 16.5 / 16.2, b2 h32 n2048 d128 36.5 / 35.8, b2 h32 n8192 d128 e64 107 / 112; more: la_fwd of b2 h12 n2048 d192, us, by rho 0.25 / 0.3 / 0.36 / 0.45 / 0.5: 39.4 / 38.0 / 38.1 / 40.7 / 42.8; b1 h4 n1000 d128
+// 16.3 / 16.2 / 15.6 / 15.5 / 16.2; b1 h8 n2048 d64 16.3 / 16.9 / 16.1 / 17.3 / 18.2).  The caller's launch options can override the count.
 static int64_t warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int64_t min_blocks = 4) {
     int64_t c = 1;
     if (wgs * 2 <= cus && nblk >= 2 * min_blocks) {
@@ -40,6 +41,7 @@ void plan_warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int forced, int
     if (c > 8) c = 8;
     if (c > nblk) c = nblk;
     if (c < 1) c = 1;
+    if (rho <= 0.0) rho = c == 2 ? 0.5 : 0.36;
     // geometric lengths, at least one block each, summing to nblk
     double wsum = 0.0, wgt = 1.0;
     for (int i = 0; i < c; ++i) { wsum += wgt; wgt *= 1.0 - rho; }
@@ -83,8 +85,10 @@ struct ScanPlan {
 };
 
 // Estimates, in microseconds, behind the choices below.  A workgroup takes about block_us per 64-token
-// block (measured, by feature dim and columns per workgroup) and half of that for a block it only folds
-// into the state.  Warm-up blocks: with the geometric chunk lengths of choose_chunks the longest
+// block (measured, by feature dim and columns per workgroup) and, when the lines between the forms were drawn, half of that for
+// a block it only folds into the state; with the warm-up walk of its own (a third) both the warm-up form and the collect launches became
+// quicker, and the lines stayed where they were: over 120 shapes (d 64 .. 256, b*h 1 .. 64, n 2048 .. 8192) the other side is more than 4 % quicker
+// in four, 12 % at most (b1 h32 n2048 d192).  Warm-up blocks: with the geometric chunk lengths of choose_chunks the longest
 // workgroup runs the fraction `frac` of a single walk.  Scanned states: a chunk one and a half times,
 // plus two more launches and the scan (16 us measured, and 10 for the host's share).
 // `width` of a workgroup: 0 = 64 columns of z / out, 1 = 128 (96 where there are 192 to share out), 2 = all

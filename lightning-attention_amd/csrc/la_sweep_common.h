@@ -170,9 +170,9 @@ int sweep_pipe_trio(const SweepTrio& t, int dtype, hipStream_t st);
 
 // Count (up to 8) and first blocks, chunk_start[0 .. 8], of the warm-up chunks for a launch that would have
 // `wgs` workgroups with one chunk each, on a walk of nblk blocks and `cus` compute units; `forced` > 0 overrides the count.
-// `rho`: what a warm-up block costs of a full one; `min_blocks`: fewest blocks per chunk (on average).
+// `rho`: what a warm-up block costs of a full one (0: the pipelined kernel's); `min_blocks`: fewest blocks per chunk (on average).
 // Defined in la_sweep.hip.
-void plan_warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start, double rho = 0.5, int64_t min_blocks = 4);
+void plan_warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int forced, int* nchunk, int* chunk_start, double rho = 0.0, int64_t min_blocks = 4);
 
 // Raises a kernel's dynamic LDS limit above the 64 KB default, once per kernel and device (the call is
 // not free and the limit stays).  `done` is the instantiation's own flag array, one entry per device.

@@ -280,17 +280,17 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     auto z_col = [&](int u) { return ZAL ? lane_zcol : col0 + ((tid + NL * u) % CPR) * 8; };
     auto z_lds = [&](int u) { return (unsigned)(z_row(u) * ZS + (z_col(u) - col0)) * (unsigned)sizeof(T); };
     // Fetches feature chunk HC of block number b of the walk and, with its first chunk, the z slice
-    // that travels with it.  Blocks at or beyond it_end, and the x tile of warm-up blocks, are fetched
+    // that travels with it.  Blocks at or beyond it_end are fetched
     // at the out-of-range offset: zeros, no memory traffic, and the loads are issued unconditionally
     // (no branches, no draining `s_waitcnt vmcnt(0)` at joins).
     auto load_step = [&](auto hc, int64_t b, u32x4 (&xr)[XC], u32x4 (&yr)[XC], u32x4 (&zr)[ZC]) __attribute__((always_inline)) {
         constexpr int HC = decltype(hc)::value;
         constexpr int FC0 = HC * DKH;  // first feature of the chunk
         const int64_t t = REVERSE ? nblk - 1 - b : b;
-        const bool valid = b < it_end, need_x = valid && b >= it_first;
+        const bool valid = b < it_end;
         // the z slice that travels with this block's x / y tiles
         const int64_t bz = b - ZLAG, tz = REVERSE ? nblk - 1 - bz : bz;
-        const bool validz = bz >= it0 && bz < it_end;
+        const bool validz = bz >= it_first && bz < it_end;
         if (DENSE) {
             // Plain tensors: one per-lane offset, rows >= n fall outside the buffer and the hardware
             // range check zeroes them.  Kept as its own code path because it is measurably faster
@@ -302,7 +302,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
                 const int c = tid + NL * u;
                 const int row = c / CPX, col = FC0 + (c % CPX) * 8;
                 const unsigned off = col < dk ? ((tok0 + row) * (unsigned)dk + col) * (unsigned)sizeof(T) : kOob;
-                xr[u] = buf_load16p<PX>(xb, need_x ? off : kOob);
+                xr[u] = buf_load16p<PX>(xb, valid ? off : kOob);
                 yr[u] = buf_load16p<PY>(yb, valid ? off : kOob);
             }
             if constexpr (HC == 0) {
@@ -318,7 +318,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
         }
         const unsigned tok0 = valid ? (unsigned)(t * 64) : 0u;
         // rows of this block that exist (0 for a block that is not fetched)
-        const int rows = valid ? (int)min(64u, nrows - tok0) : 0, rows_x = need_x ? rows : 0;
+        const int rows = valid ? (int)min(64u, nrows - tok0) : 0;
         if constexpr (ROWAL) {
             const unsigned lane_x = FC0 + lane_col < dk ? (lane_row * xts + FC0 + lane_col) * (unsigned)sizeof(T) : kOob;
             const unsigned lane_y = FC0 + lane_col < dk ? (lane_row * yts + FC0 + lane_col) * (unsigned)sizeof(T) : kOob;
@@ -326,7 +326,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
             for (int u = 0; u < XC; ++u) {
                 // a wave-uniform offset must stay inside the buffer: 0 when none of these rows exists
                 const unsigned tk = u * CROWS < rows ? tok0 + u * CROWS : 0u;
-                xr[u] = buf_load16p<PX>(xb, lane_row < rows_x - u * CROWS ? lane_x : kOob, tk * xts * (unsigned)sizeof(T));
+                xr[u] = buf_load16p<PX>(xb, lane_row < rows - u * CROWS ? lane_x : kOob, tk * xts * (unsigned)sizeof(T));
                 yr[u] = buf_load16p<PY>(yb, lane_row < rows - u * CROWS ? lane_y : kOob, tk * yts * (unsigned)sizeof(T));
             }
         } else {
@@ -336,7 +336,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
                 const int row = c / CPX, col = FC0 + (c % CPX) * 8;
                 const unsigned ox = col < dk ? (row * xts + col) * (unsigned)sizeof(T) : kOob;
                 const unsigned oy = col < dk ? (row * yts + col) * (unsigned)sizeof(T) : kOob;
-                xr[u] = buf_load16p<PX>(xb, row < rows_x ? ox : kOob, tok0 * xts * (unsigned)sizeof(T));
+                xr[u] = buf_load16p<PX>(xb, row < rows ? ox : kOob, tok0 * xts * (unsigned)sizeof(T));
                 yr[u] = buf_load16p<PY>(yb, row < rows ? oy : kOob, tok0 * yts * (unsigned)sizeof(T));
             }
         }
@@ -390,19 +390,19 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
             }
         }
     };
+    // SILU: silu(t) = t / (1 + exp(-t)) in float32, rounded back to the tensors' type; padding stays zero
+    auto silu16 = [](u32x4 v) {
+        typedef T T8 __attribute__((ext_vector_type(8)));
+        T8 t = __builtin_bit_cast(T8, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float f = (float)t[i];
+            t[i] = (T)(f * __builtin_amdgcn_rcpf(1.f + __expf(-f)));
+        }
+        return __builtin_bit_cast(u32x4, t);
+    };
     auto stage_step = [&](auto hc, int buf, int zslot, const u32x4 (&xr)[XC], const u32x4 (&yr)[XC], const u32x4 (&zr)[ZC], int64_t bout, bool flush) __attribute__((always_inline)) {
         constexpr int HC = decltype(hc)::value;
-        // SILU: silu(t) = t / (1 + exp(-t)) in float32, rounded back to the tensors' type; padding stays zero
-        auto silu16 = [](u32x4 v) {
-            typedef T T8 __attribute__((ext_vector_type(8)));
-            T8 t = __builtin_bit_cast(T8, v);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float f = (float)t[i];
-                t[i] = (T)(f * __builtin_amdgcn_rcpf(1.f + __expf(-f)));
-            }
-            return __builtin_bit_cast(u32x4, t);
-        };
         const unsigned xd = opaque(buf * XYB + (ROWAL ? lane_stage_xy : 0u));
         const unsigned zd = opaque(ZBASE + zslot * ZTB + (ZAL ? lane_stage_z : 0u));
         auto zoff = [&](int u) { return ZAL ? (unsigned)(u * ZROWS * ZS) * E : z_lds(u); };
@@ -498,7 +498,6 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
             }
         }
     };
-
     // zero both P buffers once: tiles on the masked side of the diagonal are never written
     for (int c = tid; c < 2 * L::PT / 8; c += 512) reinterpret_cast<uint4*>(smem + PBASE)[c] = make_uint4(0, 0, 0, 0);
     // state-wave lane offsets: x fragment halves (row r, columns 4g..), transposed reads of y and
@@ -546,7 +545,6 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
         constexpr int ROLE = decltype(role)::value;
         constexpr int HF = decltype(hf)::value;
         const bool have_next = it + 1 < it_end;
-        const bool warm = it < it_first;  // warm-up block: state update only
         const int bcur = (int)((unsigned)(it * NF + HF) % 3u);
         const int bnext = bcur == 2 ? 0 : bcur + 1;
         const int bstage = bnext == 2 ? 0 : bnext + 1;
@@ -569,7 +567,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
             }
             // the score tile runs one step ahead of the state waves
             const int64_t bc = it + (HF + 1) / NF;
-            if (bc < it_end && bc >= it_first) score_step(std::integral_constant<int, HC>{}, bnext, (int)(bc & 1));
+            if (bc < it_end) score_step(std::integral_constant<int, HC>{}, bnext, (int)(bc & 1));
         }
         if (ROLE == 1 && cols_active) {
             const unsigned xq = opaque(bcur * XYB + lane_xq);
@@ -591,7 +589,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
                         zf[h][ks] = cat<V8, V4>(ldt(zq + (32 * ks * ZS + 16 * h) * E), ldt(zq + ((32 * ks + 4) * ZS + 16 * h) * E));
             };
             if constexpr (!LEAN) read_z();
-            if (!warm) {
+            {
                 // out^T[c][i] = Lout[i] * sum_k state[k][c] x[i][k]  +  sum_j z[j][c] P[i][j]
                 // One slab: all x fragments are requested up front; LDS answers in order, so the
                 // MFMAs of contraction step ks start as soon as its own fragments are there while
@@ -721,13 +719,13 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
                         }
                 }
             }
-            if (have_next || mode == kCollect) {
+            if (have_next) {
                 // state = lam^64 state + y^T (z * Lupd), the rows of this feature chunk
                 constexpr int KT0 = HF * KTH;
                 // transposed y reads in batches where the state leaves no registers for all of them at once
                 constexpr int UB = (NF == 2 && NH == 2 && KTH > 6) ? 4 : LEAN ? 2 : KTH;
                 if constexpr (LEAN) {
-                    if (HF != NF - 1 || warm) read_z();
+                    if (HF != NF - 1) read_z();
                     if (DECAY) {
                         // (scaled before the y^T fragments are fetched: the factors and the fragments never share registers)
 #pragma unroll
@@ -797,7 +795,7 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // The two kinds of waves run separate copies of the loop (one barrier per step in each),
     // so that neither carries the other's registers.
     auto walk = [&](auto role) __attribute__((always_inline)) {
-        int64_t it = it0;
+        int64_t it = it_first;
         if constexpr (NF == 1) {
             for (; it + 1 < it_end; it += 2) {
                 iteration(role, C0{}, it, xrA, yrA, zrA);
@@ -824,26 +822,175 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // the compiler lays the branches out one after the other and keeps alive, while the first one
     // runs, whatever the second one needs of the values computed before this point - which must
     // therefore not include the score waves' prefetch registers.
+    // asked for ahead of the warm-up, whose own loads then cover their latency
+    auto first_loads = [&]() __attribute__((always_inline)) {
+        load_step(C0{}, it_first, xrA, yrA, zrA);
+        if constexpr (NF == 1) load_step(C0{}, it_first + 1, xrB, yrB, zrB);
+        else load_step(C1{}, it_first, xrB, yrB, zrB);
+    };
     auto prologue = [&]() __attribute__((always_inline)) {
-        const int b0 = (int)((unsigned)(it0 * NF) % 3u), b1 = b0 == 2 ? 0 : b0 + 1;
+        const int b0 = (int)((unsigned)(it_first * NF) % 3u), b1 = b0 == 2 ? 0 : b0 + 1;
         if constexpr (NF == 1) {
-            load_step(C0{}, it0, xrA, yrA, zrA);
-            load_step(C0{}, it0 + 1, xrB, yrB, zrB);
-            stage_step(C0{}, b0, NZ == 3 ? b0 : (int)((it0 + 1) & 1), xrA, yrA, zrA, 0, false);
-            load_step(C0{}, it0 + 2, xrA, yrA, zrA);
-            stage_step(C0{}, b1, NZ == 3 ? b1 : (int)(it0 & 1), xrB, yrB, zrB, 0, false);
-            load_step(C0{}, it0 + 3, xrB, yrB, zrB);
+            stage_step(C0{}, b0, NZ == 3 ? b0 : (int)((it_first + 1) & 1), xrA, yrA, zrA, 0, false);
+            load_step(C0{}, it_first + 2, xrA, yrA, zrA);
+            stage_step(C0{}, b1, NZ == 3 ? b1 : (int)(it_first & 1), xrB, yrB, zrB, 0, false);
+            load_step(C0{}, it_first + 3, xrB, yrB, zrB);
         } else {
-            load_step(C0{}, it0, xrA, yrA, zrA);
-            load_step(C1{}, it0, xrB, yrB, zrB);
-            stage_step(C0{}, b0, (int)(it0 & 1), xrA, yrA, zrA, 0, false);
-            load_step(C0{}, it0 + 1, xrA, yrA, zrA);
+            stage_step(C0{}, b0, (int)(it_first & 1), xrA, yrA, zrA, 0, false);
+            load_step(C0{}, it_first + 1, xrA, yrA, zrA);
             stage_step(C1{}, b1, 0, xrB, yrB, zrB, 0, false);
-            load_step(C1{}, it0 + 1, xrB, yrB, zrB);
+            load_step(C1{}, it_first + 1, xrB, yrB, zrB);
         }
         __syncthreads();
-        if (it0 >= it_first && it0 < it_end) score_step(C0{}, b0, (int)(it0 & 1));
+        if (it_first < it_end) score_step(C0{}, b0, (int)(it_first & 1));
         __syncthreads();
+    };
+
+    // Warm-up blocks, [it0, it_first): the state update alone, in a walk of its own.  A step is a whole block whatever NF
+    // is: its y tile goes where a step's x and y tiles go later (buffer by parity, the second half of the features in the
+    // y tile's place), its z slice into a z slot.  The loader waves have nothing to fetch, compute or write back but these two,
+    // and keep WD blocks in flight beside the one in LDS.  A block costs a third of a full one (half of one when these blocks went
+    // through the steps of the main walk, with empty x tiles, two barriers a block for NF = 2 and the output slots read for nothing):
+    // la_fwd, us, d128 b1 h8 n2048 32.5 -> 23.5, d192 b2 h12 n2048 49.3 -> 38.1, d256 b1 h8 n1024 28.6 -> 23.4, fp16 b6 h8 n1213 d128 e64 22.8 ->
+    // 19.8; the collect launch of b4 h16 n4096 d128 28 -> 25.
+    constexpr int WD = NF == 1 ? 3 : 2;
+    constexpr int YC = NF * XC;  // 16-byte chunks of a y block per loader thread
+    auto warm_load = [&]() __attribute__((always_inline)) {
+        unsigned oy[ROWAL ? NF : YC], oz[ZAL ? 1 : ZC];
+#pragma unroll
+        for (int hf = 0; hf < NF; ++hf)
+#pragma unroll
+            for (int u = 0; u < (ROWAL ? 1 : XC); ++u) {
+                const int c = tid + NL * u, row = c / CPX, col = hf * DKH + (c % CPX) * 8;
+                oy[ROWAL ? hf : hf * XC + u] = col < dk ? (row * yts + col) * (unsigned)sizeof(T) : kOob;
+            }
+#pragma unroll
+        for (int u = 0; u < (ZAL ? 1 : ZC); ++u) oz[u] = z_col(u) < colend ? (z_row(u) * zts + z_col(u)) * (unsigned)sizeof(T) : kOob;
+        u32x4 wy[WD][YC], wz[WD][ZC];
+        // (rows >= n lie beyond the buffer, whose last row is n - 1; the additions saturate, so that what is out of range stays so.
+        // Streamed as in the main walk: with y streamed as well a collect launch takes the next one's hits in the last-level cache,
+        // forward of b1 h16 n32768 d128 131.8 -> 147.7 us; all cached 418 -> 425 for forward + backward.)
+        auto fetch = [&](auto set, int64_t b) __attribute__((always_inline)) {
+            constexpr int S = decltype(set)::value;
+            const int64_t t = REVERSE ? nblk - 1 - b : b;
+            const unsigned ty = b < it_first ? (unsigned)(t * 64) * yts * (unsigned)sizeof(T) : kOob;
+            const unsigned tz = b < it_first ? (unsigned)(t * 64) * zts * (unsigned)sizeof(T) : kOob;
+#pragma unroll
+            for (int u = 0; u < YC; ++u) {
+                const unsigned lane = ROWAL ? oy[u / XC] : oy[u], down = ROWAL ? (u % XC) * CROWS * yts * (unsigned)sizeof(T) : 0u;
+                wy[S][u] = buf_load16p<kCached>(yb, __builtin_elementwise_add_sat(lane, ty + down));
+            }
+#pragma unroll
+            for (int u = 0; u < ZC; ++u) {
+                const unsigned lane = ZAL ? oz[0] : oz[u], down = ZAL ? u * ZROWS * zts * (unsigned)sizeof(T) : 0u;
+                wz[S][u] = buf_load16p<PZ>(zb, __builtin_elementwise_add_sat(lane, tz + down));
+            }
+        };
+        auto put = [&](auto set, int64_t b) __attribute__((always_inline)) {
+            constexpr int S = decltype(set)::value;
+            const unsigned yd = opaque((unsigned)(b & 1) * XYB + (ROWAL ? lane_stage_xy : 0u));
+            const unsigned zd = opaque(ZBASE + (unsigned)(b & 1) * ZTB + (ZAL ? lane_stage_z : 0u));
+#pragma unroll
+            for (int u = 0; u < YC; ++u) {
+                const int c = tid + NL * (u % XC);
+                const unsigned so = ROWAL ? (unsigned)((u % XC) * CROWS * XS) * E : (unsigned)((c / CPX) * XS + (c % CPX) * 8) * E;
+                *reinterpret_cast<u32x4*>(smem + yd + (u / XC) * YOFF + so) = SILU ? silu16(wy[S][u]) : wy[S][u];
+            }
+#pragma unroll
+            for (int u = 0; u < ZC; ++u)
+                *reinterpret_cast<u32x4*>(smem + zd + (ZAL ? (unsigned)(u * ZROWS * ZS) * E : z_lds(u))) = SILU ? silu16(wz[S][u]) : wz[S][u];
+        };
+        typedef std::integral_constant<int, 1> S1;
+        typedef std::integral_constant<int, WD - 1> SL;
+        fetch(C0{}, it0);
+        fetch(S1{}, it0 + 1);
+        if constexpr (WD == 3) fetch(SL{}, it0 + 2);
+        put(C0{}, it0);
+        fetch(C0{}, it0 + WD);
+        __syncthreads();
+        // (left by breaks: no joins of paths with different loads in flight)
+        for (int64_t b = it0;;) {
+            put(S1{}, b + 1);
+            fetch(S1{}, b + 1 + WD);
+            __syncthreads();
+            if (++b >= it_first) break;
+            if constexpr (WD == 3) {
+                put(SL{}, b + 1);
+                fetch(SL{}, b + 1 + WD);
+                __syncthreads();
+                if (++b >= it_first) break;
+            }
+            put(C0{}, b + 1);
+            fetch(C0{}, b + 1 + WD);
+            __syncthreads();
+            if (++b >= it_first) break;
+        }
+    };
+    auto warm_fold = [&]() __attribute__((always_inline)) {
+        __syncthreads();
+        for (int64_t b = it0; b < it_first; ++b) {
+            if (cols_active) {
+                const unsigned yq = opaque((unsigned)(b & 1) * XYB + lane_yt);
+                const unsigned zq = opaque(ZBASE + (unsigned)(b & 1) * ZTB + lane_zt);
+                V8 zf[NH][2];
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks)
+                        zf[h][ks] = cat<V8, V4>(ldt(zq + (32 * ks * ZS + 16 * h) * E), ldt(zq + ((32 * ks + 4) * ZS + 16 * h) * E));
+                constexpr int UB = NH * KT > 16 ? 2 : KTH % 4 ? 3 : 4;  // transposed y reads ahead of their use, by the registers left
+                static_assert(KTH % UB == 0, "batches of state tiles");
+                V8 ay[2][UB][2];
+                auto read_y = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int kt = 0; kt < UB; ++kt)
+#pragma unroll
+                        for (int ks = 0; ks < 2; ++ks) {
+                            const int t = t0 + kt;
+                            const unsigned py = yq + (t / KTH) * YOFF + (32 * ks * XS + 16 * (t % KTH)) * E;
+                            ay[t0 / UB % 2][kt][ks] = cat<V8, V4>(ldt(py), ldt(py + 4 * XS * E));
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                read_y(0);
+                if (DECAY) {
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks) {
+                        f32x4 c0, c1;
+                        if constexpr (NH > 2) {
+                            const unsigned ca = opaque(CFBASE + (16 * g + 8 * ks) * 4);
+                            c0 = *reinterpret_cast<const f32x4*>(smem + ca);
+                            c1 = *reinterpret_cast<const f32x4*>(smem + ca + 16);
+                        }
+#pragma unroll
+                        for (int h = 0; h < NH; ++h)
+#pragma unroll
+                            for (int u = 0; u < 8; ++u)
+                                zf[h][ks][u] = (T)((float)zf[h][ks][u] * (NH > 2 ? (u < 4 ? c0[u] : c1[u - 4]) : cf[4 + 8 * ks + u]));
+                    }
+                }
+#pragma unroll
+                for (int t0 = 0; t0 < KT; t0 += UB) {
+                    if (t0 + UB < KT) read_y(t0 + UB);
+                    if (DECAY) {
+#pragma unroll
+                        for (int kt = 0; kt < UB; ++kt)
+#pragma unroll
+                            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                                for (int v = 0; v < 4; ++v) st[h][t0 + kt][v] *= lamB;
+                    }
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                        for (int kt = 0; kt < UB; ++kt)
+#pragma unroll
+                            for (int h = 0; h < NH; ++h) st[h][t0 + kt] = M::mma(ay[t0 / UB % 2][kt][ks], zf[h][ks], st[h][t0 + kt]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __syncthreads();
+        }
     };
     // the state a workgroup starts from: zero, or what the scan (kApply) or the pass before (kResume) left
     auto init_state = [&]() __attribute__((always_inline)) {
@@ -901,18 +1048,31 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
                 for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(dst + (size_t)(h * KT + kt) * 256) = st[h][kt];
         }
     };
+    const bool warm_up = it0 < it_first, produces = it_first < it_end;  // (uniform over the workgroup, as the barriers need)
     if (!state_role) {
-        prologue();
-        walk(std::integral_constant<int, 0>{});
-        flush_last();
+        constexpr bool EARLY = NH < 3 || DENSE;  // (three slabs and strides of their own: no registers for these beside the warm-up's)
+        if (EARLY) first_loads();
+        if (warm_up) warm_load();
+        if (produces) {
+            if (!EARLY) first_loads();
+            prologue();
+            walk(std::integral_constant<int, 0>{});
+            flush_last();
+        }
     } else {
-        __syncthreads();
-        __syncthreads();
         // The state waves are the critical path and every SIMD holds one wave of each kind: when both
         // have an instruction ready (right after the barrier all eight waves go for LDS), theirs goes first.
         __builtin_amdgcn_s_setprio(1);
-        init_state();
-        walk(std::integral_constant<int, 1>{});
+        if (warm_up) {
+            init_state();
+            warm_fold();
+        }
+        if (produces) {
+            __syncthreads();
+            __syncthreads();
+            if (!warm_up) init_state();
+            walk(std::integral_constant<int, 1>{});
+        }
         leave_state();
     }
 }
