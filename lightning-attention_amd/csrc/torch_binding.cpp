@@ -11,9 +11,10 @@
 //   lightning_attn_hip::attn(q, k, v, s?, chunks, scan, wide, paired, once, save_states) -> o
 //       lightning_attn2 / lightning_attn2_no_decay (lightning_attn/ops/triton/lightning_attn2.py:398-507,
 //       lightning_attn2_no_decay.py:367-471)
+//   lightning_attn_hip::attn_auto(q, k, v, s?) -> o, or nothing where the arguments need Python's conversions
 //   lightning_attn_hip::srmsnorm(x, eps) -> y
 //       _SrmsNorm (lightning_attn/ops/triton/srmsnorm.py:76-175)
-//   lightning_attn_hip::attn_silu(q, k, v, s?, chunks, scan, wide, paired, once) -> o      (no backward pass)
+//   lightning_attn_hip::attn_silu(q, k, v, s?, chunks, scan, wide, paired, once) -> o      (no backward pass), attn_silu_auto likewise
 //   lightning_attn_hip::norm_gate(o, g, weight, bias, eps) -> y
 //       the attention block's activation and gated output norm (examples/module/tnl_attn.py:51-54, 66-69)
 #include <ATen/ATen.h>
@@ -123,15 +124,18 @@ struct Attn : public torch::autograd::Function<Attn> {
                           sv_bytes ? saved.data_ptr<float>() : nullptr, sv_bytes, stream_of(q)),
               "la_fwd");
         ctx->save_for_backward({q, k, v, s, saved});
-        ctx->saved_data["opts"] = std::vector<int64_t>{chunks, scan, wide, paired, once};
+        if (op.given) ctx->saved_data["opts"] = std::vector<int64_t>{chunks, scan, wide, paired, once};
         return o;
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto sv = ctx->get_saved_variables();
         const Tensor &q = sv[0], &k = sv[1], &v = sv[2], &s = sv[3], &saved = sv[4];
-        const auto ov = ctx->saved_data["opts"].toIntVector();
-        const Opts op = make_opts(ov[0], ov[1], ov[2], ov[3], ov[4], true);
+        Opts op = make_opts(0, 0, 0, 0, 0, true);
+        if (const auto it = ctx->saved_data.find("opts"); it != ctx->saved_data.end()) {
+            const auto ov = it->second.toIntVector();
+            op = make_opts(ov[0], ov[1], ov[2], ov[3], ov[4], true);
+        }
         const la_launch_opts* lo = op.given ? &op.o : nullptr;
         const int64_t b = q.size(0), h = q.size(1), n = q.size(2), d = q.size(3), e = v.size(3);
         Tensor dout = grads[0];
@@ -172,31 +176,65 @@ Tensor attn(const Tensor& q, const Tensor& k, const Tensor& v, const c10::option
     return Attn::apply(q, k, v, s, chunks, scan, wide, paired, once, save_states && for_backward);
 }
 
+// `x` as dense rows: itself where it is contiguous (no view of it is made: 0.8 us each), else a copy.
+struct Rows {
+    Tensor t;
+    int64_t rows, cols;
+    explicit Rows(const Tensor& x) {
+        if (x.dim() > 0 && x.numel() > 0 && x.is_contiguous()) {
+            t = x;
+            cols = x.size(-1);
+            rows = x.numel() / cols;
+            return;
+        }
+        t = x.reshape({-1, x.size(-1)}).contiguous();
+        rows = t.size(0);
+        cols = t.size(1);
+    }
+};
+
+// Arguments the operators above take as they are; for anything else attn_auto and attn_silu_auto give nothing back, and the Python
+// operators convert, split or refuse.  Asked in Python, one property at a time, the same questions cost 2.5 us a call.
+bool as_they_are(const Tensor& q, const Tensor& k, const Tensor& v, const c10::optional<Tensor>& s) {
+    const auto t = q.scalar_type();
+    if (!q.is_cuda() || (t != at::kBFloat16 && t != at::kHalf && t != at::kFloat) || k.scalar_type() != t || v.scalar_type() != t) return false;
+    if (q.dim() != 4 || v.dim() != 4 || k.device() != q.device() || v.device() != q.device() || k.sizes() != q.sizes()) return false;
+    if (v.sizes().slice(0, 3) != q.sizes().slice(0, 3)) return false;
+    const int64_t d = q.size(3), e = v.size(3), widest = t == at::kFloat ? 128 : 256;
+    if (d <= 0 || e <= 0 || d % 8 || e % 8 || d > widest || e > widest) return false;
+    return !s.has_value() || !s->defined() || s->numel() == q.size(1);
+}
+
+c10::optional<Tensor> attn_auto(const Tensor& q, const Tensor& k, const Tensor& v, const c10::optional<Tensor>& s) {
+    if (!as_they_are(q, k, v, s)) return c10::nullopt;
+    return attn(q, k, v, s, 0, 0, 0, 0, 0, true);
+}
+
 struct SrmsNorm : public torch::autograd::Function<SrmsNorm> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, double eps) {
         // eps too small for fp16 (srmsnorm.py:80-81)
         if (x.scalar_type() == at::kHalf && eps < 1.6e-5) eps = 1.6e-5;
-        Tensor x2 = x.reshape({-1, x.size(-1)});
-        if (!x2.is_contiguous()) x2 = x2.contiguous();
-        const int64_t rows = x2.size(0), cols = x2.size(1);
+        const Rows r(x);
+        const Tensor& x2 = r.t;
+        const int64_t rows = r.rows, cols = r.cols;
         // same bound as the reference: one row may not exceed 64 KB (srmsnorm.py:94-97)
         TORCH_CHECK(cols <= 65536 / (int64_t)x.element_size(), "This layer norm doesn't support feature dim >= 64KB.");
-        Tensor y = at::empty_like(x2);
+        Tensor y = at::empty(x.sizes(), x.options().memory_format(at::MemoryFormat::Contiguous));
         Tensor rstd = at::empty({rows}, x.options().dtype(at::kFloat));
         const c10::DeviceGuard guard(x.device());
-        check(srmsnorm_fwd(x2.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), rows, cols, rows > 1 ? x2.stride(0) : cols,
+        check(srmsnorm_fwd(x2.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), rows, cols, cols,
                            (float)eps, dtype_code(x.scalar_type()), stream_of(x)),
               "srmsnorm_fwd");
         ctx->save_for_backward({x, rstd});
-        return y.reshape(x.sizes());
+        return y;
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto sv = ctx->get_saved_variables();
         const Tensor &x = sv[0], &rstd = sv[1];
-        Tensor x2 = x.reshape({-1, x.size(-1)});
-        if (!x2.is_contiguous()) x2 = x2.contiguous();
-        const int64_t rows = x2.size(0), cols = x2.size(1);
+        const Rows r(x);
+        const Tensor& x2 = r.t;
+        const int64_t rows = r.rows, cols = r.cols;
         Tensor dy = grads[0];
         TORCH_CHECK(dy.defined() && dy.device() == x.device(), "SimpleRMSNorm backward: the upstream gradient is not on ", x.device());
         dy = dy.contiguous();
@@ -205,10 +243,10 @@ struct SrmsNorm : public torch::autograd::Function<SrmsNorm> {
                     "Something is wrong in the backward graph, possibly because of an inplace operation after the layernorm");
         Tensor dx = at::empty_like(dy);
         const c10::DeviceGuard guard(x.device());
-        check(srmsnorm_bwd(x2.data_ptr(), dy.data_ptr(), rstd.data_ptr<float>(), dx.data_ptr(), rows, cols,
-                           rows > 1 ? x2.stride(0) : cols, dtype_code(x.scalar_type()), stream_of(x)),
+        check(srmsnorm_bwd(x2.data_ptr(), dy.data_ptr(), rstd.data_ptr<float>(), dx.data_ptr(), rows, cols, cols,
+                           dtype_code(x.scalar_type()), stream_of(x)),
               "srmsnorm_bwd");
-        return {dx.reshape(dy.sizes()), Tensor()};
+        return {dx, Tensor()};
     }
 };
 
@@ -246,6 +284,14 @@ Tensor attn_silu(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, con
                       dense ? nullptr : strides, b, h, n, d, e, code, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, lo, stream_of(q)),
           "la_fwd_silu");
     return o;
+}
+
+// The same where no gradient is wanted and the fused kernel takes the arguments as they are, else nothing.
+c10::optional<Tensor> attn_silu_auto(const Tensor& q, const Tensor& k, const Tensor& v, const c10::optional<Tensor>& s) {
+    if (q.scalar_type() == at::kFloat || !as_they_are(q, k, v, s)) return c10::nullopt;
+    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return c10::nullopt;
+    if (!la_fwd_silu_supported(q.size(3), v.size(3), dtype_code(q.scalar_type()))) return c10::nullopt;
+    return attn_silu(q, k, v, s, 0, 0, 0, 0, 0);
 }
 
 // row-major and 16-byte aligned (a dense view into a larger buffer may start off that grid)
@@ -303,6 +349,8 @@ Tensor norm_gate(const Tensor& o, const Tensor& g, const Tensor& weight, const T
 
 TORCH_LIBRARY(lightning_attn_hip, m) {
     m.def("attn", &attn);
+    m.def("attn_auto", &attn_auto);
+    m.def("attn_silu_auto", &attn_silu_auto);
     m.def("srmsnorm", &srmsnorm);
     m.def("attn_silu", &attn_silu);
     m.def("norm_gate", &norm_gate);

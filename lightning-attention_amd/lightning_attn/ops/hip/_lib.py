@@ -168,11 +168,18 @@ def native_ops():
                         lib()  # the kernel library first: the binding links against it
                         torch.ops.load_library(TORCH_LIB_PATH)
                         ops = torch.ops.lightning_attn_hip
-                        ops.attn, ops.srmsnorm, ops.attn_silu, ops.norm_gate  # resolve now
+                        ops.attn, ops.attn_auto, ops.srmsnorm, ops.attn_silu, ops.attn_silu_auto, ops.norm_gate  # resolve now
                     except (OSError, RuntimeError, AttributeError):
                         ops = False
                 _native = ops
     return _native or None
+
+
+def plain_ops():
+    """native_ops() for a call under the library's own choices: None where launch options are in force on this thread."""
+    if _native and _native_enabled and getattr(_tls, "opts", None) is None:
+        return _native
+    return None if getattr(_tls, "opts", None) is not None else native_ops()
 
 
 def use_native_ops(on):

@@ -8,6 +8,7 @@ dims are split into slices of q/k whose partial outputs add up (the scores are
 additive over feature slices) and into column groups of v."""
 import torch
 
+from .hip import _lib
 from .hip.lightning_attn2 import lightning_attn2, lightning_attn2_no_decay, lightning_attn_silu, silu_fused_ok
 
 _VARIANTS = ("chunk_loop", "parallel")
@@ -27,6 +28,10 @@ def _pad8(t):
     return torch.nn.functional.pad(t, (0, extra)) if extra else t
 
 
+def _tensors(q, k, v, s, T=torch.Tensor):
+    return isinstance(q, T) and isinstance(k, T) and isinstance(v, T) and (s is None or isinstance(s, T))
+
+
 def lightning_attn_func(q, k, v, s=None, variant="chunk_loop"):
     """o = (q k^T * M) v with M[i,j] = exp(-s_h (i-j)) [i >= j]; s=None means no decay.
 
@@ -35,6 +40,12 @@ def lightning_attn_func(q, k, v, s=None, variant="chunk_loop"):
     q, k, v."""
     if variant not in _VARIANTS:
         raise ValueError("variant must be one of %s, got %r" % (_VARIANTS, variant))
+    if _tensors(q, k, v, s):
+        # the whole of the common case behind one call; None: the arguments need what follows
+        ops = _lib.plain_ops()
+        o = ops.attn_auto(q, k, v, s) if ops is not None else None
+        if o is not None:
+            return o
     b, h, n, d = q.shape
     e = v.shape[-1]
     assert is_support(d) and is_support(e), "feature dims must be positive (got d=%d, e=%d)" % (d, e)
@@ -68,6 +79,11 @@ def lightning_attn_silu_func(q, k, v, s=None, variant="chunk_loop"):
     three activation passes disappear; otherwise this is the three PyTorch calls followed by lightning_attn_func."""
     if variant not in _VARIANTS:
         raise ValueError("variant must be one of %s, got %r" % (_VARIANTS, variant))
+    if _tensors(q, k, v, s):
+        ops = _lib.plain_ops()
+        o = ops.attn_silu_auto(q, k, v, s) if ops is not None else None
+        if o is not None:
+            return o
     d, e = q.shape[-1], v.shape[-1]
     if d % 8 == 0 and e % 8 == 0 and silu_fused_ok(q, k, v):
         return lightning_attn_silu(q, k, v, s)
