@@ -15,7 +15,8 @@
 //
 // What bounds it: the fp32 matrix instruction (32 cycles each, 256 FLOP per cycle and CU).  A block of feature dim 64 and 64
 // columns costs the busiest of four wavefronts 48 of them for its score tiles, 64 + 40 for the output and 64 for the state: 2.9 us
-// at 2.4 GHz, measured 4.2 with one workgroup on a CU and 2.55 each with two.  Feature dim 128 leaves room in LDS for one
+// at 2.4 GHz, measured 4.2 with half of the CUs at work, 5.1 with a workgroup on each and 8.9 for two on each (98 of the 154 TFLOP/s that
+// a large product reaches: forward of 512 sequences, n1536, 215 us).  Feature dim 128 leaves room in LDS for one
 // workgroup only: there two wavefronts share a slab of columns, each with half of the features, so that a SIMD has a second
 // one to issue from (b4 h32 n2048: forward 264 -> 236 us, backward 767 -> 692).  Few sequences: 32 columns to a workgroup, the
 // halves of the features on a wavefront each (a block 3.05 us, 5.15 at feature dim 128), and the walk cut into chunks whose
