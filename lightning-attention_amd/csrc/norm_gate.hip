@@ -285,7 +285,9 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
         }
     }
     // column sums of this workgroup: the thread groups of its rows hold the same columns and are
-    // added up in a fixed order first, those of a wavefront by shuffles
+    // added up in a fixed order first, those of a wavefront by shuffles (after which its first TPR lanes, `owner`, speak for it)
+    const bool owner = TPR >= 64 || (threadIdx.x & 63) < TPR;
+    const int grp = threadIdx.x / (TPR < 64 ? 64 : TPR);
     if (TPR < 64) {
 #pragma unroll
         for (int u = 0; u < NV; ++u)
@@ -296,14 +298,9 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
                     aw[u][t] += __shfl_xor(aw[u][t], m, 64);
                     ab[u][t] += __shfl_xor(ab[u][t], m, 64);
                 }
-        if ((threadIdx.x & 63) >= TPR) {
-            if (SIDE > 1) __syncthreads();
-            return;
-        }
     }
     if (SIDE > 1) {
-        const int grp = threadIdx.x / (TPR < 64 ? 64 : TPR);
-        if (grp > 0) {
+        if (owner && grp > 0) {
 #pragma unroll
             for (int u = 0; u < NV; ++u)
 #pragma unroll
@@ -312,8 +309,10 @@ __global__ __launch_bounds__(ng_bwd_threads(TPR, sizeof(T), FEW)) void norm_gate
                     comb[((((grp - 1) * NV + u) * E + t) * 2 + 1) * TPR + l] = ab[u][t];
                 }
         }
-        __syncthreads();
-        if (grp > 0) return;
+        __syncthreads();  // (every thread of the workgroup comes by here)
+    }
+    if (!owner || grp > 0) return;
+    if (SIDE > 1) {
 #pragma unroll
         for (int k = 0; k < SIDE - 1; ++k)
 #pragma unroll
