@@ -405,7 +405,8 @@ static void ng_shape(int64_t rows, int64_t chunks, bool backward, int* tpr, int*
     }
 }
 
-// backward, 16-bit rows of up to 1024 elements: at most one group of rows of a 256-thread workgroup per CU
+// backward, 16-bit rows of up to 1024 elements: at most one group of rows of a 256-thread workgroup per CU (with 16 or 32 threads to
+// a row, that is 16 or 8 rows per CU, never: ng_shape gives rows so few a wavefront each)
 static bool ng_few(int64_t rows, int tpr, int elt) {
     const int64_t rpg = ng_threads(tpr) / tpr;
     return elt == 2 && tpr <= 128 && (rows + rpg - 1) / rpg <= num_cus();
@@ -438,8 +439,6 @@ static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
         constexpr bool kFew = sizeof(T) == 2;                         \
         const bool few = ng_few(rows, tpr, sizeof(T));                \
         if (tpr == 8 && few) LA_NG_BWD(8, kFew, __VA_ARGS__);         \
-        else if (tpr == 16 && few) LA_NG_BWD(16, kFew, __VA_ARGS__);  \
-        else if (tpr == 32 && few) LA_NG_BWD(32, kFew, __VA_ARGS__);  \
         else if (tpr == 64 && few) LA_NG_BWD(64, kFew, __VA_ARGS__);  \
         else if (tpr == 128 && few) LA_NG_BWD(128, kFew, __VA_ARGS__); \
         else if (tpr == 8) LA_NG_BWD(8, false, __VA_ARGS__);          \

@@ -1,4 +1,4 @@
-"""The built norm_gate backward kernels (disassembled, no GPU) whose rows share a wavefront: they hand their column sums from wavefront to
+"""The built norm_gate backward kernels (disassembled, no GPU).  Those whose rows share a wavefront hand their column sums from wavefront to
 wavefront behind ONE barrier that every thread comes by.  A second one in the code means a barrier inside a branch on the lane, which
 the language leaves undefined."""
 import os
@@ -46,3 +46,10 @@ def test_one_barrier_where_rows_share_a_wavefront(kernels):
     shared = {k: n for k, n in kernels.items() if k[1] < 64}
     assert {k[1] for k in shared} == {8, 16, 32} and len({k[0] for k in shared}) == 3
     assert set(shared.values()) == {1}, shared
+
+
+def test_no_kernel_that_no_launch_takes(kernels):
+    """Workgroups of 256 threads for few rows: at most 16 (8) rows per CU where 16 (32) threads share a row - but rows are shared out
+    like that beyond 16 per CU only."""
+    assert not [k for k in kernels if k[2] and k[1] in (16, 32)]
+    assert {k[1] for k in kernels if k[2]} == {8, 64, 128}
