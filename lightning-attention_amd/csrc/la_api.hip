@@ -33,7 +33,7 @@ double kept_us(int64_t n, int64_t e, const SavedPlan& pl);
 int prepare_srmsnorm();   // srmsnorm.hip
 int prepare_norm_gate();  // norm_gate.hip
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
-              int64_t n, int64_t dk, int64_t dv, bool reverse, int chunks, hipStream_t st);
+              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, int chunks, hipStream_t st);
 int sweep_f32_bwd_once(const void* q, const void* k, const void* v, const void* dout, void* dq, void* dk, void* dv,
                        const float* s, int64_t bh, int64_t h, int64_t n, int64_t d, int chunks, hipStream_t st);
 
@@ -65,7 +65,7 @@ static int run(const Tensor& x, const Tensor& y, const Tensor& z, const Tensor& 
         // the float32 accuracy kernel takes plain (b, h, n, d) tensors only
         if (!is_dense(x, h, n, dk) || !is_dense(y, h, n, dk) || !is_dense(z, h, n, dv) || !is_dense(out, h, n, dv))
             return LA_E_UNSUPPORTED;
-        return sweep_f32(x.p, y.p, z.p, const_cast<void*>(out.p), s, bh, h, n, dk, dv, reverse, opts.chunks, st);
+        return sweep_f32(x.p, y.p, z.p, const_cast<void*>(out.p), s, bh, h, n, dk, dv, reverse, 1, opts.chunks, st);
     }
     return sweep(io(x, y, z, out), s, bh, h, n, dk, dv, dtype, reverse, ws.p, ws.bytes, opts, st);
 }
@@ -152,12 +152,17 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
         if ((rc = check_tensor(*ts[i], b, h, n, cols[i], dtype)) != LA_OK) return rc;
     // dQ_i = sum_{j<=i} lam^(i-j) (dO_i . v_j) k_j
     // (the launches follow each other on one stream, so they can all use the same scratch memory)
-    if (d == e && dtype == LA_FP32 && opts.paired != LA_OPT_OFF) {
-        // float32: the three sweeps always share a launch (plain tensors only, as in run())
+    if (d == e && dtype == LA_FP32) {
+        // float32: the three sweeps share a launch (plain tensors only, as in run()), or follow each other in workgroups of the form
+        // that launch would take - the forms sum in different orders, and opts.paired is not to change a bit
         for (int i = 0; i < 7; ++i)
             if (!is_dense(*ts[i], h, n, d)) return LA_E_UNSUPPORTED;
-        return sweep_f32_bwd_once(q.p, k.p, v.p, dout.p, const_cast<void*>(dq.p), const_cast<void*>(dk.p),
-                                  const_cast<void*>(dv.p), s, b * h, h, n, d, opts.chunks, st);
+        void *const pdq = const_cast<void*>(dq.p), *const pdk = const_cast<void*>(dk.p), *const pdv = const_cast<void*>(dv.p);
+        if (opts.paired != LA_OPT_OFF) return sweep_f32_bwd_once(q.p, k.p, v.p, dout.p, pdq, pdk, pdv, s, b * h, h, n, d, opts.chunks, st);
+        rc = sweep_f32(dout.p, v.p, k.p, pdq, s, b * h, h, n, d, d, false, 3, opts.chunks, st);
+        if (rc == LA_OK) rc = sweep_f32(v.p, dout.p, q.p, pdk, s, b * h, h, n, d, d, true, 3, opts.chunks, st);
+        if (rc == LA_OK) rc = sweep_f32(k.p, q.p, dout.p, pdv, s, b * h, h, n, d, d, true, 3, opts.chunks, st);
+        return rc;
     }
     const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : kNoPlan;
     const SavedPlan cp = sv.p && sv.carry && pl.nchunk <= 1 ? plan_carry(b * h, n, d, e, dtype, opts) : kNoPlan;

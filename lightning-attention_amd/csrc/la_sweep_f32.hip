@@ -580,10 +580,11 @@ static int f32_columns(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod)
     return f32_walk_us(narrow, nblk, dk <= 64 ? 3.05 : 5.15) < 1.03 * f32_walk_us(wide, nblk, dk <= 64 ? 4.2 : 6.9) ? 32 : 64;
 }
 
+// `nform`: how many such sweeps the form of the workgroups is chosen for (3: those of a backward pass with d == e, launched apart).
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
-              int64_t n, int64_t dk, int64_t dv, bool reverse, int chunks, hipStream_t st) {
+              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, int chunks, hipStream_t st) {
     if (dk > 128) return LA_E_UNSUPPORTED;
-    const int cols = f32_columns(bh, n, dk, dv, 1);
+    const int cols = f32_columns(bh, n, dk, dv, nform);
     SweepArgsF32 a = make_args_f32(x, y, z, out, s, bh, h, n, dk, dv, cols);
     plan_warm_up_chunks(num_cus(), (bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
 #define LA_GD(DKP, WC, KH, R) (s ? launch_one_f32<DKP, WC, KH, R, true>(a, st) : launch_one_f32<DKP, WC, KH, R, false>(a, st))

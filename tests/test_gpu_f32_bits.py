@@ -1,0 +1,38 @@
+"""float32 sweep where the number of sweeps in a launch decides between forms of a workgroup that sum in different orders (64 columns, one
+wavefront to a slab, and 32 columns, two): the launch options still change no bit of a result."""
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+from lightning_attn.ops import lightning_attn_func  # noqa: E402
+from lightning_attn.ops.hip import _lib  # noqa: E402
+
+
+def _inputs(h, n, d):
+    g = torch.Generator().manual_seed(100 * h + n + d)
+    q, k = (torch.randn(1, h, n, d, generator=g) * d ** -0.5 for _ in range(2))
+    v, do = (torch.randn(1, h, n, d, generator=g) for _ in range(2))
+    return q, k, v, torch.logspace(-2, 0, h), do
+
+
+def _pass(q, k, v, s, do, decay=True, **opts):
+    with _lib.launch_opts(**opts):
+        ts = [t.cuda().requires_grad_() for t in (q, k, v)]
+        o = lightning_attn_func(*ts, s.cuda() if decay else None)
+        return (o.detach(),) + torch.autograd.grad(o, ts, do.cuda())
+
+
+# (all with 32 columns in a sweep alone; 8 sequences, and feature dims above 64 to which both forms give the same sums, for comparison)
+@pytest.mark.parametrize("h,n,d", [(16, 1024, 64), (24, 700, 40), (9, 300, 64), (40, 513, 56), (8, 1024, 64), (4, 2048, 128)])
+@pytest.mark.parametrize("decay", [True, False])
+def test_gradients_of_separate_launches_are_the_joint_launchs(h, n, d, decay):
+    args = _inputs(h, n, d)
+    together, apart = _pass(*args, decay=decay), _pass(*args, decay=decay, paired=False)
+    for a, c in zip(together, apart):
+        assert torch.equal(a, c)
+    want = oracle.linear_attn_fwd_bwd(args[0], args[1], args[2], args[3] if decay else None, args[4], torch.float64)
+    for w, x in zip(want, together):  # (float32 accumulation over at most 2048 + 128 terms)
+        assert (x.cpu().double() - w).abs().max() <= 1e-5 * w.abs().max()
