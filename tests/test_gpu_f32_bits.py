@@ -25,8 +25,8 @@ def _pass(q, k, v, s, do, decay=True, **opts):
         return (o.detach(),) + torch.autograd.grad(o, ts, do.cuda())
 
 
-# (all with 32 columns in a sweep alone; 8 sequences, and feature dims above 64 to which both forms give the same sums, for comparison)
-@pytest.mark.parametrize("h,n,d", [(16, 1024, 64), (24, 700, 40), (9, 300, 64), (40, 513, 56), (8, 1024, 64), (4, 2048, 128)])
+# (32 columns in a sweep alone, 64 in three together; but 8 sequences, 32 in either, and d = 128, whose two forms give the same sums)
+@pytest.mark.parametrize("h,n,d", [(16, 1024, 64), (24, 700, 40), (9, 700, 64), (40, 513, 56), (8, 1024, 64), (4, 2048, 128)])
 @pytest.mark.parametrize("decay", [True, False])
 def test_gradients_of_separate_launches_are_the_joint_launchs(h, n, d, decay):
     args = _inputs(h, n, d)
@@ -35,4 +35,21 @@ def test_gradients_of_separate_launches_are_the_joint_launchs(h, n, d, decay):
         assert torch.equal(a, c)
     want = oracle.linear_attn_fwd_bwd(args[0], args[1], args[2], args[3] if decay else None, args[4], torch.float64)
     for w, x in zip(want, together):  # (float32 accumulation over at most 2048 + 128 terms)
+        assert (x.cpu().double() - w).abs().max() <= 1e-5 * w.abs().max()
+
+
+# (64 columns to a workgroup, of 256 CUs: the backward pass of the first six - of 48 sequences because 32 columns give more workgroups than CUs
+# at any length - and the forward pass of the others)
+@pytest.mark.parametrize("h,n,d", [(9, 700, 64), (24, 1085, 64), (24, 700, 40), (48, 65, 64), (48, 128, 40), (48, 192, 64),
+                                   (49, 700, 64), (64, 1085, 40), (136, 257, 64), (136, 320, 40)])
+@pytest.mark.parametrize("decay", [True, False])
+def test_warm_up_of_the_64_column_form(h, n, d, decay):
+    """Chunks behind no, one, an odd and an even number of warm-up blocks, ragged last blocks, against the walk in one piece."""
+    args = _inputs(h, n, d)
+    one = _pass(*args, decay=decay, chunks=1)
+    for chunks in (0, 2, 3, 5, 8):
+        for a, c in zip(one, _pass(*args, decay=decay, chunks=chunks)):
+            assert torch.equal(a, c), chunks
+    want = oracle.linear_attn_fwd_bwd(args[0], args[1], args[2], args[3] if decay else None, args[4], torch.float64)
+    for w, x in zip(want, one):  # (float32 accumulation over at most 1085 + 128 terms)
         assert (x.cpu().double() - w).abs().max() <= 1e-5 * w.abs().max()
