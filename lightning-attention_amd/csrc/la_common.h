@@ -36,20 +36,17 @@ template <int POLICY>
 __device__ __forceinline__ u32x4 buf_load16p(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0u) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, POLICY);
 }
-// A 16-byte store reads its data registers after the next instruction has issued, so overwriting them at once needs a wait state.  The
-// compiler puts it in where the wave-uniform offset of the instruction is a constant; on gfx950 the store reads them just as
+// A 16-byte store reads its data registers after later instructions have issued, so overwriting them needs two wait states.  The
+// compiler keeps them where the wave-uniform offset of the instruction is a constant; on gfx950 the store reads them just as
 // late when it is a scalar register (seen as address bits in the first four bytes of a lane's 16, in kernels where a v_cndmask into
-// that register came right behind the store; never in kernels without that pair).  So the data stay alive up to a wait
-// of their own behind the store.  (The offset in the per-lane register instead, where the compiler knows the hazard: SiLU forward of token-major
-// b4 h32 n8192 d128 347 -> 359 us, 350 with the wait.)
+// that register came right behind the store; never in kernels without that pair).  So these take no such offset: what is
+// uniform goes into the buffer's base.  SiLU forward of token-major b4 h32 n8192 d128: 339 us; with the offset in a scalar register and a
+// wait behind every store 346, in the per-lane register 359.
 template <int POLICY>
-__device__ __forceinline__ void buf_store16p(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff, u32x4 v) {
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, POLICY);
-    asm volatile("s_nop 1" ::"v"(v));
+__device__ __forceinline__ void buf_store16p(__amdgpu_buffer_rsrc_t r, unsigned off, u32x4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, POLICY);
 }
-__device__ __forceinline__ void buf_store16(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff, u32x4 v) {
-    buf_store16p<kCached>(r, off, soff, v);
-}
+__device__ __forceinline__ void buf_store16(__amdgpu_buffer_rsrc_t r, unsigned off, u32x4 v) { buf_store16p<kCached>(r, off, v); }
 __device__ __forceinline__ void buf_store8(__amdgpu_buffer_rsrc_t r, unsigned off, u32x2 v) {
     __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, 0);
 }

@@ -38,11 +38,18 @@ struct SweepArgs {
     int chunk_start[9];  // first 64-token block (in walk order) of each chunk; chunk_start[nchunk] = number of blocks
 };
 
-// Bounds-checked buffer over the rows of one (batch, head) sequence of a tensor with `cols` features.
+// The rows of one (batch, head) sequence of a tensor with `cols` features: first byte, number of bytes, bounds-checked buffer.
+template <typename T>
+__device__ __forceinline__ const char* seq_base(const void* p, const Layout& l, int unit, int h) {
+    return reinterpret_cast<const char*>(static_cast<const T*>(p) + (int64_t)(unit / h) * l.bs + (int64_t)(unit % h) * l.hs);
+}
+template <typename T>
+__device__ __forceinline__ unsigned seq_bytes(const Layout& l, int64_t n, int cols) {
+    return (unsigned)(((n - 1) * l.ts + cols) * (int64_t)sizeof(T));
+}
 template <typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t seq_rsrc(const void* p, const Layout& l, int unit, int h, int64_t n, int cols) {
-    const T* base = static_cast<const T*>(p) + (int64_t)(unit / h) * l.bs + (int64_t)(unit % h) * l.hs;
-    return make_rsrc(base, (unsigned)(((n - 1) * l.ts + cols) * (int64_t)sizeof(T)));
+    return make_rsrc(seq_base<T>(p, l, unit, h), seq_bytes<T>(l, n, cols));
 }
 
 template <typename T>

@@ -374,7 +374,7 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
             const unsigned ooff = col < dv ? (unsigned)(r * dv + col) * 4u : kOob;
 #pragma unroll
             for (int i = 0; i < 4 / KH; ++i)
-                buf_store16(ob, ooff + (unsigned)(16 * (decltype(first)::value + i) * dv) * 4u, 0u, __builtin_bit_cast(u32x4, o[i]));
+                buf_store16(ob, ooff + (unsigned)(16 * (decltype(first)::value + i) * dv) * 4u, __builtin_bit_cast(u32x4, o[i]));
         };
         if (wave_active) {
 #pragma unroll

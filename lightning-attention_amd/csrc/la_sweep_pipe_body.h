@@ -169,6 +169,8 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const __amdgpu_buffer_rsrc_t yb = seq_rsrc<T>(a.y, a.ly, unit, a.h, n, dk);
     const __amdgpu_buffer_rsrc_t zb = seq_rsrc<T>(a.z, a.lz, unit, a.h, n, dv);
     const __amdgpu_buffer_rsrc_t ob = seq_rsrc<T>(a.out, a.lo, unit, a.h, n, dv);
+    const char* const obase = seq_base<T>(a.out, a.lo, unit, a.h);
+    const unsigned obytes = seq_bytes<T>(a.lo, n, dv);
     const unsigned xts = (unsigned)a.lx.ts, yts = (unsigned)a.ly.ts, zts = (unsigned)a.lz.ts, ots = (unsigned)a.lo.ts;
     const unsigned nrows = (unsigned)n;
     // this workgroup's columns of z / out: [col0, colend); a slice may be narrower than the ZW columns LDS holds
@@ -369,24 +371,23 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     const unsigned lane_o = lane_zcol < colend ? (lane_zrow * ots + lane_zcol) * (unsigned)sizeof(T) : kOob;
     auto store_out = [&](int64_t bout, bool flush, const u32x4 (&o)[ZC]) {
         const int64_t t = REVERSE ? nblk - 1 - bout : bout;
+        if constexpr (DENSE) {
 #pragma unroll
-        for (int u = 0; u < ZC; ++u) {
-            if (DENSE) {
+            for (int u = 0; u < ZC; ++u) {
                 // rows >= n fall outside the buffer and are dropped by the hardware range check
                 const int zc = z_col(u);
                 const unsigned off = zc < colend ? (((unsigned)(t * 64) + z_row(u)) * (unsigned)dv + zc) * (unsigned)sizeof(T) : kOob;
-                buf_store16p<PO>(ob, flush ? off : kOob, 0u, o[u]);
-            } else if constexpr (!ZAL) {
-                const unsigned tok0 = flush ? (unsigned)(t * 64) : 0u;
-                const int rows = flush ? (int)min(64u, nrows - tok0) : 0;
-                const int row = z_row(u), zc = z_col(u);
-                const unsigned oo = zc < colend ? (row * ots + zc) * (unsigned)sizeof(T) : kOob;
-                buf_store16p<PO>(ob, row < rows ? oo : kOob, tok0 * ots * (unsigned)sizeof(T), o[u]);
-            } else {
-                const unsigned tok0 = flush ? (unsigned)(t * 64) : 0u;
-                const int rows = flush ? (int)min(64u, nrows - tok0) : 0;
-                const unsigned tk = u * ZROWS < rows ? tok0 + u * ZROWS : 0u;
-                buf_store16p<PO>(ob, lane_zrow < rows - u * ZROWS ? lane_o : kOob, tk * ots * (unsigned)sizeof(T), o[u]);
+                buf_store16p<PO>(ob, flush ? off : kOob, o[u]);
+            }
+        } else {
+            // the rows from this block's first one on as a buffer of their own (an empty one if nothing is to be written)
+            const unsigned first = flush ? (unsigned)(t * 64) * ots * (unsigned)sizeof(T) : 0u;
+            const __amdgpu_buffer_rsrc_t obt = make_rsrc(obase + first, flush ? obytes - first : 0u);
+#pragma unroll
+            for (int u = 0; u < ZC; ++u) {
+                const int zc = z_col(u);
+                const unsigned off = ZAL ? lane_o + u * ZROWS * ots * (unsigned)sizeof(T) : zc < colend ? (z_row(u) * ots + zc) * (unsigned)sizeof(T) : kOob;
+                buf_store16p<PO>(obt, off, o[u]);
             }
         }
     };
