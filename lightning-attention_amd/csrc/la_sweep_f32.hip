@@ -562,7 +562,10 @@ static const double kWarmCost = 0.27;
 static const int64_t kMinBlocks = 2;
 
 // Columns of z / out per workgroup of a launch of nprod sweeps: 32 in place of 64 where that gives no more workgroups than there
-// are CUs and a single round of them, in the chunks the CUs left over allow, is estimated faster.  Per block 3.05 against
+// are CUs and a single round of them, in the chunks the CUs left over allow, is estimated faster - and for rows of up to 32 columns, where
+// half of a 64-column workgroup's slabs would be idle, on two of a CU's four SIMDs, and there are as many workgroups either way (64 / 32, us:
+// backward of 200 sequences n8192 d24 1685 / 1010, 512 n1000 d24 331 / 247, n113 90 sequences 16.9 / 13.8; forward of 300 n2048 d128 e24
+// 435 / 333, 264 n2048 d8 160 / 127).  Per block 3.05 against
 // 4.2 us (feature dim 64), 5.15 against 6.9 (128); twice the workgroups leave half the chunks.  us of 64 / 32 columns, forward of d64
 // n2048: 8 sequences 44.5 / 35.8, 24 48 / 41, 48 59 / 64, 128 90 / 104; backward 8 63 / 46, 16 63 / 66, 24 76 / 100; d128: 8 forward 74 / 57,
 // 24 94 / 105, backward 8 93 / 104, 16 144 / 173.
@@ -576,6 +579,7 @@ static double f32_walk_us(int64_t wgs, int64_t nblk, double block_us) {
 static int f32_columns(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod) {
     const int64_t nblk = (n + 63) / 64, units = (bh + 7) / 8 * 8 * nprod;
     const int64_t narrow = units * ((dv + 31) / 32), wide = units * ((dv + 63) / 64);
+    if (dv <= 32) return 32;
     if (narrow > num_cus()) return 64;
     return f32_walk_us(narrow, nblk, dk <= 64 ? 3.05 : 5.15) < 1.03 * f32_walk_us(wide, nblk, dk <= 64 ? 4.2 : 6.9) ? 32 : 64;
 }

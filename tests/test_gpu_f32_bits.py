@@ -53,3 +53,16 @@ def test_warm_up_of_the_64_column_form(h, n, d, decay):
     want = oracle.linear_attn_fwd_bwd(args[0], args[1], args[2], args[3] if decay else None, args[4], torch.float64)
     for w, x in zip(want, one):  # (float32 accumulation over at most 1085 + 128 terms)
         assert (x.cpu().double() - w).abs().max() <= 1e-5 * w.abs().max()
+
+
+@pytest.mark.parametrize("h,n,d", [(90, 113, 24), (96, 200, 32), (264, 130, 8), (264, 64, 32)])
+def test_rows_of_up_to_32_columns_in_more_workgroups_than_cus(h, n, d):
+    """32 columns to a workgroup also beyond one round of them: together and apart, in one walk and cut up."""
+    args = _inputs(h, n, d)
+    one = _pass(*args)
+    for opts in ({"paired": False}, {"chunks": 1}, {"chunks": 2}, {"chunks": 3, "paired": False}):
+        for a, c in zip(one, _pass(*args, **opts)):
+            assert torch.equal(a, c), opts
+    want = oracle.linear_attn_fwd_bwd(*args, torch.float64)
+    for w, x in zip(want, one):  # (float32 accumulation over at most 200 + 64 terms)
+        assert (x.cpu().double() - w).abs().max() <= 1e-5 * w.abs().max()
