@@ -169,20 +169,24 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
     const int zrow = tid / (4 * WC), zcol = col0 + (tid % (4 * WC)) * 4;
     const unsigned xoff = lcol < dk ? (unsigned)(lrow * dk + lcol) * 4u : kOob;
     const unsigned zoff = zcol < dv ? (unsigned)(zrow * dv + zcol) * 4u : kOob;
-    auto load_block = [&](int64_t it) {
+    auto block_rsrc = [&](const float* base, int cols, int64_t it) {
         const int64_t tok0 = (REVERSE ? nblk - 1 - it : it) * 64;
-        const unsigned rows = (unsigned)min((int64_t)64, n - tok0);
-        const __amdgpu_buffer_rsrc_t xb = make_rsrc(xg + tok0 * dk, rows * dk * 4u);
-        const __amdgpu_buffer_rsrc_t yb = make_rsrc(yg + tok0 * dk, rows * dk * 4u);
-        const __amdgpu_buffer_rsrc_t zb = make_rsrc(zg + tok0 * dv, rows * dv * 4u);
+        return make_rsrc(base + tok0 * cols, (unsigned)min((int64_t)64, n - tok0) * cols * 4u);
+    };
+    auto load_xy = [&](u32x4 (&to)[XC], const float* base, int64_t it) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t b = block_rsrc(base, dk, it);
 #pragma unroll
-        for (int u = 0; u < XC; ++u) {
-            const unsigned off = xoff + (unsigned)(u * (NT * 4 / DKP) * dk) * 4u;
-            xr[u] = buf_load16(xb, off);
-            yr[u] = buf_load16(yb, off);
-        }
+        for (int u = 0; u < XC; ++u) to[u] = buf_load16(b, xoff + (unsigned)(u * (NT * 4 / DKP) * dk) * 4u);
+    };
+    auto load_z = [&](int64_t it) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t b = block_rsrc(zg, dv, it);
 #pragma unroll
-        for (int u = 0; u < ZN; ++u) zr[u] = buf_load16(zb, zoff + (unsigned)(u * (NT / (4 * WC)) * dv) * 4u);
+        for (int u = 0; u < ZN; ++u) zr[u] = buf_load16(b, zoff + (unsigned)(u * (NT / (4 * WC)) * dv) * 4u);
+    };
+    auto load_block = [&](int64_t it) __attribute__((always_inline)) {
+        load_xy(xr, xg, it);
+        load_xy(yr, yg, it);
+        load_z(it);
     };
     auto stage = [&]() {
 #pragma unroll
@@ -318,7 +322,10 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
 
     for (int64_t it = it_first; it < it_end; ++it) {
         const bool have_next = it + 1 < it_end;
-        if (have_next) load_block(it + 1);
+        // The next block is requested in three parts, spread over this one: all twelve loads at the top hold up the first fragments (us,
+        // together / apart: backward of d64 n2048, 96 sequences, 229 / 224, 24 sequences 74.0 / 72.4; forward of 128 sequences of d64 n2048 92.4 /
+        // 87.4, n8192 378 / 362; d128 n2048, 64 sequences backward 455 / 446).
+        if (have_next) load_xy(xr, xg, it + 1);
 
         // 1. S^T tiles -> masked, decayed P[i][j]
         auto frag = [&](const float* tile, int row16, int kt) { return *reinterpret_cast<const f32x4*>(tile + (16 * row16 + r) * XS + 16 * kt + 4 * g); };
@@ -363,7 +370,9 @@ __device__ __forceinline__ void sweep_f32_body(const SweepArgsF32& a, const unsi
             }
         }
         put_p(0, itA, jt0, s0);
+        if (have_next) load_z(it + 1);
         __syncthreads();
+        if (have_next) load_xy(yr, yg, it + 1);
 
         f32x4 oacc[4];
         // rows 16 i4 .. 16 i4 + 15 of this wave's slab go to memory
