@@ -176,10 +176,11 @@ def native_ops():
 
 
 def plain_ops():
-    """native_ops() for a call under the library's own choices: None where launch options are in force on this thread."""
-    if _native and _native_enabled and getattr(_tls, "opts", None) is None:
-        return _native
-    return None if getattr(_tls, "opts", None) is not None else native_ops()
+    """native_ops() for a call under the library's own choices: None where launch options are in force on this thread, and under
+    torch.jit.trace, which records operators that give back a tensor but refuses one that may give back nothing."""
+    if getattr(_tls, "opts", None) is not None or torch._C._is_tracing():  # (torch.jit.is_tracing: 0.4 us a call)
+        return None
+    return _native if _native and _native_enabled else native_ops()
 
 
 def use_native_ops(on):

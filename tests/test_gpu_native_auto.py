@@ -77,3 +77,18 @@ def test_norm_of_any_number_of_dims(shape, dtype):
                 _lib.use_native_ops(prev)
         for a, b in zip(*got):
             assert a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning", "ignore::DeprecationWarning")
+def test_traced_calls():
+    q, k, v, do = (_t((2, 3, 70, 64), torch.bfloat16) for _ in range(4))
+    s = torch.tensor([0.1, 0.2, 0.5], device="cuda")
+    leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+    traced = torch.jit.trace(lambda q, k, v, s: lightning_attn_func(q, k, v, s), (*leaves, s), check_trace=False)
+    got, want = (f(*leaves, s) for f in (traced, lightning_attn_func))
+    assert torch.equal(got, want)
+    for a, b in zip(torch.autograd.grad(got, leaves, do), torch.autograd.grad(want, leaves, do)):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda q, k, v, s: lightning_attn_silu_func(q, k, v, s), (q, k, v, s), check_trace=False)
+        assert torch.equal(traced(q * 2, k, v, s), lightning_attn_silu_func(q * 2, k, v, s))

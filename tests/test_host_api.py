@@ -7,7 +7,7 @@ import re
 import pytest
 import torch
 
-from lightning_attn.ops import SimpleRMSNorm, lightning_attn_func, lightning_attn2, lightning_attn2_no_decay
+from lightning_attn.ops import SimpleRMSNorm, lightning_attn_func, lightning_attn_silu_func, lightning_attn2, lightning_attn2_no_decay
 from lightning_attn.ops.hip import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -293,3 +293,14 @@ def test_triton_package_names_stay_operators_after_submodule_imports():
     ) % ([os.path.join(root, "lightning-attention_amd"), root],)
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+@pytest.mark.parametrize("silu", [False, True])
+def test_no_operator_that_may_give_nothing_back_is_traced(silu):
+    """torch.jit.trace refuses such operators (attn_auto, attn_silu_auto), so the traced call is the Python operators', which here
+    refuse the tensors for what they are."""
+    t = torch.zeros(1, 2, 8, 16, dtype=torch.bfloat16)
+    with pytest.raises(Exception) as want:
+        (lightning_attn_silu_func if silu else lightning_attn_func)(t, t, t, torch.zeros(2))
+    with pytest.raises(type(want.value), match=re.escape(str(want.value))):
+        torch.jit.trace(lambda q, k, v, s: (lightning_attn_silu_func if silu else lightning_attn_func)(q, k, v, s), (t, t, t, torch.zeros(2)))
