@@ -420,6 +420,15 @@ static int64_t ng_grid(int64_t rows, int tpr, bool backward, int elt) {
     return groups < cap ? groups : cap;
 }
 
+// Bytes that the column sums (d weight, d bias) of a backward launch take, a row of them per workgroup.  Rows that share a wavefront
+// are asked for in as many bytes as if they did not (`asked`): the same from 16 rows per CU on, so that memory which is enough for many
+// of them is enough for the few that get a wavefront each.
+static size_t ng_part_bytes(int64_t rows, int64_t cols, int elt, bool asked) {
+    int tpr = 0, nv = 0;
+    ng_shape(rows, cols * elt / 16, true, &tpr, &nv);
+    return (size_t)ng_grid(rows, asked && tpr < 64 ? 64 : tpr, true, elt) * 2 * (size_t)cols * sizeof(float);
+}
+
 #define LA_NG_GO(KERNEL, NV, TPR, THREADS, ...) hipLaunchKernelGGL((KERNEL<T, NV, TPR>), grid, dim3(THREADS), 0, st, __VA_ARGS__)
 #define LA_NG_DISPATCH_FWD(KERNEL, ...)                               \
     do {                                                              \
@@ -510,9 +519,7 @@ extern "C" int norm_gate_supported(int64_t cols, int dtype) {
 
 extern "C" size_t norm_gate_workspace_bytes(int64_t rows, int64_t cols, int dtype) {
     if (rows <= 0 || !norm_gate_supported(cols, dtype)) return 0;
-    int tpr = 0, nv = 0;
-    la::ng_shape(rows, cols / (dtype == LA_FP32 ? 4 : 8), true, &tpr, &nv);
-    return (size_t)la::ng_grid(rows, tpr, true, dtype == LA_FP32 ? 4 : 2) * 2 * (size_t)cols * sizeof(float);
+    return la::ng_part_bytes(rows, cols, dtype == LA_FP32 ? 4 : 2, true);
 }
 
 extern "C" int norm_gate_fwd(const void* o, const void* g, const void* weight, const void* bias, void* y, float* mean,
@@ -549,7 +556,7 @@ extern "C" int norm_gate_bwd(const void* o, const void* g, const void* weight, c
     if (!o || !g || !weight || !bias || !mean || !rstd || !dy || !d_o || !d_g) return LA_E_NULLPTR;
     for (const void* p : {o, g, weight, bias, dy, (const void*)d_o, (const void*)d_g})
         if (!la::aligned16(p)) return LA_E_ALIGN;
-    if (!workspace || ws_bytes < norm_gate_workspace_bytes(rows, cols, dtype) || (reinterpret_cast<uintptr_t>(workspace) & 3u))
+    if (!workspace || ws_bytes < la::ng_part_bytes(rows, cols, dtype == LA_FP32 ? 4 : 2, false) || (reinterpret_cast<uintptr_t>(workspace) & 3u))
         return LA_E_WORKSPACE;
     float* part = static_cast<float*>(workspace);
     switch (dtype) {

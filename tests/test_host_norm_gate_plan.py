@@ -15,3 +15,12 @@ def test_workgroups_of_the_backward_pass():
             assert groups(10 ** 6, cols, dtype) == 256
         assert groups(200, 2048, dtype) == 50 and groups(200, 8192, dtype) == 200
     assert groups(1024, 64, 2) == 256 and groups(10 ** 6, 64, 2) == 1024
+
+
+def test_workspace_of_many_short_rows_is_enough_for_fewer():
+    """(rows that share a wavefront leave fewer partial sums than the fewer rows which get a wavefront each)"""
+    L = _lib.lib()
+    for dtype, most in ((0, 256), (1, 256), (2, 1024)):
+        for cols in (64, 128, 200, 256) if dtype < 2 else (32, 64, 100, 128):
+            for rows in (4096, 4097, 5000, 8192, 8193, 16385, 10 ** 6):
+                assert L.norm_gate_workspace_bytes(rows, cols, dtype) == most * 2 * cols * 4, (rows, cols, dtype)
