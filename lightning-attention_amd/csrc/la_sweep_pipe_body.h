@@ -368,7 +368,8 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // (256-byte) row segment.  (Stored straight from the accumulators, each wave would write 32-byte
     // pieces of every row, which the memory system handles far worse: 0.083 against 0.048 ms for the
     // output traffic alone at b4 h32 n8192 d128.)
-    const unsigned lane_o = lane_zcol < colend ? (lane_zrow * ots + lane_zcol) * (unsigned)sizeof(T) : kOob;
+    // (a stride may be so long, with fewer than 64 rows, that the offset of a row beyond them would wrap: kept out of range)
+    const unsigned lane_o = lane_zcol < colend ? (unsigned)min(((uint64_t)lane_zrow * ots + lane_zcol) * sizeof(T), (uint64_t)kOob) : kOob;
     auto store_out = [&](int64_t bout, bool flush, const u32x4 (&o)[ZC]) {
         const int64_t t = REVERSE ? nblk - 1 - bout : bout;
         if constexpr (DENSE) {
@@ -386,7 +387,8 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
 #pragma unroll
             for (int u = 0; u < ZC; ++u) {
                 const int zc = z_col(u);
-                const unsigned off = ZAL ? lane_o + u * ZROWS * ots * (unsigned)sizeof(T) : zc < colend ? (z_row(u) * ots + zc) * (unsigned)sizeof(T) : kOob;
+                const unsigned down = (unsigned)(u * ZROWS) < nrows ? u * ZROWS * ots * (unsigned)sizeof(T) : kOob - 1;
+                const unsigned off = ZAL ? lane_o + down : zc < colend && (unsigned)z_row(u) < nrows ? (z_row(u) * ots + zc) * (unsigned)sizeof(T) : kOob;
                 buf_store16p<PO>(obt, off, o[u]);
             }
         }
