@@ -355,3 +355,11 @@ TORCH_LIBRARY(lightning_attn_hip, m) {
     m.def("attn_silu", &attn_silu);
     m.def("norm_gate", &norm_gate);
 }
+
+// Under torch.vmap the arguments go back to the Python operators, which end in attn or attn_silu: those functorch runs sample by sample, but
+// operators that may give nothing back it refuses.
+TORCH_LIBRARY_IMPL(lightning_attn_hip, FuncTorchBatched, m) {
+    typedef const Tensor& In;
+    m.impl("attn_auto", [](In, In, In, const c10::optional<Tensor>&) -> c10::optional<Tensor> { return c10::nullopt; });
+    m.impl("attn_silu_auto", [](In, In, In, const c10::optional<Tensor>&) -> c10::optional<Tensor> { return c10::nullopt; });
+}

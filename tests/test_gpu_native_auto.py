@@ -92,3 +92,12 @@ def test_traced_calls():
     with torch.no_grad():
         traced = torch.jit.trace(lambda q, k, v, s: lightning_attn_silu_func(q, k, v, s), (q, k, v, s), check_trace=False)
         assert torch.equal(traced(q * 2, k, v, s), lightning_attn_silu_func(q * 2, k, v, s))
+
+
+@pytest.mark.filterwarnings("ignore:There is a performance drop")
+def test_mapped_calls():
+    q, k, v = (_t((4, 2, 3, 70, 64), torch.bfloat16).roll(i, 0) for i in range(3))
+    s = torch.tensor([0.1, 0.2, 0.5], device="cuda")
+    for f in (lightning_attn_func, lightning_attn_silu_func):
+        got = torch.vmap(f, in_dims=(0, 0, 0, None))(q, k, v, s)
+        assert torch.equal(got, torch.stack([f(q[i], k[i], v[i], s) for i in range(4)]))

@@ -304,3 +304,13 @@ def test_no_operator_that_may_give_nothing_back_is_traced(silu):
         (lightning_attn_silu_func if silu else lightning_attn_func)(t, t, t, torch.zeros(2))
     with pytest.raises(type(want.value), match=re.escape(str(want.value))):
         torch.jit.trace(lambda q, k, v, s: (lightning_attn_silu_func if silu else lightning_attn_func)(q, k, v, s), (t, t, t, torch.zeros(2)))
+
+
+@pytest.mark.parametrize("silu", [False, True])
+def test_no_operator_that_may_give_nothing_back_is_mapped(silu):
+    """torch.vmap has no way with such operators either: what it refuses here is the Python operator for CPU tensors."""
+    t = torch.zeros(3, 1, 2, 8, 16, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError) as want:
+        torch.vmap(lightning_attn2, in_dims=(0, 0, 0, None))(t, t, t, torch.zeros(2))
+    with pytest.raises(RuntimeError, match=re.escape(str(want.value))):
+        torch.vmap(lightning_attn_silu_func if silu else lightning_attn_func, in_dims=(0, 0, 0, None))(t, t, t, torch.zeros(2))
