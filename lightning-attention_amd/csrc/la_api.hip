@@ -49,7 +49,9 @@ static bool is_dense(const Tensor& t, int64_t h, int64_t n, int64_t cols) {
 }
 
 static SweepIO io(const Tensor& x, const Tensor& y, const Tensor& z, const Tensor& out) {
-    return SweepIO{x.p, y.p, z.p, const_cast<void*>(out.p), x.l, y.l, z.l, out.l};
+    // (the stride of a single row is never checked; the kernels count the output's in 32 bits, where this one is 2 GiB, beyond any sequence)
+    const Layout lo = {out.l.bs, out.l.hs, out.l.ts < (1LL << 30) ? out.l.ts : 1LL << 30};
+    return SweepIO{x.p, y.p, z.p, const_cast<void*>(out.p), x.l, y.l, z.l, lo};
 }
 
 // caller's scratch memory (may be absent)

@@ -368,8 +368,10 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
     // (256-byte) row segment.  (Stored straight from the accumulators, each wave would write 32-byte
     // pieces of every row, which the memory system handles far worse: 0.083 against 0.048 ms for the
     // output traffic alone at b4 h32 n8192 d128.)
-    // (a stride may be so long, with fewer than 64 rows, that the offset of a row beyond them would wrap: kept out of range)
+    // (with fewer than 64 rows a stride may be so long that the offset of a row beyond them would wrap in 32 bits: such offsets are cut off
+    // and added up with saturation, which leaves them out of range)
     const unsigned lane_o = lane_zcol < colend ? (unsigned)min(((uint64_t)lane_zrow * ots + lane_zcol) * sizeof(T), (uint64_t)kOob) : kOob;
+    const unsigned down_o = (unsigned)min((uint64_t)ZROWS * ots * sizeof(T), (uint64_t)kOob);
     auto store_out = [&](int64_t bout, bool flush, const u32x4 (&o)[ZC]) {
         const int64_t t = REVERSE ? nblk - 1 - bout : bout;
         if constexpr (DENSE) {
@@ -384,11 +386,12 @@ __device__ __forceinline__ void sweep_pipe_body(const SweepPair& pair, const uns
             // the rows from this block's first one on as a buffer of their own (an empty one if nothing is to be written)
             const unsigned first = flush ? (unsigned)(t * 64) * ots * (unsigned)sizeof(T) : 0u;
             const __amdgpu_buffer_rsrc_t obt = make_rsrc(obase + first, flush ? obytes - first : 0u);
+            unsigned off = lane_o;
 #pragma unroll
             for (int u = 0; u < ZC; ++u) {
                 const int zc = z_col(u);
-                const unsigned down = (unsigned)(u * ZROWS) < nrows ? u * ZROWS * ots * (unsigned)sizeof(T) : kOob - 1;
-                const unsigned off = ZAL ? lane_o + down : zc < colend && (unsigned)z_row(u) < nrows ? (z_row(u) * ots + zc) * (unsigned)sizeof(T) : kOob;
+                if (!ZAL) off = zc < colend && (unsigned)z_row(u) < nrows ? (z_row(u) * ots + zc) * (unsigned)sizeof(T) : kOob;
+                else if (u) off = __builtin_elementwise_add_sat(off, down_o);
                 buf_store16p<PO>(obt, off, o[u]);
             }
         }
