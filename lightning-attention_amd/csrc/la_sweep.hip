@@ -23,10 +23,13 @@ int prepare_plans() { return num_cus() > 0 ? 0 : (int)hipErrorInvalidDevice; }
 
 // Sequence chunks per (batch, head, slice).  With few sequences a single sweep per sequence
 // leaves most of the 256 CUs idle; the walk is then cut into up to 8 chunks whose workgroups
-// rebuild their incoming state themselves.  A warm-up block costs about a third of a full block, half of one where two chunks a
-// sequence fill the chip, so chunk lengths shrink geometrically (len_c ~ (1 - rho)^c) to make all workgroups
-// finish together (two chunks, rho 0.36 / 0.5: b4 h32 n1024 d64 16.5 / 16.2, b2 h32 n2048 d128 36.5 / 35.8, b2 h32 n8192 d128 e64 107 / 112; more: la_fwd of b2 h12 n2048 d192, us, by rho 0.25 / 0.3 / 0.36 / 0.45 / 0.5: 39.4 / 38.0 / 38.1 / 40.7 / 42.8; b1 h4 n1000 d128
-// 16.3 / 16.2 / 15.6 / 15.5 / 16.2; b1 h8 n2048 d64 16.3 / 16.9 / 16.1 / 17.3 / 18.2).  The caller's launch options can override the count.
+// rebuild their incoming state themselves.  A warm-up block costs about a third of a full block, half of one where there are two chunks a
+// sequence, so chunk lengths shrink geometrically (len_c ~ (1 - rho)^c) to make all workgroups finish together.  Two chunks that fill the chip,
+// us by rho 0.36 / 0.5: b4 h32 n1024 d64 16.5 / 16.2, b2 h32 n2048 d128 36.5 / 35.8, b2 h32 n8192 d128 e64 107 / 112; two chunks of a
+// walk of 8 to 11 blocks, most of the chip idle: the few warm-up blocks are mostly their latency, b1 h24 n560 d128 14.3 / 13.6, b1 h40 n576 d64
+// 10.9 / 10.3, b1 h16 n570 d256 20.7 / 20.0, b1 h8 n640 d128 14.6 / 14.3, but d192 17.7 / 18.8.  More chunks, la_fwd of b2 h12 n2048 d192 by
+// rho 0.25 / 0.3 / 0.36 / 0.45 / 0.5: 39.4 / 38.0 / 38.1 / 40.7 / 42.8; b1 h4 n1000 d128 16.3 / 16.2 / 15.6 / 15.5 / 16.2; b1 h8 n2048 d64
+// 16.3 / 16.9 / 16.1 / 17.3 / 18.2.  The caller's launch options can override the count.
 static int64_t warm_up_chunks(int64_t cus, int64_t wgs, int64_t nblk, int64_t min_blocks = 4) {
     int64_t c = 1;
     if (wgs * 2 <= cus && nblk >= 2 * min_blocks) {
