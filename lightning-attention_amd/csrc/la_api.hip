@@ -33,9 +33,9 @@ double kept_us(int64_t n, int64_t e, const SavedPlan& pl);
 int prepare_srmsnorm();   // srmsnorm.hip
 int prepare_norm_gate();  // norm_gate.hip
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
-              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, int chunks, hipStream_t st);
+              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, const Opts& opts, hipStream_t st);
 int sweep_f32_bwd_once(const void* q, const void* k, const void* v, const void* dout, void* dq, void* dk, void* dv,
-                       const float* s, int64_t bh, int64_t h, int64_t n, int64_t d, int chunks, hipStream_t st);
+                       const float* s, int64_t bh, int64_t h, int64_t n, int64_t d, const Opts& opts, hipStream_t st);
 
 // A tensor argument: device pointer + where its (batch, head, token) rows start.
 struct Tensor {
@@ -67,7 +67,7 @@ static int run(const Tensor& x, const Tensor& y, const Tensor& z, const Tensor& 
         // the float32 accuracy kernel takes plain (b, h, n, d) tensors only
         if (!is_dense(x, h, n, dk) || !is_dense(y, h, n, dk) || !is_dense(z, h, n, dv) || !is_dense(out, h, n, dv))
             return LA_E_UNSUPPORTED;
-        return sweep_f32(x.p, y.p, z.p, const_cast<void*>(out.p), s, bh, h, n, dk, dv, reverse, 1, opts.chunks, st);
+        return sweep_f32(x.p, y.p, z.p, const_cast<void*>(out.p), s, bh, h, n, dk, dv, reverse, 1, opts, st);
     }
     return sweep(io(x, y, z, out), s, bh, h, n, dk, dv, dtype, reverse, ws.p, ws.bytes, opts, st);
 }
@@ -160,10 +160,10 @@ static int bwd(const Tensor& q, const Tensor& k, const Tensor& v, const float* s
         for (int i = 0; i < 7; ++i)
             if (!is_dense(*ts[i], h, n, d)) return LA_E_UNSUPPORTED;
         void *const pdq = const_cast<void*>(dq.p), *const pdk = const_cast<void*>(dk.p), *const pdv = const_cast<void*>(dv.p);
-        if (opts.paired != LA_OPT_OFF) return sweep_f32_bwd_once(q.p, k.p, v.p, dout.p, pdq, pdk, pdv, s, b * h, h, n, d, opts.chunks, st);
-        rc = sweep_f32(dout.p, v.p, k.p, pdq, s, b * h, h, n, d, d, false, 3, opts.chunks, st);
-        if (rc == LA_OK) rc = sweep_f32(v.p, dout.p, q.p, pdk, s, b * h, h, n, d, d, true, 3, opts.chunks, st);
-        if (rc == LA_OK) rc = sweep_f32(k.p, q.p, dout.p, pdv, s, b * h, h, n, d, d, true, 3, opts.chunks, st);
+        if (opts.paired != LA_OPT_OFF) return sweep_f32_bwd_once(q.p, k.p, v.p, dout.p, pdq, pdk, pdv, s, b * h, h, n, d, opts, st);
+        rc = sweep_f32(dout.p, v.p, k.p, pdq, s, b * h, h, n, d, d, false, 3, opts, st);
+        if (rc == LA_OK) rc = sweep_f32(v.p, dout.p, q.p, pdk, s, b * h, h, n, d, d, true, 3, opts, st);
+        if (rc == LA_OK) rc = sweep_f32(k.p, q.p, dout.p, pdv, s, b * h, h, n, d, d, true, 3, opts, st);
         return rc;
     }
     const SavedPlan pl = sv.p ? plan_saved(b * h, n, d, e, dtype, opts) : kNoPlan;

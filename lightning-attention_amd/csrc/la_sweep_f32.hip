@@ -578,28 +578,27 @@ static const int64_t kMinBlocks = 2;
 // 4.2 us (feature dim 64), 5.15 against 6.9 (128); twice the workgroups leave half the chunks.  us of 64 / 32 columns, forward of d64
 // n2048: 8 sequences 44.5 / 35.8, 24 48 / 41, 48 59 / 64, 128 90 / 104; backward 8 63 / 46, 16 63 / 66, 24 76 / 100; d128: 8 forward 74 / 57,
 // 24 94 / 105, backward 8 93 / 104, 16 144 / 173.
-static double f32_walk_us(int64_t wgs, int64_t nblk, double block_us) {
-    const int64_t cus = num_cus();
+static double f32_walk_us(int64_t cus, int64_t wgs, int64_t nblk, double block_us) {
     int64_t c = cus / wgs < nblk / kMinBlocks ? cus / wgs : nblk / kMinBlocks;
     double sum = 0.0, weight = 1.0;
     for (int64_t i = 0; i < (c < 1 ? 1 : c > 8 ? 8 : c); ++i) { sum += weight; weight *= 1.0 - kWarmCost; }
     return (double)nblk * block_us / sum;
 }
-static int f32_columns(int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod) {
+static int f32_columns(int64_t cus, int64_t bh, int64_t n, int64_t dk, int64_t dv, int nprod) {
     const int64_t nblk = (n + 63) / 64, units = (bh + 7) / 8 * 8 * nprod;
     const int64_t narrow = units * ((dv + 31) / 32), wide = units * ((dv + 63) / 64);
     if (dv <= 32) return 32;
-    if (narrow > num_cus()) return 64;
-    return f32_walk_us(narrow, nblk, dk <= 64 ? 3.05 : 5.15) < 1.03 * f32_walk_us(wide, nblk, dk <= 64 ? 4.2 : 6.9) ? 32 : 64;
+    if (narrow > cus) return 64;
+    return f32_walk_us(cus, narrow, nblk, dk <= 64 ? 3.05 : 5.15) < 1.03 * f32_walk_us(cus, wide, nblk, dk <= 64 ? 4.2 : 6.9) ? 32 : 64;
 }
 
 // `nform`: how many such sweeps the form of the workgroups is chosen for (3: those of a backward pass with d == e, launched apart).
 int sweep_f32(const void* x, const void* y, const void* z, void* out, const float* s, int64_t bh, int64_t h,
-              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, int chunks, hipStream_t st) {
+              int64_t n, int64_t dk, int64_t dv, bool reverse, int nform, const Opts& opts, hipStream_t st) {
     if (dk > 128) return LA_E_UNSUPPORTED;
-    const int cols = f32_columns(bh, n, dk, dv, nform);
+    const int cols = f32_columns(opts.cus, bh, n, dk, dv, nform);
     SweepArgsF32 a = make_args_f32(x, y, z, out, s, bh, h, n, dk, dv, cols);
-    plan_warm_up_chunks(num_cus(), (bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
+    plan_warm_up_chunks(opts.cus, (bh + 7) / 8 * 8 * a.nslice, (n + 63) / 64, opts.chunks, &a.nchunk, a.chunk_start, kWarmCost, kMinBlocks);
 #define LA_GD(DKP, WC, KH, R) (s ? launch_one_f32<DKP, WC, KH, R, true>(a, st) : launch_one_f32<DKP, WC, KH, R, false>(a, st))
 #define LA_GO(DKP, WC, KH) (reverse ? LA_GD(DKP, WC, KH, true) : LA_GD(DKP, WC, KH, false))
     if (dk <= 64) return cols == 32 ? LA_GO(64, 2, 2) : LA_GO(64, 4, 1);
@@ -611,14 +610,14 @@ int sweep_f32(const void* x, const void* y, const void* z, void* out, const floa
 // float32 backward pass with d == e: dQ = fwd(dO, v, k), dK = rev(v, dO, q), dV = rev(k, q, dO) in one
 // launch (the sweeps are independent; with few sequences they run side by side).
 int sweep_f32_bwd_once(const void* q, const void* k, const void* v, const void* dout, void* dq, void* dk, void* dv,
-                       const float* s, int64_t bh, int64_t h, int64_t n, int64_t d, int chunks, hipStream_t st) {
+                       const float* s, int64_t bh, int64_t h, int64_t n, int64_t d, const Opts& opts, hipStream_t st) {
     if (d > 128) return LA_E_UNSUPPORTED;
-    const int cols = f32_columns(bh, n, d, d, 3);
+    const int cols = f32_columns(opts.cus, bh, n, d, d, 3);
     SweepTrioF32 t;
     t.a[0] = make_args_f32(dout, v, k, dq, s, bh, h, n, d, d, cols);
     t.a[1] = make_args_f32(v, dout, q, dk, s, bh, h, n, d, d, cols);
     t.a[2] = make_args_f32(k, q, dout, dv, s, bh, h, n, d, d, cols);
-    plan_warm_up_chunks(num_cus(), (bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, chunks, &t.a[0].nchunk, t.a[0].chunk_start, kWarmCost, kMinBlocks);
+    plan_warm_up_chunks(opts.cus, (bh + 7) / 8 * 8 * t.a[0].nslice * 3, (n + 63) / 64, opts.chunks, &t.a[0].nchunk, t.a[0].chunk_start, kWarmCost, kMinBlocks);
     for (int i = 1; i < 3; ++i) {
         t.a[i].nchunk = t.a[0].nchunk;
         for (int j = 0; j < 9; ++j) t.a[i].chunk_start[j] = t.a[0].chunk_start[j];
