@@ -175,10 +175,13 @@ def native_ops():
     return _native or None
 
 
+_is_tracing = torch._C._is_tracing  # (torch.jit.is_tracing goes by way of Python: 0.4 us a call)
+
+
 def plain_ops():
     """native_ops() for a call under the library's own choices: None where launch options are in force on this thread, and under
     torch.jit.trace, which records operators that give back a tensor but refuses one that may give back nothing."""
-    if getattr(_tls, "opts", None) is not None or torch._C._is_tracing():  # (torch.jit.is_tracing: 0.4 us a call)
+    if getattr(_tls, "opts", None) is not None or _is_tracing():
         return None
     return _native if _native and _native_enabled else native_ops()
 

@@ -40,10 +40,15 @@ def lightning_attn_func(q, k, v, s=None, variant="chunk_loop"):
     q, k, v."""
     if variant not in _VARIANTS:
         raise ValueError("variant must be one of %s, got %r" % (_VARIANTS, variant))
-    if _tensors(q, k, v, s):
+    ops = _lib.plain_ops()
+    if ops is not None:
         # the whole of the common case behind one call; None: the arguments need what follows
-        ops = _lib.plain_ops()
-        o = ops.attn_auto(q, k, v, s) if ops is not None else None
+        try:
+            o = ops.attn_auto(q, k, v, s)
+        except RuntimeError:
+            if _tensors(q, k, v, s):
+                raise
+            o = None
         if o is not None:
             return o
     b, h, n, d = q.shape
@@ -79,9 +84,14 @@ def lightning_attn_silu_func(q, k, v, s=None, variant="chunk_loop"):
     three activation passes disappear; otherwise this is the three PyTorch calls followed by lightning_attn_func."""
     if variant not in _VARIANTS:
         raise ValueError("variant must be one of %s, got %r" % (_VARIANTS, variant))
-    if _tensors(q, k, v, s):
-        ops = _lib.plain_ops()
-        o = ops.attn_silu_auto(q, k, v, s) if ops is not None else None
+    ops = _lib.plain_ops()
+    if ops is not None:
+        try:
+            o = ops.attn_silu_auto(q, k, v, s)
+        except RuntimeError:
+            if _tensors(q, k, v, s):
+                raise
+            o = None
         if o is not None:
             return o
     d, e = q.shape[-1], v.shape[-1]

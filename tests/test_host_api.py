@@ -314,3 +314,22 @@ def test_no_operator_that_may_give_nothing_back_is_mapped(silu):
         torch.vmap(lightning_attn2, in_dims=(0, 0, 0, None))(t, t, t, torch.zeros(2))
     with pytest.raises(RuntimeError, match=re.escape(str(want.value))):
         torch.vmap(lightning_attn_silu_func if silu else lightning_attn_func, in_dims=(0, 0, 0, None))(t, t, t, torch.zeros(2))
+
+
+@pytest.mark.parametrize("at", range(4))
+@pytest.mark.parametrize("bad", [None, 2.0, [1.0, 2.0], "x", True])
+@pytest.mark.parametrize("func", [lightning_attn_func, lightning_attn_silu_func])
+def test_arguments_that_are_no_tensors(func, bad, at):
+    """The native call refuses them in its own words; what the caller sees is the Python operators' error."""
+    args = [torch.zeros(1, 2, 8, 16) for _ in range(3)] + [torch.zeros(2)]
+    args[at] = bad
+    seen = []
+    for native in (True, False):
+        prev = _lib.use_native_ops(native)
+        try:
+            with pytest.raises(Exception) as e:
+                func(*args)
+            seen.append((type(e.value), str(e.value)))
+        finally:
+            _lib.use_native_ops(prev)
+    assert seen[0] == seen[1]
