@@ -15,13 +15,13 @@
 //
 // What bounds it: the fp32 matrix instruction (32 cycles each, 256 FLOP per cycle and CU).  A block of feature dim 64 and 64
 // columns costs the busiest of four wavefronts 48 of them for its score tiles, 64 + 40 for the output and 64 for the state: 2.9 us
-// at 2.4 GHz, measured 4.2 with half of the CUs at work, 5.1 with a workgroup on each and 8.9 for two on each (98 of the 154 TFLOP/s that
-// a large product reaches: forward of 512 sequences, n1536, 215 us).  Feature dim 128 leaves room in LDS for one
+// at 2.4 GHz, measured 4.1 with half of the CUs at work, 4.5 with a workgroup on each and 8.0 for two on each (105 of the 154 TFLOP/s that
+// a large product reaches: forward of 512 sequences, n1536, 200 us).  Feature dim 128 leaves room in LDS for one
 // workgroup only: there two wavefronts share a slab of columns, each with half of the features, so that a SIMD has a second
-// one to issue from (b4 h32 n2048: forward 264 -> 236 us, backward 767 -> 692).  Few sequences: 32 columns to a workgroup, the
-// halves of the features on a wavefront each (a block 3.05 us, 5.15 at feature dim 128), and the walk cut into chunks whose
+// one to issue from (b4 h32 n2048: forward 264 -> 230 us, backward 767 -> 668).  Few sequences: 32 columns to a workgroup, the
+// halves of the features on a wavefront each (a block 3.05 us, 5.0 at feature dim 128), and the walk cut into chunks whose
 // warm-up blocks are fetched from memory in fragment layout, 0.75 us each (1.5 through LDS, a barrier a block).
-// b1 h8 d64, forward + backward, us: n = 1024 30.7 + 31.9 -> 21.2 + 24.2, 4096 109 + 112 -> 70 + 80; b1 h4 n8192 d128 394 + 428 -> 209 + 398.
+// Forward + backward, us: b1 h8 d64 n1024 30.7 + 31.9 -> 20.7 + 24.8, n4096 109 + 112 -> 63 + 73; b1 h4 n8192 d128 394 + 428 -> 199 + 327.
 #include <type_traits>
 
 #include "la_sweep_common.h"
@@ -564,9 +564,9 @@ static SweepArgsF32 make_args_f32(const void* x, const void* y, const void* z, v
     return a;
 }
 
-// What a warm-up block costs of a full one (0.75 of 3.05 us, 1.1 of 4.2; 1.4 of 5.15, 2.0 of 6.9), and the fewest blocks a
-// chunk is worth cutting off for.  b1 h8 n1024 d64 forward, 32 columns, us, by number of chunks 1 / 2 / 4 / 5 / 8: 52 / 34 / 27.5 /
-// 23 / 21: as many as there are CUs for, down to two blocks each.
+// What a warm-up block costs of a full one (0.75 of 3.05 us, 1.1 of 4.1; 1.4 of 5.0, 2.0 of 6.8), and the fewest blocks a
+// chunk is worth cutting off for.  b1 h8 n1024 d64 forward, 32 columns, us, by number of chunks 1 / 2 / 4 / 5 / 8: 52 / 33 / 24 /
+// 22 / 21: as many as there are CUs for, down to two blocks each.
 static const double kWarmCost = 0.27;
 static const int64_t kMinBlocks = 2;
 
@@ -575,7 +575,8 @@ static const int64_t kMinBlocks = 2;
 // half of a 64-column workgroup's slabs would be idle, on two of a CU's four SIMDs, and there are as many workgroups either way (64 / 32, us:
 // backward of 200 sequences n8192 d24 1685 / 1010, 512 n1000 d24 331 / 247, n113 90 sequences 16.9 / 13.8; forward of 300 n2048 d128 e24
 // 435 / 333, 264 n2048 d8 160 / 127).  Per block 3.05 against
-// 4.2 us (feature dim 64), 5.15 against 6.9 (128); twice the workgroups leave half the chunks.  us of 64 / 32 columns, forward of d64
+// 4.2 us (feature dim 64), 5.15 against 6.9 (128); twice the workgroups leave half the chunks.  us of 64 / 32 columns, both taken when the line
+// was drawn, with the next block requested in one piece (blocks are 1 - 4 % quicker since, in either form): forward of d64
 // n2048: 8 sequences 44.5 / 35.8, 24 48 / 41, 48 59 / 64, 128 90 / 104; backward 8 63 / 46, 16 63 / 66, 24 76 / 100; d128: 8 forward 74 / 57,
 // 24 94 / 105, backward 8 93 / 104, 16 144 / 173.
 static double f32_walk_us(int64_t cus, int64_t wgs, int64_t nblk, double block_us) {
