@@ -40,8 +40,9 @@ __device__ __forceinline__ u32x4 buf_load16p(__amdgpu_buffer_rsrc_t r, unsigned 
 // compiler keeps them where the wave-uniform offset of the instruction is a constant; on gfx950 the store reads them just as
 // late when it is a scalar register (seen as address bits in the first four bytes of a lane's 16, in kernels where a v_cndmask into
 // that register came right behind the store; never in kernels without that pair).  So these take no such offset: what is
-// uniform goes into the buffer's base.  SiLU forward of token-major b4 h32 n8192 d128: 339 us; with the offset in a scalar register and a
-// wait behind every store 346, in the per-lane register 359.
+// uniform goes into the buffer's base.  us, against the offset in a scalar register and a wait behind every store, token-major: SiLU forward of
+// b4 h32 n8192 d128 346 -> 339 (346 with the offset in the per-lane register), O and dK + dV of b4 h32 n2048 d256 127 + 249 -> 125 + 247; the other way
+// O of b2 h12 n2048 d192 38.4 -> 39.0, dQ of b4 h32 n2048 d128 52.7 -> 53.5, the pass of b4 h16 n4096 d128 236 -> 237.5.
 template <int POLICY>
 __device__ __forceinline__ void buf_store16p(__amdgpu_buffer_rsrc_t r, unsigned off, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, POLICY);

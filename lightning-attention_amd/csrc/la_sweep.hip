@@ -90,8 +90,9 @@ struct ScanPlan {
 // Estimates, in microseconds, behind the choices below.  A workgroup takes about block_us per 64-token
 // block (measured, by feature dim and columns per workgroup) and, when the lines between the forms were drawn, half of that for
 // a block it only folds into the state; with the warm-up walk of its own (a third) both the warm-up form and the collect launches became
-// quicker, and the lines stayed where they were: over 120 shapes (d 64 .. 256, b*h 1 .. 64, n 2048 .. 8192) the other side is more than 4 % quicker
-// in four, 12 % at most (b1 h32 n2048 d192).  Warm-up blocks: with the geometric chunk lengths of choose_chunks the longest
+// quicker, and the lines stayed where they were: over 120 shapes (d 64 .. 256, b*h 1 .. 64, n 2048 .. 8192) `scan` the other way is more than 4 % quicker
+// in four, 12 % at most (b1 h32 n2048 d192).  (At d = 97 .. 128 that goes back to 64 columns too: 128 columns with warm-up blocks were not among them.  b4 h16
+// n4096 d128, us, forward / step: as chosen 82 / 234, 128 columns with warm-up blocks 80 / 257, 64 with them 75 / 255 - without the states that dQ starts from.)  Warm-up blocks: with the geometric chunk lengths of choose_chunks the longest
 // workgroup runs the fraction `frac` of a single walk.  Scanned states: a chunk one and a half times,
 // plus two more launches and the scan (16 us measured, and 10 for the host's share).
 // `width` of a workgroup: 0 = 64 columns of z / out, 1 = 128 (96 where there are 192 to share out), 2 = all

@@ -35,7 +35,7 @@
 
 namespace la {
 
-// Threads of a workgroup: TPR threads share a row; rows of one or two wavefronts travel four or two to a
+// Threads of a workgroup: TPR threads share a row; rows of up to two wavefronts travel 256 / TPR to a
 // workgroup of 256, wider rows take a workgroup of 256, 512 or 1024 threads to themselves.
 constexpr int ng_threads(int tpr) { return tpr >= 256 ? tpr : 256; }
 // The backward kernel with 16-bit elements: 1024 threads (its registers leave a CU 16 wavefronts either way), so that a CU
